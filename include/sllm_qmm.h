@@ -104,7 +104,9 @@ sllm_status sllm_weight_from_quant(const char *qtype, const void *raw, size_t ra
  *      float32 loop (modelMatmulFloatIntoF32, float32_ops.go:462-482); the
  *      matmuls here rebuild each of those float32 weights exactly from the
  *      native blocks and multiply fp32 activations by them, so only the order
- *      of the row sums differs (no int8 activation codes for these types).
+ *      of the row sums differs (no int8 activation codes for these types);
+ *      the prefill GEMM sums a 16-element sub-block's exact code products
+ *      first and applies its scale and min to the sums.
  * Other types return SLLM_ERR_QTYPE (the reference's dense-fp32 branch).
  */
 sllm_status sllm_weight_from_gguf(uint32_t ggml_type, const void *raw, size_t raw_bytes,
@@ -441,6 +443,7 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  call path)
  *   gemm_min_rows       >= 0       activation rows from which the GEMM is used (0: 8 for
  *                                  weights of 2^24 elements or more, 16 for smaller ones;
+ *                                  Q5_0, Q2K and Q3K: 5 from 2^25 elements, else 8;
  *                                  the GEMM and GEMV sum a row's blocks in different
  *                                  orders, so a row's last bits can change with it)
  *   gemm_shape          0..5       GEMM workgroups: 1 = 64 x 128 tiles, 2 = 64 x 64 tiles with
@@ -450,10 +453,9 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  loads in flight (0: 1, above 128 rows 5; for Q5K1 3,
  *                                  and 4 up to 32 rows; for Q5K1 in one MFMA per block,
  *                                  see sllm_weight_q5k1_one_mfma, 4 up to 32 rows, 2 up
- *                                  to 128, else 1); Q5_0: 1 = 64 x 256
- *                                  tiles, 2 = 64 x 128 (0: 2 up to 4096 weight rows and
- *                                  128 activation rows, else 1). The shape moves the fp32
- *                                  summation splits
+ *                                  to 128, else 1); Q5_0, Q2K, Q3K: 256 columns of 1 =
+ *                                  32, 2 = 64, 3 = 128 rows (0: by the rows). The shape
+ *                                  moves the fp32 summation splits
  *   gemm_splits         0..64      GEMM K splits, added in split order (0: by tile count;
  *                                  the split count moves the fp32 summation splits)
  *   attn_target_blocks  1..65536   attention: about this many workgroups when splitting (512)

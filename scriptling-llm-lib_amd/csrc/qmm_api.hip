@@ -20,6 +20,7 @@ struct sllm_weight {
                      // SLLM_Q6K_STREAM: Q8_0 planes + the streamed Q6_K planes)
     int64_t q6_exceptions = 0;  // SLLM_Q6K_STREAM: blocks the GEMV recomputes in fp64
     bool q5_one_mfma = false;   // Q5K1 with dh = 16 d in every block: the GEMM's SLLM_Q5K1F form
+    bool kq_gemm = false;       // Q2K / Q3K whose scales are all finite: the GEMM takes it
     int groups = 0, rows = 0, cols = 0;
     int device = 0;
     void *base = nullptr;
@@ -469,9 +470,16 @@ bool uses_gemm(const sllm_weight *w, int x_rows) {
     // Measured (us, GEMV at M = 8 / GEMM at M = 8): Q4_1 14336x4096 36.0 /
     // 28.3, Q8_0 4096x14336 54.6 / 42.4, Q5K1 4096x4096 20.2 / 17.7; Q4_1
     // 1024x4096 at M = 8 13.7 / 20.1 and M = 16 27.2 / 19.1, Q4_0 8192x2048 at
-    // M = 16 30.5 / 17.9.
+    // M = 16 30.5 / 17.9. The formats with fp32 activations go through the bf16
+    // GEMM from 5 rows for weights of at least 2^25 elements and from 8 for
+    // smaller ones. Measured (us, GEMV / GEMM): Q5_0 14336x4096 at M = 4 36.7 /
+    // 36.5, M = 5 48.5 / 37; Q3_K 4096x14336 at M = 5 71.6 / 43; Q5_0 4096x4096
+    // at M = 6 22.1 / 21, M = 8 28.6 / 22; Q2_K 4096x4096 at M = 6 20.6 / 25,
+    // M = 8 27.2 / 25; Q5_0 1536x768 at M = 8 11.2 / 11.5, M = 12 16.4 / 11.8.
     int min_rows = tuning().gemm_min_rows;
+    if (min_rows == 0 && act_f32(w->fmt)) min_rows = (int64_t)w->rows * w->cols >= ((int64_t)1 << 25) ? 5 : 8;
     if (min_rows == 0) min_rows = (int64_t)w->rows * w->cols >= ((int64_t)1 << 24) ? 8 : 16;
+    if (kq_native(w->fmt) && !w->kq_gemm) return false;
     return x_rows >= min_rows && gemm_supported(w->fmt, w->groups);
 }
 
@@ -825,17 +833,20 @@ sllm_status sllm_weight_from_gguf(uint32_t t, const void *raw, size_t raw_bytes,
     sllm_weight *w = nullptr;
     if ((st = alloc_weight(fmt, rows, cols, &w, layout)) != SLLM_OK) return st;
     uint32_t q6stat[2] = {0, 0};
-    int q5bad = 1;
+    int form_bad = 1;  // the format's GEMM form does not hold for some block
     st = with_upload(raw, need, 256, [&](Ctx *c) -> sllm_status {
         const uint8_t *dev = (const uint8_t *)c->buf;
         if (t == 8 || t == 2 || t == 3 || t == 6) return pack_from_raw(fmt, dev, rows, cols / 32, w->planes, nullptr, c->stream);
-        if (t == 13) {
+        if (t == 13 || kq_native(fmt)) {
+            const int64_t nb = (int64_t)rows * (cols / 32);
             int *bad = (int *)((char *)c->buf + ((need + 255) & ~(size_t)255));
             SLLM_HIP(hipMemsetAsync(bad, 0, sizeof(int), c->stream));
             sllm_status ps = pack_from_gguf(t, dev, rows, cols, w->planes, c->stream);
-            if (ps == SLLM_OK) ps = check_q5k1_one_mfma(w->planes, (int64_t)rows * (cols / 32), bad, c->stream);
+            if (ps == SLLM_OK)
+                ps = t == 13 ? check_q5k1_one_mfma(w->planes, nb, bad, c->stream)
+                             : check_kq_finite(fmt, w->planes, nb, bad, c->stream);
             if (ps != SLLM_OK) return ps;
-            SLLM_HIP(hipMemcpyAsync(&q5bad, bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+            SLLM_HIP(hipMemcpyAsync(&form_bad, bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
             return SLLM_OK;
         }
         if (w->layout != SLLM_Q6K_STREAM) return pack_from_gguf(t, dev, rows, cols, w->planes, c->stream);
@@ -848,7 +859,8 @@ sllm_status sllm_weight_from_gguf(uint32_t t, const void *raw, size_t raw_bytes,
     if (st == SLLM_OK && q6stat[1] != 0)
         st = set_error(SLLM_ERR_DEVICE, "Q6_K stream pack: the fp64 requantization disagrees with the Q8_0 planes");
     w->q6_exceptions = q6stat[0];
-    w->q5_one_mfma = t == 13 && q5bad == 0;
+    w->q5_one_mfma = t == 13 && form_bad == 0;
+    w->kq_gemm = kq_native(fmt) && form_bad == 0;
     if (st != SLLM_OK) {
         sllm_weight_destroy(w);
         return st;

@@ -213,7 +213,14 @@ sllm_status launch_gemm(int fmt, const Planes &P, const float *x, float *dst, in
 sllm_status launch_gemm_dots(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M,
                              void *ws, size_t ws_bytes, int32_t *dots, hipStream_t s);
 size_t gemm_workspace_bytes(int fmt, int N, int G, int M);
-bool gemm_supported(int fmt, int G);  // Q5_0 and K not a multiple of 128 stay on the GEMV
+bool gemm_supported(int fmt, int G);  // int8 formats: K a multiple of 128 (others stay on the GEMV)
+// Formats with fp32 activations (Q5_0, Q2_K, Q3_K): the same products on the bf16
+// matrix cores; ws holds at least bgemm_workspace_bytes.
+sllm_status launch_bgemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws,
+                         hipStream_t s);
+size_t bgemm_workspace_bytes(int fmt, int N, int G, int M);
+// dst = part[0] + part[1] + ... + part[S - 1] (n floats each), in split order.
+sllm_status launch_reduce_splits(const float *part, float *dst, size_t n, int S, hipStream_t s);
 sllm_status launch_quantize_act(const float *x, int rows, int G, int8_t *xq, float *xs, int32_t *sx,
                                 hipStream_t s);
 sllm_status launch_block_dots(int fmt, const Planes &P, const float *x, int N, int G, int M,
@@ -232,6 +239,10 @@ sllm_status pack_q6k_stream(const uint8_t *raw_dev, int rows, int cols, const Mu
 // *bad_dev (cleared by the caller) set unless every block of a Q5K1 weight's
 // planes has dh = 16 d: the condition for the GEMM's one-MFMA form.
 sllm_status check_q5k1_one_mfma(const MutPlanes &P, int64_t nb, int *bad_dev, hipStream_t s);
+// *bad_dev (cleared by the caller) set where a native k-quant's super-block scale
+// (d, Q2_K's dmin) is not finite: the GEMM factors the scale out of a group's
+// sum, where the reference's inf * 0 per element gives NaN.
+sllm_status check_kq_finite(int fmt, const MutPlanes &P, int64_t nb, int *bad_dev, hipStream_t s);
 // GGUF super-block bytes of a native k-quant weight from its (host copy of the) planes.
 void export_kq_native(int fmt, const MutPlanes &p, int64_t nb, uint8_t *out);
 

@@ -465,6 +465,22 @@ sllm_status pack_from_gguf(uint32_t t, const uint8_t *raw_dev, int rows, int col
     return SLLM_OK;
 }
 
+namespace {
+__global__ void kq_finite_kernel(const uint32_t *__restrict__ sb, int64_t n, bool both, int *bad) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t w = sb[i];
+        if ((w & 0x7c00u) == 0x7c00u || (both && (w & 0x7c000000u) == 0x7c000000u)) *bad = 1;
+    }
+}
+}  // namespace
+
+sllm_status check_kq_finite(int fmt, const MutPlanes &P, int64_t nb, int *bad_dev, hipStream_t s) {
+    hipLaunchKernelGGL(kq_finite_kernel, dim3(grid_for(nb / 8)), dim3(256), 0, s, P.sb, nb / 8, fmt == SLLM_Q2K,
+                       bad_dev);
+    SLLM_HIP(hipGetLastError());
+    return SLLM_OK;
+}
+
 void export_kq_native(int fmt, const MutPlanes &p, int64_t nb, uint8_t *o) {
     // inverse of pack_q2k_kernel / pack_q3k_kernel, one super-block at a time
     const int per = fmt == SLLM_Q2K ? 84 : 110;

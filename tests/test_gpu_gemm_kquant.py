@@ -1,0 +1,109 @@
+"""GPU tests of the prefill GEMM of the native Q2_K / Q3_K weights (bf16 matrix
+cores over the exact three-way split of the fp32 activations).
+
+Bound: a weight is dl * q - ml. The GEMM forms every product of q and of ml
+exactly or with one rounding and adds them in some order, the oracle multiplies
+the rounded weights and adds sequentially: both are within (K + K / 32 + 64) u
+of sum |x| (|dl q| + |ml|), u = 2^-24.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import sllm_qmm as sq
+
+from _helpers import make_x
+from test_gpu_kquant_native import PER, make_kq
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -24
+
+
+@pytest.fixture(autouse=True)
+def _params():
+    sq.set_param("gemm_min_rows", 1)
+    yield
+    for p in ("gemm_min_rows", "gemm_shape", "gemm_splits"):
+        sq.set_param(p, 0)
+
+
+def parts(t, raw, N, K):
+    """|dl q| + |ml| of every weight."""
+    a = raw.reshape(-1, PER[t]).copy()
+    if t == 11:
+        return np.abs(oracle.dense_weights(t, raw, N, K)).astype(np.float64)
+    b = a.copy()
+    a[:, 82:84] = 0
+    b[:, 80:82] = 0
+    return sum(np.abs(oracle.dense_weights(t, r.reshape(-1), N, K)).astype(np.float64) for r in (a, b))
+
+
+def gemm(w, x):
+    M, K = x.shape
+    xd = torch.from_numpy(x).cuda()
+    y = torch.full((M, w.rows), float("nan"), device="cuda")
+    sq.matmul_dev(w, xd.data_ptr(), M, K, y.data_ptr())
+    torch.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("t", [10, 11])
+@pytest.mark.parametrize("N,K,M,shape,splits", [
+    (1, 256, 1, 0, 0), (300, 768, 32, 0, 0), (300, 768, 33, 0, 0), (257, 512, 65, 0, 0), (31, 256, 129, 0, 0),
+    (513, 1280, 200, 0, 0), (520, 1024, 100, 1, 3), (520, 1024, 100, 2, 5), (520, 1024, 100, 3, 2),
+    (256, 2048, 4, 0, 32)])
+def test_gemm_within_bound(t, N, K, M, shape, splits):
+    sq.set_param("gemm_shape", shape)
+    sq.set_param("gemm_splits", splits)
+    raw = make_kq(t, N, K, 31 + M)
+    w = sq.load_weight_f32_direct(t, raw, N, K)
+    x = make_x(M, K, seed=M)
+    ref = oracle.matmul_dense(oracle.dense_weights(t, raw, N, K), x).astype(np.float64)
+    bound = (K + K // 32 + 64) * U * (np.abs(x).astype(np.float64) @ parts(t, raw, N, K).T) + 1e-30
+    assert np.all(np.abs(gemm(w, x) - ref) <= bound)
+
+
+@pytest.mark.parametrize("t", [10, 11])
+def test_activations_outside_the_factored_range(t):
+    # huge, tiny, infinite and NaN activations in single rows and blocks: the
+    # blocks that hold one are computed weight by weight, as the reference does
+    N, K, M = 70, 512, 40
+    raw = make_kq(t, N, K, 5)
+    w = sq.load_weight_f32_direct(t, raw, N, K)
+    W = oracle.dense_weights(t, raw, N, K)
+    x = make_x(M, K, seed=6)
+    x[3] *= np.float32(2.0 ** 100)
+    x[7] *= np.float32(2.0 ** -110)
+    x[11, 64:96] = np.float32(3e38)
+    x[35, 5] = np.inf
+    x[36, 300] = -np.inf
+    x[37, 511] = np.nan
+    got = gemm(w, x).astype(np.float64)
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref = oracle.matmul_dense(W, x).astype(np.float64)
+        bound = (K + K // 32 + 64) * U * (np.abs(x).astype(np.float64) @ parts(t, raw, N, K).T) + 1e-44
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(got[inf], ref[inf])
+    fin = np.isfinite(ref)
+    assert np.all(np.abs(got[fin] - ref[fin]) <= bound[fin])
+
+
+@pytest.mark.parametrize("t", [10, 11])
+def test_weights_with_infinite_scales_stay_on_the_gemv(t):
+    # inf * 0 per weight is NaN, inf * (a group's sum) is not: such a weight
+    # gives the same bits whether the GEMM is allowed or not
+    N, K, M = 40, 512, 9
+    raw = make_kq(t, N, K, 8).reshape(-1, PER[t])
+    at = 80 if t == 10 else 108
+    raw[5, at:at + 2] = [0x00, 0x7C]
+    if t == 10:
+        raw[9, 82:84] = [0x00, 0xFC]
+    w = sq.load_weight_f32_direct(t, raw.reshape(-1), N, K)
+    x = make_x(M, K, seed=9)
+    a = gemm(w, x)
+    sq.set_param("gemm_min_rows", 1 << 20)
+    assert np.array_equal(a.view(np.uint32), gemm(w, x).view(np.uint32))
