@@ -323,12 +323,17 @@ typedef struct sllm_attn_params {
  * the cache (q head h reads kv head h / nRep; fusedAttentionHeadF32,
  * float32_ops.go:190-235) to out_dev, heads merged (seq_len x n_heads*d_k,
  * mergeHeadsDataF32 float32_ops.go:262-273). q/k/v are not modified.
- * Scores are the reference's sequential float32 dots; the softmax sums and
+ * Scores are float32 dots (the reference's sequential ones, except on the matrix
+ * cores); the softmax sums and
  * the weighted sum of values are reassociated (split over the positions and
  * combined), and the per-head RMSNorm sums its squares in the library's
  * fixed order. One row (decode): two launches (the attention over splits of
  * the cached positions, which also prepares the row, then the combine of the
- * splits); several rows: three (the row preparation first). Asynchronous on
+ * splits); several rows: three (the row preparation first). Prompts (more
+ * than 512 pairs of row and kv head, d_k up to 128, out_dev 16-byte aligned)
+ * run on the fp32 matrix cores, where a score is the dots of the head's two
+ * halves added; they use more workspace where it can be had (not on a
+ * stream under capture whose workspace is smaller). Asynchronous on
  * `stream`; allocates nothing once the stream's workspace has grown to the
  * call's size.
  */

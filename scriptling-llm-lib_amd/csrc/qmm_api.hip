@@ -159,6 +159,20 @@ sllm_status workspace(hipStream_t stream, size_t need, void **out, size_t *cap) 
     return SLLM_OK;
 }
 
+// Whether workspace(stream, need) would succeed as far as capture goes: the
+// stream's workspace is large enough, or the stream is not being captured.
+bool workspace_at_hand(hipStream_t stream, size_t need) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    const uint64_t key = ((uint64_t)(uintptr_t)stream << 8) ^ (uint64_t)dev;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        auto it = g_ws.find(key);
+        if (it != g_ws.end() && it->second.cap >= need) return true;
+    }
+    return !capturing(stream);
+}
+
 // The scratch of sllm_attention_noalloc_dev: the attention's rotated q rows
 // and split states, which sllm_attention_dev keeps in the stream's
 // workspace, in a static device array so that the call allocates nothing.
@@ -642,6 +656,12 @@ sllm_status attention_impl(sllm_kv_cache *kv, int layer, const sllm_attn_params 
     int splits = 0, tps = 0, tw = 0, hs = 1;
     size_t wsb = 0;
     attention_plan(seq_len, p->n_heads, kv->n_kv, kv->d_k, cl + seq_len, &splits, &tps, &tw, &hs, &wsb);
+    // The matrix-core kernel needs more scratch where rows are long: where that
+    // cannot be had (the static scratch, a stream under capture), the split
+    // kernel's plan holds.
+    size_t fwsb = 0;
+    bool flash = attention_flash(seq_len, p->n_heads, kv->n_kv, kv->d_k, cl, out, &fwsb) &&
+                 (noalloc ? fwsb <= kStaticScratchBytes : fwsb <= wsb || workspace_at_hand(s, fwsb));
     void *ws = nullptr;
     size_t cap = 0;
     if (noalloc) {
@@ -651,7 +671,7 @@ sllm_status attention_impl(sllm_kv_cache *kv, int layer, const sllm_attn_params 
                                                  std::to_string(kStaticScratchBytes) +
                                                  " (fewer rows per call, or sllm_attention_dev)");
         if ((st = static_scratch(&ws)) != SLLM_OK) return st;
-    } else if ((st = workspace(s, wsb, &ws, &cap)) != SLLM_OK) {
+    } else if ((st = workspace(s, flash ? fwsb : wsb, &ws, &cap)) != SLLM_OK) {
         return st;
     }
     AttnArgs a{};
@@ -688,7 +708,7 @@ sllm_status attention_impl(sllm_kv_cache *kv, int layer, const sllm_attn_params 
     a.tps = tps;
     a.tw = tw;
     a.hs = hs;
-    if ((st = launch_attention(a, s)) != SLLM_OK) return st;
+    if ((st = flash ? launch_attention_flash(a, s) : launch_attention(a, s)) != SLLM_OK) return st;
     kv->len[(size_t)layer] = cl + seq_len;
     return SLLM_OK;
 }

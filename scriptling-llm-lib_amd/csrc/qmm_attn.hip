@@ -38,6 +38,7 @@ constexpr int kDotSteps = 4;  // 4-element steps of a score's LDS reads issued t
 // union type, can keep a register array in scratch memory).
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float lane_bcast(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
@@ -97,31 +98,56 @@ __device__ void prep_row(float *row, const float *src, int dk, const float *bias
     wave_lds_sync();
 }
 
-// Several rows (prefill): one wave per (row, head) - q heads into the
-// workspace, kv heads into the cache (k: bias, norm, RoPE; v: bias) at
-// rows cache_len + s (the append, model_f32.go:445-448).
-__global__ void __launch_bounds__(64) attn_prep_kernel(AttnArgs a) {
-    __shared__ float row[kMaxDk];
-    const int s = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
-    const bool isq = t < a.n_heads;
-    const int h = isq ? t : t - a.n_heads;
+// Several rows (prefill): gridDim.y workgroups per row - q heads into the workspace, kv
+// heads into the cache (k: bias, norm, RoPE; v: bias) at rows cache_len + s
+// (the append, model_f32.go:445-448). The row's rotation (the same for every
+// head) is formed once per workgroup in LDS, then a wave takes every eighth head
+// of the workgroup's: with a workgroup and an fp64 sincos of its own for every
+// head, 1024 rows of 32 + 8 heads took 15.9 us (now 13.0). Few rows get a
+// workgroup for every eight heads, so that no wave takes two in turn.
+constexpr int kPrepWaves = 8;
+__global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_kernel(AttnArgs a) {
+    __shared__ float rows[kPrepWaves][kMaxDk];
+    __shared__ float rc[kMaxDk / 2], rs[kMaxDk / 2];
+    const int s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int dk = a.d_k;
-    const int cols = (isq ? a.n_heads : a.n_kv) * dk;
-    prep_row(row, (isq ? a.q : a.k) + (size_t)s * cols + (size_t)h * dk, dk, isq ? a.q_bias : a.k_bias, h * dk,
-             isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, a.freqs, a.half_dim, a.start_pos + s,
-             lane);
-    if (isq) {
-        float *dst = a.qrot + ((size_t)s * a.n_heads + h) * dk;
-        for (int d = lane; d < dk; d += 64) dst[d] = row[d];
-    } else {
-        const size_t at = ((size_t)h * a.cap + (size_t)(a.cache_len + s)) * dk;
-        const float *vs = a.v + (size_t)s * cols + (size_t)h * dk;
-        for (int d = lane; d < dk; d += 64) {
-            a.cache_k[at + d] = row[d];
-            float x = vs[d];
-            if (a.v_bias && h * dk + d < a.vb_len) x = x + a.v_bias[h * dk + d];
-            a.cache_v[at + d] = x;
+    for (int i = threadIdx.x; i < a.half_dim; i += 64 * kPrepWaves) {
+        const float ang = a.freqs[i] * (float)(a.start_pos + s);
+        double sd, cd;
+        sincos((double)ang, &sd, &cd);
+        rc[i] = (float)cd;
+        rs[i] = (float)sd;
+    }
+    __syncthreads();
+    float *row = rows[wave];
+    for (int t = blockIdx.y * kPrepWaves + wave; t < a.n_heads + a.n_kv; t += gridDim.y * kPrepWaves) {
+        const bool isq = t < a.n_heads;
+        const int h = isq ? t : t - a.n_heads;
+        const int cols = (isq ? a.n_heads : a.n_kv) * dk;
+        prep_row(row, (isq ? a.q : a.k) + (size_t)s * cols + (size_t)h * dk, dk, isq ? a.q_bias : a.k_bias, h * dk,
+                 isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, nullptr, 0, 0, lane);
+        // RoPE (applyRopeInPlaceF32, float32_ops.go:174-188)
+        for (int i = lane; i < a.half_dim; i += 64) {
+            const float c = rc[i], sn = rs[i];
+            const float x0 = row[2 * i], x1 = row[2 * i + 1];
+            row[2 * i] = x0 * c - x1 * sn;
+            row[2 * i + 1] = x0 * sn + x1 * c;
         }
+        wave_lds_sync();
+        if (isq) {
+            float *dst = a.qrot + ((size_t)s * a.n_heads + h) * dk;
+            for (int d = lane; d < dk; d += 64) dst[d] = row[d];
+        } else {
+            const size_t at = ((size_t)h * a.cap + (size_t)(a.cache_len + s)) * dk;
+            const float *vs = a.v + (size_t)s * cols + (size_t)h * dk;
+            for (int d = lane; d < dk; d += 64) {
+                a.cache_k[at + d] = row[d];
+                float x = vs[d];
+                if (a.v_bias && h * dk + d < a.vb_len) x = x + a.v_bias[h * dk + d];
+                a.cache_v[at + d] = x;
+            }
+        }
+        wave_lds_sync();  // the row is read before the next head's is written
     }
 }
 
@@ -518,6 +544,360 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a) {
     }
 }
 
+// ---------------------------------------------------------- prompts ----
+//
+// attn_flash_kernel: several query rows (from kFlashRows on, d_k up to 128) on
+// the fp32 matrix cores. A wave owns 32 query rows of one q head; the four
+// waves of a workgroup share one kv head's K and V tiles of 32 positions in LDS
+// (GQA: the q heads of the group; otherwise further row blocks). Both products
+// are taken transposed, so that a lane is a query row throughout:
+//   S^T = K Q^T: A = K (LDS), B = Q (registers for the whole kernel). Lane half h
+//     takes the head's dimensions DK / 2 h .. (the order of the MFMA's k is
+//     free), so K is read with 16-byte LDS reads;
+//   softmax: a lane holds 16 of the tile's positions of its row, lane ^ 32 the
+//     other 16: no reduction over lanes but one exchange;
+//   O^T = V^T P^T: accumulator v of S^T is position 8 (v / 4) + 4 h + v % 4, so as
+//     B operand of a two-deep MFMA it pairs positions p and p + 4: P goes from
+//     accumulator to operand without leaving its registers, V is read to match.
+// Scores are fp32 dots of the same products as the reference's (in two halves,
+// added by the MFMA), the exponentials float32(exp(float64(score - running
+// max))), the sums fp32: as the split kernel, in another association.
+//
+// What bounds it: the fp32 matrix cores (64 cycles per 32 x 32 x 2; 2 DK of
+// them per tile); the split kernel spent 64-lane VALU dots and one pass over K
+// and V per query row (1024 rows of 32 / 8 heads, d_k 128: 896 us).
+// Causal rows differ in length: a row block's tiles are cut into chunks of C
+// tiles (workgroups of their own; heaviest first) whose states
+// attn_flash_combine_kernel merges; C is about the tiles one workgroup slot gets
+// in all, so that no workgroup outlasts the rest.
+// Positions past a row's limit get weight 0 by selection. A non-finite V
+// element would still turn the earlier rows' 0 into NaN inside the MFMA: such
+// elements are staged as 0, their positions noted, and their products added to
+// the rows that see them on the VALU.
+constexpr int kFlashTile = 32;
+constexpr int kFlashWaves = 4;
+
+struct FlashPlan {
+    int groups;   // workgroups of units per kv head
+    int chunk;    // most tiles per chunk
+    int chunks;   // most chunks of a group
+};
+// Tiles of each chunk of a group with so many tiles: chunks of one group are even.
+__host__ __device__ inline int flash_chunk(const FlashPlan &f, int tiles) {
+    const int n = (tiles + f.chunk - 1) / f.chunk;
+    return (tiles + n - 1) / n;
+}
+
+// exp(x) for x <= 0 (or NaN) to float32, in float32 operations: r = x - n ln 2 in
+// two parts (the first exact: n has at most 8 bits, the first constant 16), the
+// Taylor polynomial of exp(r) - 1 - r to r^8 (remainder 2^-32), and 1 + r added
+// with its rounding error carried along (Fast2Sum). Over [-80, 0] its rms error
+// is 0.2897 ulp (the rounded fp64 exp 0.2886), one argument in 67 differs from
+// that by an ulp; attention outputs are as far from 64 bits with either.
+__device__ __forceinline__ float exp_neg(float x) {
+    const float n = __builtin_rintf(x * 1.44269504f);
+    const float rh = __builtin_fmaf(n, -0.693145752f, x);  // 0x3f317200: 16 bits of ln 2
+    const float rl = n * -1.42860677e-6f;
+    const float r = rh + rl;
+    float p = 2.48015873e-5f;  // 1 / 8!
+    p = __builtin_fmaf(p, r, 1.98412698e-4f);
+    p = __builtin_fmaf(p, r, 1.38888889e-3f);
+    p = __builtin_fmaf(p, r, 8.33333333e-3f);
+    p = __builtin_fmaf(p, r, 4.16666667e-2f);
+    p = __builtin_fmaf(p, r, 1.66666667e-1f);
+    p = __builtin_fmaf(p, r, 0.5f);
+    const float t = __builtin_fmaf(r * r, p, rl);
+    const float s = 1.0f + rh;
+    const float e = rh - (s - 1.0f);
+    const float y = __builtin_ldexpf(s + (e + t), (int)n);
+    return x < -104.0f ? 0.0f : y;
+}
+
+template <int DT, bool FULL>
+__global__ void __launch_bounds__(64 * kFlashWaves) __attribute__((amdgpu_waves_per_eu(2)))
+attn_flash_kernel(AttnArgs a, FlashPlan f) {
+    constexpr int DK = 32 * DT, HD = DK / 2;  // padded head size; dimensions per lane half
+    constexpr int KS = DK + 4;                // LDS row stride: 16-byte reads of successive rows hit distinct banks
+    constexpr int T = 64 * kFlashWaves;
+    constexpr int PER = kFlashTile * (DK / 4) / T;  // 16-byte pieces of K (and of V) per thread
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    // [2 buffers][K tile, V tile], then the masks
+    auto ktile = [&](int b) { return lds + b * 2 * kFlashTile * KS; };
+    auto vtile = [&](int b) { return lds + (b * 2 + 1) * kFlashTile * KS; };
+    // masks of the tile's positions with non-finite V elements, one for each of
+    // three successive tiles: read, filled and cleared in the same step
+    unsigned *badm = (unsigned *)(lds + 4 * kFlashTile * KS);
+
+    const int dk = FULL ? DK : a.d_k;
+    const int g = blockIdx.x;                           // kv head (fastest: one head per XCD)
+    const int ug = (int)gridDim.y - 1 - (int)blockIdx.y;  // longest rows first
+    const int ch = blockIdx.z;
+    const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nrb = (a.seq + 31) / 32, U = nrb * a.rep;
+    auto kv_of = [&](int rb) { return a.cache_len + min(a.seq, 32 * (rb + 1)); };  // positions a row block sees
+    const int last = min(ug * kFlashWaves + kFlashWaves - 1, U - 1);
+    const int tiles = (kv_of(last / a.rep) + kFlashTile - 1) / kFlashTile;
+    const int clen = flash_chunk(f, tiles);
+    const int t0 = ch * clen, t1 = min(tiles, t0 + clen);
+    if (t0 >= tiles) return;
+    const int unit = min(ug * kFlashWaves + wave, U - 1);
+    const bool mine = ug * kFlashWaves + wave < U;
+    const int rb = unit / a.rep, hq = g * a.rep + unit % a.rep;
+    const int wkv = kv_of(rb);
+    const int row = min(rb * 32 + r32, a.seq - 1);  // rows past seq repeat the last one, never stored
+    const int limit = a.cache_len + row + 1;        // positions this lane's row sees
+
+    const float *kb = a.cache_k + (size_t)g * a.cap * dk;
+    const float *vb = a.cache_v + (size_t)g * a.cap * dk;
+    const int kvmax = kv_of(last / a.rep);
+
+    // A thread stages pieces of 16 bytes (dimensions c .. c + 3) of positions p0, p0
+    // + PS, ... of K, then of V (the same registers). Positions past the last
+    // repeat it: their weights are 0 and V is staged finite.
+    constexpr int PS = T / (DK / 4);
+    static_assert(T % (DK / 4) == 0 || DK == 96, "a thread's pieces share their dimensions");
+    v4f st[PER];
+    auto piece = [&](int i, int &p, int &c) {
+        if (DK == 96) {
+            const int e = threadIdx.x + T * i;
+            p = e / (DK / 4);
+            c = e % (DK / 4) * 4;
+        } else {
+            p = (int)threadIdx.x / (DK / 4) + PS * i;
+            c = (int)threadIdx.x % (DK / 4) * 4;
+        }
+    };
+    auto load_tile = [&](const float *src, int t) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            int p, c;
+            piece(i, p, c);
+            const uint32_t pos = (uint32_t)min(t * kFlashTile + p, kvmax - 1);
+            // 32-bit byte offsets: one head's rows stay below 4 GiB
+            st[i] = *(const v4f *)((const char *)src + (pos * (uint32_t)dk + (uint32_t)(FULL ? c : min(c, dk - 4))) * 4u);
+        }
+    };
+    auto store_k = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            int p, c;
+            piece(i, p, c);
+            const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+            *(v4f *)(ktile(b) + p * KS + c) = FULL || c < dk ? st[i] : z;
+        }
+    };
+    auto store_v = [&](int b, unsigned *bm) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            int p, c;
+            piece(i, p, c);
+            bool bad = false;
+            v4f v = st[i];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const bool fin = __builtin_isfinite(v[k]);
+                bad |= !fin;
+                v[k] = fin ? v[k] : 0.0f;
+            }
+            *(v4f *)(vtile(b) + p * KS + c) = v;
+            if (bad) atomicOr(bm, 1u << p);
+        }
+    };
+
+    // this lane's half of its query row
+    v4f q[HD / 4];
+    {
+        const float *qr = a.qrot + ((size_t)row * a.n_heads + hq) * dk + HD * h;
+#pragma unroll
+        for (int j = 0; j < HD / 4; j++) {
+            const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+            q[j] = FULL || HD * h + 4 * j < dk ? *(const v4f *)(qr + 4 * j) : z;
+        }
+    }
+    v16f o[DT];
+#pragma unroll
+    for (int t = 0; t < DT; t++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[t][v] = 0.0f;
+    float m = -INFINITY, l = 0.0f;
+
+    if (threadIdx.x < 3) badm[threadIdx.x] = 0;
+    load_tile(kb, t0);
+    store_k(0);
+    load_tile(vb, t0);
+    __syncthreads();
+    store_v(0, badm);
+    __syncthreads();
+    int b3 = 0;  // (t - t0) % 3
+    for (int t = t0; t < t1; t++, b3 = b3 == 2 ? 0 : b3 + 1) {
+        const int b = (t - t0) & 1;
+        if (threadIdx.x == 0) badm[b3 == 0 ? 2 : b3 - 1] = 0;  // the tile before's, read by all
+        const bool more = t + 1 < t1, work = t * kFlashTile < wkv;
+        v16f s = {};
+        if (more) load_tile(kb, t + 1);
+        if (work) {
+            // S^T: rows = positions, columns = query rows
+            const float *kt = ktile(b) + r32 * KS + HD * h;
+#pragma unroll
+            for (int j = 0; j < HD / 4; j++) {
+                const v4f kv = *(const v4f *)(kt + 4 * j);
+#pragma unroll
+                for (int k = 0; k < 4; k++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[k], q[j][k], s, 0, 0, 0);
+            }
+            // online softmax over the lane's 16 positions and lane ^ 32's
+            const int left = limit - t * kFlashTile - 4 * h;  // position index 8 (v / 4) + v % 4 counts if below
+            float mt = -INFINITY;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                s[v] = s[v] * a.scale;
+                if (8 * (v >> 2) + (v & 3) < left) mt = fmaxf(mt, s[v]);
+            }
+            mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+            const float mn = fmaxf(m, mt);
+            const bool any = limit > t * kFlashTile;  // this row sees some position of the tile
+            // the first positions a row meets: exp(-inf) = 0 exactly
+            float alpha = 1.0f;
+            if (any && !(m == mn)) alpha = (m == -INFINITY && mn < INFINITY) ? 0.0f : (float)exp((double)(m - mn));
+            float es = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const bool in = 8 * (v >> 2) + (v & 3) < left;
+                const float e = exp_neg(s[v] - mn);
+                s[v] = in ? e : 0.0f;
+                es = es + s[v];
+            }
+            es = es + __shfl_xor(es, 32, 64);
+            if (any) {
+                l = l * alpha + es;
+                m = mn;
+            }
+            if (__ballot(alpha != 1.0f)) {
+#pragma unroll
+                for (int tt = 0; tt < DT; tt++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) o[tt][v] = o[tt][v] * alpha;
+            }
+        }
+        // the other buffer is free since the barrier at the end of the tile before
+        if (more) {
+            store_k(b ^ 1);
+            load_tile(vb, t + 1);
+        }
+        if (work) {
+            // O^T += V^T P^T
+            const float *vt = vtile(b) + 4 * h * KS + r32;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const float *vp = vt + (8 * (v >> 2) + (v & 3)) * KS;
+#pragma unroll
+                for (int tt = 0; tt < DT; tt++)
+                    o[tt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vp[32 * tt], s[v], o[tt], 0, 0, 0);
+            }
+            // non-finite V elements of the tile, for the rows that see them
+            unsigned bad = badm[b3];
+            while (bad) {
+                const int p = __builtin_ctz(bad);
+                bad &= bad - 1;
+                const int want = (p & 3) + 4 * (p >> 3), ph = (p >> 2) & 1;  // accumulator and lane half of position p
+                float w = 0.0f;
+#pragma unroll
+                for (int v = 0; v < 16; v++) w = v == want ? s[v] : w;
+                w = __shfl(w, r32 + 32 * ph, 64);
+                const float *vrow = vb + (size_t)(t * kFlashTile + p) * dk;
+                if (t * kFlashTile + p < limit) {
+#pragma unroll
+                    for (int tt = 0; tt < DT; tt++)
+#pragma unroll
+                        for (int v = 0; v < 16; v++) {
+                            const int d = 32 * tt + 8 * (v >> 2) + 4 * h + (v & 3);
+                            const float x = d < dk ? vrow[d] : 0.0f;
+                            if (!__builtin_isfinite(x)) o[tt][v] = __builtin_fmaf(w, x, o[tt][v]);
+                            __builtin_amdgcn_sched_barrier(0);  // rare path: one load at a time, few registers
+                        }
+                }
+            }
+        }
+        if (more) store_v(b ^ 1, &badm[b3 == 2 ? 0 : b3 + 1]);
+        __syncthreads();
+    }
+
+    if (!mine) return;
+    const int qi = rb * 32 + r32;
+    const bool live = qi < a.seq;
+    if (tiles <= f.chunk) {
+        const float inv = 1.0f / l;
+        float *dst = a.out + ((size_t)min(qi, a.seq - 1) * a.n_heads + hq) * dk;
+#pragma unroll
+        for (int tt = 0; tt < DT; tt++)
+#pragma unroll
+            for (int v = 0; v < 16; v += 4) {
+                const int d = 32 * tt + 2 * v + 4 * h;
+                const v4f w = {o[tt][v] * inv, o[tt][v + 1] * inv, o[tt][v + 2] * inv, o[tt][v + 3] * inv};
+                if (live && d < dk) *(v4f *)(dst + d) = w;
+            }
+    } else {
+        // this chunk's state: [kv head][group][chunk][wave][row]: d_k values; (max, sum) behind all of them
+        const size_t at = ((((size_t)g * f.groups + ug) * f.chunks + ch) * kFlashWaves + wave) * 32 + r32;
+        const size_t all = (size_t)a.n_kv * f.groups * f.chunks * kFlashWaves * 32;
+        float *dst = a.part + at * dk;
+#pragma unroll
+        for (int tt = 0; tt < DT; tt++)
+#pragma unroll
+            for (int v = 0; v < 16; v += 4) {
+                const int d = 32 * tt + 2 * v + 4 * h;
+                const v4f w = {o[tt][v], o[tt][v + 1], o[tt][v + 2], o[tt][v + 3]};
+                if (d < dk) *(v4f *)(dst + d) = w;
+            }
+        if (h == 0) {
+            a.part[all * dk + at * 2] = m;
+            a.part[all * dk + at * 2 + 1] = l;
+        }
+    }
+}
+
+// The chunks of one (row, head), half a wave each (four dimensions per lane),
+// merged in chunk order as attn_combine_kernel merges splits (rows with one
+// chunk are written already). VALU-bound: every lane forms the few chunk weights
+// for itself, which is cheaper than one lane forming and handing them round
+// (1024 rows of 32 heads, d_k 128: 24.6 us with a wave per pair).
+__global__ void __launch_bounds__(256) attn_flash_combine_kernel(AttnArgs a, FlashPlan f) {
+    const int lane = threadIdx.x & 31;
+    const int pair = blockIdx.x * 8 + (threadIdx.x >> 5);  // qi * n_heads + head
+    if (pair >= a.seq * a.n_heads) return;
+    const int qi = pair / a.n_heads, hq = pair - qi * a.n_heads;
+    const int g = hq / a.rep, dk = a.d_k;
+    const int U = (a.seq + 31) / 32 * a.rep;
+    const int unit = qi / 32 * a.rep + hq % a.rep;
+    const int ug = unit / kFlashWaves, wave = unit % kFlashWaves;
+    const int last = min(ug * kFlashWaves + kFlashWaves - 1, U - 1);
+    const int kv = a.cache_len + min(a.seq, 32 * (last / a.rep + 1));
+    const int tiles = (kv + kFlashTile - 1) / kFlashTile;
+    if (tiles <= f.chunk) return;
+    // chunks this row sees anything of
+    const int n = (a.cache_len + qi) / (flash_chunk(f, tiles) * kFlashTile) + 1;
+    const size_t base = (((size_t)g * f.groups + ug) * f.chunks * kFlashWaves + wave) * 32 + qi % 32;
+    const size_t step = (size_t)kFlashWaves * 32;  // between chunks
+    const v2f *ml = (const v2f *)(a.part + (size_t)a.n_kv * f.groups * f.chunks * step * dk) + base;
+    const int d = 4 * lane, dc = d < dk ? d : 0;
+    const float *pv = a.part + base * dk + dc;
+    float M = -INFINITY;
+#pragma unroll 4
+    for (int c = 0; c < n; c++) M = fmaxf(M, ml[c * step].x);
+    float L = 0.0f;
+    v4f O = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int c = 0; c < n; c++) {
+        const v2f s = ml[c * step];
+        const v4f v = *(const v4f *)(pv + c * step * dk);
+        const float w = s.x != -INFINITY ? exp_neg(s.x - M) : 0.0f;
+        L = L + s.y * w;
+        O = O + v * w;
+    }
+    const float inv = 1.0f / L;
+    if (d < dk) *(v4f *)(a.out + (size_t)pair * dk + d) = O * inv;
+}
+
 }  // namespace
 
 namespace {
@@ -622,6 +1002,90 @@ void launch_split(const AttnArgs &a, dim3 grid, size_t lds, hipStream_t s) {
     }
 }
 
+namespace {
+sllm_status launch_prep(const AttnArgs &a, hipStream_t s) {
+    const int heads = a.n_heads + a.n_kv, most = (heads + kPrepWaves - 1) / kPrepWaves;
+    const int per_row = a.seq >= 2 * cus_per_device() ? 1 : most;
+    hipLaunchKernelGGL(attn_prep_kernel, dim3(a.seq, per_row), dim3(64 * kPrepWaves), 0, s, a);
+    SLLM_HIP(hipGetLastError());
+    return SLLM_OK;
+}
+}  // namespace
+
+namespace {
+// (query row, kv head) pairs above which a prompt takes attn_flash_kernel: up to
+// there the split kernel's one workgroup per pair all run at once, and its
+// shorter chain wins. Measured (us, split / matrix cores; q heads / kv heads /
+// d_k, rows): 32/8/128 64 13.2 / 21.3, 128 27.7 / 24.7, 1024 884 / 184; 32/32/64
+// 31 26.1 / 18.2 (99 cached), 200 139.5 / 32.5; 9/3/64 128 13.4 / 17.8, 200 23.9
+// / 21.5; 32/4/128 128 23.8 / 28.3, 200 54.7 / 44.8; 16/16/80 64 19.9 / 17.4.
+constexpr int kFlashPairs = 512;
+
+FlashPlan flash_plan(int seq, int n_heads, int n_kv, int d_k, int cache_len, size_t *part) {
+    const int rep = n_heads / n_kv, U = (seq + 31) / 32 * rep;
+    FlashPlan f;
+    f.groups = (U + kFlashWaves - 1) / kFlashWaves;
+    int64_t total = 0;
+    int most = 0;
+    for (int ug = 0; ug < f.groups; ug++) {
+        const int last = ug * kFlashWaves + kFlashWaves - 1 < U - 1 ? ug * kFlashWaves + kFlashWaves - 1 : U - 1;
+        const int rows = 32 * (last / rep + 1) < seq ? 32 * (last / rep + 1) : seq;
+        most = (cache_len + rows + kFlashTile - 1) / kFlashTile;
+        total += most;
+    }
+    // about two workgroups per resident one (two per CU); few tiles in all are cut
+    // to one, two or three each, where a workgroup's fixed cost (first loads, the
+    // merge) weighs against the idle CUs. Measured (us): 32/8/128, 128 rows
+    // with chunks of 1 / 3 24.7 / 35.2; 200 rows 1 / 2 / 3 36.7 / 32.2 / 37.8; 512
+    // rows 2 / 3 / 5 66.0 / 59.8 / 75.5; 1024 rows 3 / 5 / 9 148 / 139 / 149.7
+    const int64_t all = total * n_kv, slots = 2 * (int64_t)tuning().attn_target_blocks;
+    const int64_t c = (all + slots - 1) / slots, least = all > 1024 ? 3 : (all > 128 ? 2 : 1);
+    f.chunk = (int)(c < least ? least : c);
+    for (;; f.chunk *= 2) {
+        f.chunks = (most + f.chunk - 1) / f.chunk;
+        *part = f.chunks > 1 ? (size_t)n_kv * f.groups * f.chunks * kFlashWaves * 32 * (d_k + 2) * sizeof(float) : 0;
+        if (*part <= ((size_t)256 << 20)) return f;
+    }
+}
+
+template <int DT>
+void launch_flash_dt(const AttnArgs &a, const FlashPlan &f, hipStream_t s) {
+    constexpr size_t lds = (size_t)(4 * kFlashTile * (32 * DT + 4) + 4) * sizeof(float);
+    const dim3 grid(a.n_kv, f.groups, f.chunks), block(64 * kFlashWaves);
+    if (a.d_k == 32 * DT) hipLaunchKernelGGL((attn_flash_kernel<DT, true>), grid, block, lds, s, a, f);
+    else hipLaunchKernelGGL((attn_flash_kernel<DT, false>), grid, block, lds, s, a, f);
+}
+}  // namespace
+
+bool attention_flash(int seq, int n_heads, int n_kv, int d_k, int cache_len, const float *out, size_t *ws_bytes) {
+    if ((int64_t)seq * n_kv <= kFlashPairs || d_k > 128 || ((uintptr_t)out & 15) != 0) return false;
+    size_t part = 0;
+    const FlashPlan f = flash_plan(seq, n_heads, n_kv, d_k, cache_len, &part);
+    if (f.groups > 65535 || f.chunks > 65535) return false;  // grid y, z
+    const size_t qrot = (size_t)seq * n_heads * d_k * sizeof(float);
+    *ws_bytes = ((qrot + 255) & ~(size_t)255) + part;
+    return true;
+}
+
+sllm_status launch_attention_flash(const AttnArgs &a, hipStream_t s) {
+    size_t part = 0;
+    const FlashPlan f = flash_plan(a.seq, a.n_heads, a.n_kv, a.d_k, a.cache_len, &part);
+    const sllm_status st = launch_prep(a, s);
+    if (st != SLLM_OK) return st;
+    switch ((a.d_k + 31) / 32) {
+    case 1: launch_flash_dt<1>(a, f, s); break;
+    case 2: launch_flash_dt<2>(a, f, s); break;
+    case 3: launch_flash_dt<3>(a, f, s); break;
+    default: launch_flash_dt<4>(a, f, s); break;
+    }
+    SLLM_HIP(hipGetLastError());
+    if (f.chunks > 1) {
+        hipLaunchKernelGGL(attn_flash_combine_kernel, dim3((a.seq * a.n_heads + 7) / 8), dim3(256), 0, s, a, f);
+        SLLM_HIP(hipGetLastError());
+    }
+    return SLLM_OK;
+}
+
 sllm_status launch_attention(const AttnArgs &a, hipStream_t s) {
     if (a.hs < 1 || a.rep % a.hs) return set_error(SLLM_ERR_ARG, "attention: head slices must divide rep");
     const size_t lds = attn_lds_bytes(a.tw, a.rep, a.rep / a.hs, a.d_k);
@@ -631,8 +1095,8 @@ sllm_status launch_attention(const AttnArgs &a, hipStream_t s) {
         launch_split<true>(b, dim3(a.splits, a.n_kv * a.hs), lds, s);
         SLLM_HIP(hipGetLastError());
     } else {
-        hipLaunchKernelGGL(attn_prep_kernel, dim3(a.seq, a.n_heads + a.n_kv), dim3(64), 0, s, a);
-        SLLM_HIP(hipGetLastError());
+        const sllm_status st = launch_prep(a, s);
+        if (st != SLLM_OK) return st;
         // grid y is (row, kv head, head slice), at most 65535: long prefills
         // run in chunks of rows (every row's k / v is already in the cache)
         const int per = 65535 / (a.n_kv * a.hs);
