@@ -477,7 +477,11 @@ sllm_status with_upload(const void *host, size_t bytes, size_t extra, F fn) {
     return st;
 }
 
-bool uses_gemm(const sllm_weight *w, int x_rows) {
+// bf: whether the bf16 GEMM of the fp32-activation formats may run; false on a
+// stream under capture whose workspace cannot hold what it needs (those calls
+// take the GEMV, which needs none).
+bool uses_gemm(const sllm_weight *w, int x_rows, bool bf) {
+    if (act_f32(w->fmt) && !bf) return false;
     // 0 (the default): the GEMM from 8 activation rows for weights of at least
     // 2^24 elements, from 16 for smaller ones. The GEMV takes up to 4 rows per
     // launch and streams the weight once per launch; the GEMM streams it once.
@@ -512,19 +516,28 @@ int gemm_fmt(const sllm_weight *w) { return w->fmt == SLLM_Q5K1 && w->q5_one_mfm
 // One weight's matmul on device buffers: the GEMV, or the GEMM with the given
 // activation workspace (at least gemm_workspace_bytes).
 sllm_status run_matmul(const sllm_weight *w, const float *x, int x_rows, float *dst, hipStream_t s, void *ws,
-                       size_t cap) {
+                       size_t cap, bool bf) {
     const Planes P = as_const(w->planes);
-    if (!uses_gemm(w, x_rows)) return launch_gemv(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
+    if (!uses_gemm(w, x_rows, bf)) return launch_gemv(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
     return launch_gemm(gemm_fmt(w), P, x, dst, w->rows, w->groups, x_rows, ws, cap, s);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// The workspace bytes of a call, need(bf), and bf: true unless the stream is being
+// captured and its workspace is too small for the bf16 GEMM's share.
+template <class F>
+size_t fit_workspace(hipStream_t s, bool &bf, F need) {
+    const size_t n = need(true);
+    bf = n == 0 || workspace_at_hand(s, n);
+    return bf ? n : need(false);
+}
+
 // GEMM activation workspace the GEMM-bound weights of a set need (the largest).
-size_t multi_gemm_ws(const sllm_weight *const *ws, int count, int x_rows) {
+size_t multi_gemm_ws(const sllm_weight *const *ws, int count, int x_rows, bool bf) {
     size_t need = 0;
     for (int i = 0; i < count; i++)
-        if (uses_gemm(ws[i], x_rows)) {
+        if (uses_gemm(ws[i], x_rows, bf)) {
             const size_t b = gemm_workspace_bytes(gemm_fmt(ws[i]), ws[i]->rows, ws[i]->groups, x_rows);
             need = b > need ? b : need;
         }
@@ -535,15 +548,15 @@ size_t multi_gemm_ws(const sllm_weight *const *ws, int count, int x_rows) {
 // up to kMaxSegs per launch (with the RMSNorm prologue when nw is given);
 // GEMM-bound weights run one by one with the workspace [gws, gws + gcap).
 sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, int x_rows, float *const *dst,
-                       hipStream_t s, void *gws, size_t gcap, const float *nw, float eps) {
+                       hipStream_t s, void *gws, size_t gcap, const float *nw, float eps, bool bf) {
     sllm_status st = SLLM_OK;
     std::vector<char> done((size_t)count, 0);
     for (int i = 0; i < count; i++) {
         if (done[(size_t)i]) continue;
         const sllm_weight *w = ws[i];
-        if (uses_gemm(w, x_rows)) {
+        if (uses_gemm(w, x_rows, bf)) {
             done[(size_t)i] = 1;
-            if ((st = run_matmul(w, x, x_rows, dst[i], s, gws, gcap)) != SLLM_OK) return st;
+            if ((st = run_matmul(w, x, x_rows, dst[i], s, gws, gcap, bf)) != SLLM_OK) return st;
             continue;
         }
         Planes P[kMaxSegs];
@@ -551,7 +564,7 @@ sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, 
         int N[kMaxSegs];
         int n = 0;
         for (int j = i; j < count && n < kMaxSegs; j++) {
-            if (done[(size_t)j] || gemv_fmt(ws[j]) != gemv_fmt(w) || uses_gemm(ws[j], x_rows)) continue;
+            if (done[(size_t)j] || gemv_fmt(ws[j]) != gemv_fmt(w) || uses_gemm(ws[j], x_rows, bf)) continue;
             P[n] = as_const(ws[j]->planes);
             D[n] = dst[j];
             N[n] = ws[j]->rows;
@@ -564,37 +577,37 @@ sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, 
 }
 
 // Whether gate / up fit the one paired GEMV launch.
-bool swiglu_paired(const sllm_weight *wg, const sllm_weight *wu, int x_rows) {
-    return !uses_gemm(wg, x_rows) && !uses_gemm(wu, x_rows) && gemv_fmt(wg) == gemv_fmt(wu);
+bool swiglu_paired(const sllm_weight *wg, const sllm_weight *wu, int x_rows, bool bf) {
+    return !uses_gemm(wg, x_rows, bf) && !uses_gemm(wu, x_rows, bf) && gemv_fmt(wg) == gemv_fmt(wu);
 }
 
 // Workspace the unpaired SwiGLU path needs: the GEMM workspace, then gate / up
 // buffers the caller did not provide.
 size_t swiglu_ws_bytes(const sllm_weight *wg, const sllm_weight *wu, int x_rows, const float *gate,
-                       const float *up) {
-    if (swiglu_paired(wg, wu, x_rows)) return 0;
+                       const float *up, bool bf) {
+    if (swiglu_paired(wg, wu, x_rows, bf)) return 0;
     const sllm_weight *pair[2] = {wg, wu};
     const size_t mm = align256((size_t)x_rows * wg->rows * sizeof(float));
-    return multi_gemm_ws(pair, 2, x_rows) + (gate ? 0 : mm) + (up ? 0 : mm);
+    return multi_gemm_ws(pair, 2, x_rows, bf) + (gate ? 0 : mm) + (up ? 0 : mm);
 }
 
 sllm_status swiglu_impl(const sllm_weight *wg, const sllm_weight *wu, const float *x, int x_rows, float *h,
-                        float *gate, float *up, hipStream_t s, void *ws, const float *nw, float eps) {
+                        float *gate, float *up, hipStream_t s, void *ws, const float *nw, float eps, bool bf) {
     const int N = wg->rows;
-    if (swiglu_paired(wg, wu, x_rows))
+    if (swiglu_paired(wg, wu, x_rows, bf))
         return launch_gemv_swiglu(gemv_fmt(wg), as_const(wg->planes), as_const(wu->planes), x, h, gate, up, N,
                                   wg->groups, x_rows, s, nw, eps);
     // Prefill or mixed formats: the two matmuls, then the elementwise SwiGLU;
     // x is already normed here (nw is only passed for the paired launch).
     const sllm_weight *pair[2] = {wg, wu};
-    const size_t gw = multi_gemm_ws(pair, 2, x_rows);
+    const size_t gw = multi_gemm_ws(pair, 2, x_rows, bf);
     const size_t mm = align256((size_t)x_rows * N * sizeof(float));
     char *tail = (char *)ws + gw;
     float *g = gate ? gate : (float *)tail;
     float *u = up ? up : (float *)(tail + (gate ? 0 : mm));
     sllm_status st;
-    if ((st = run_matmul(wg, x, x_rows, g, s, ws, gw)) != SLLM_OK) return st;
-    if ((st = run_matmul(wu, x, x_rows, u, s, ws, gw)) != SLLM_OK) return st;
+    if ((st = run_matmul(wg, x, x_rows, g, s, ws, gw, bf)) != SLLM_OK) return st;
+    if ((st = run_matmul(wu, x, x_rows, u, s, ws, gw, bf)) != SLLM_OK) return st;
     return launch_swiglu(g, u, h, (size_t)x_rows * N, s);
 }
 
@@ -1007,10 +1020,10 @@ sllm_status sllm_matmul_dev(const sllm_weight *w, const float *x, int x_rows, in
     hipStream_t s = (hipStream_t)stream;
     void *ws = nullptr;
     size_t cap = 0;
-    if (uses_gemm(w, x_rows) && (st = workspace(s, gemm_workspace_bytes(gemm_fmt(w), w->rows, w->groups, x_rows), &ws,
-                                                 &cap)) != SLLM_OK)
-        return st;
-    return run_matmul(w, x, x_rows, dst, s, ws, cap);
+    bool bf = true;
+    const size_t need = fit_workspace(s, bf, [&](bool b) { return multi_gemm_ws(&w, 1, x_rows, b); });
+    if (need && (st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
+    return run_matmul(w, x, x_rows, dst, s, ws, cap, bf);
 }
 
 sllm_status sllm_matmul_argmax_dev(const sllm_weight *w, const float *x, int x_cols, float *logits, int *argmax,
@@ -1055,9 +1068,10 @@ sllm_status sllm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_weight *wu,
     hipStream_t s = (hipStream_t)stream;
     void *ws = nullptr;
     size_t cap = 0;
-    const size_t need = swiglu_ws_bytes(wg, wu, x_rows, gate, up);
+    bool bf = true;
+    const size_t need = fit_workspace(s, bf, [&](bool b) { return swiglu_ws_bytes(wg, wu, x_rows, gate, up, b); });
     if (need && (st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
-    return swiglu_impl(wg, wu, x, x_rows, h, gate, up, s, ws, nullptr, 0.0f);
+    return swiglu_impl(wg, wu, x, x_rows, h, gate, up, s, ws, nullptr, 0.0f, bf);
 }
 
 sllm_status sllm_rmsnorm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_weight *wu, const float *x,
@@ -1071,16 +1085,19 @@ sllm_status sllm_rmsnorm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_wei
     if ((st = ensure_init()) != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     // one row (decode) with a paired gate / up: the norm is the GEMV's prologue
-    if (x_rows == 1 && swiglu_paired(wg, wu, x_rows))
-        return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, nullptr, norm_w, eps);
+    if (x_rows == 1 && swiglu_paired(wg, wu, x_rows, true))
+        return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, nullptr, norm_w, eps, true);
     // several rows / mixed formats: normed rows into the workspace first
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
     void *ws = nullptr;
     size_t cap = 0;
-    if ((st = workspace(s, nb + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr), &ws, &cap)) != SLLM_OK) return st;
+    bool bf = true;
+    const size_t need =
+        fit_workspace(s, bf, [&](bool b) { return nb + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, b); });
+    if ((st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
     float *normed = (float *)ws;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
-    return swiglu_impl(wg, wu, normed, x_rows, h, nullptr, nullptr, s, (char *)ws + nb, nullptr, 0.0f);
+    return swiglu_impl(wg, wu, normed, x_rows, h, nullptr, nullptr, s, (char *)ws + nb, nullptr, 0.0f, bf);
 }
 
 sllm_status sllm_matmul_swiglu_into_f32(const sllm_weight *wg, const sllm_weight *wu, const float *x, int x_rows,
@@ -1139,9 +1156,10 @@ sllm_status sllm_matmul_multi_dev(const sllm_weight *const *ws, int count, const
     hipStream_t s = (hipStream_t)stream;
     void *gws = nullptr;
     size_t cap = 0;
-    const size_t need = multi_gemm_ws(ws, count, x_rows);
+    bool bf = true;
+    const size_t need = fit_workspace(s, bf, [&](bool b) { return multi_gemm_ws(ws, count, x_rows, b); });
     if (need && (st = workspace(s, need, &gws, &cap)) != SLLM_OK) return st;
-    return multi_impl(ws, count, x, x_rows, dst, s, gws, need, nullptr, 0.0f);
+    return multi_impl(ws, count, x, x_rows, dst, s, gws, need, nullptr, 0.0f, bf);
 }
 
 sllm_status sllm_rmsnorm_matmul_multi_dev(const sllm_weight *const *ws, int count, const float *x,
@@ -1154,18 +1172,20 @@ sllm_status sllm_rmsnorm_matmul_multi_dev(const sllm_weight *const *ws, int coun
         return set_error(SLLM_ERR_ARG, "x and the norm weight must be 16-byte aligned");
     if ((st = ensure_init()) != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
-    const size_t gneed = multi_gemm_ws(ws, count, x_rows);
     // one row (decode): the norm is the GEMV's prologue
-    if (x_rows == 1 && gneed == 0) return multi_impl(ws, count, x, x_rows, dst, s, nullptr, 0, norm_w, eps);
+    if (x_rows == 1 && multi_gemm_ws(ws, count, x_rows, true) == 0)
+        return multi_impl(ws, count, x, x_rows, dst, s, nullptr, 0, norm_w, eps, true);
+    const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
+    bool bf = true;
+    const size_t gneed = fit_workspace(s, bf, [&](bool b) { return nb + multi_gemm_ws(ws, count, x_rows, b); }) - nb;
     // several rows: normed rows into the workspace first, then every weight
     // reads them (GEMV and GEMM alike)
-    const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
     void *ws_ = nullptr;
     size_t cap = 0;
     if ((st = workspace(s, nb + gneed, &ws_, &cap)) != SLLM_OK) return st;
     float *normed = (float *)ws_;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
-    return multi_impl(ws, count, normed, x_rows, dst, s, (char *)ws_ + nb, gneed, nullptr, 0.0f);
+    return multi_impl(ws, count, normed, x_rows, dst, s, (char *)ws_ + nb, gneed, nullptr, 0.0f, bf);
 }
 
 sllm_status sllm_rmsnorm_matmul_argmax_dev(const sllm_weight *w, const float *x, const float *norm_w, float eps,
@@ -1346,13 +1366,17 @@ sllm_status sllm_matmul_add_dev(const sllm_weight *w, const float *x, int x_rows
     if (st != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     const Planes P = as_const(w->planes);
-    if (!uses_gemm(w, x_rows)) return launch_gemv_add(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
     // GEMM: the product into the workspace behind the GEMM's own, then dst += it
-    const size_t gb = align256(gemm_workspace_bytes(gemm_fmt(w), w->rows, w->groups, x_rows));
     const size_t n = (size_t)x_rows * w->rows;
+    bool bf = true;
+    const size_t need = fit_workspace(s, bf, [&](bool b) {
+        return uses_gemm(w, x_rows, b) ? multi_gemm_ws(&w, 1, x_rows, b) + n * sizeof(float) : (size_t)0;
+    });
+    if (!need) return launch_gemv_add(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
+    const size_t gb = need - n * sizeof(float);
     void *ws = nullptr;
     size_t cap = 0;
-    if ((st = workspace(s, gb + n * sizeof(float), &ws, &cap)) != SLLM_OK) return st;
+    if ((st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
     float *tmp = (float *)((char *)ws + gb);
     if ((st = launch_gemm(gemm_fmt(w), P, x, tmp, w->rows, w->groups, x_rows, ws, gb, s)) != SLLM_OK) return st;
     return launch_add(dst, tmp, n, s);

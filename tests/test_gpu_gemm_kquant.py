@@ -107,3 +107,24 @@ def test_weights_with_infinite_scales_stay_on_the_gemv(t):
     a = gemm(w, x)
     sq.set_param("gemm_min_rows", 1 << 20)
     assert np.array_equal(a.view(np.uint32), gemm(w, x).view(np.uint32))
+
+
+@pytest.mark.parametrize("t", [10, 11])
+def test_capture_without_workspace_takes_the_gemv(t):
+    # the GEMV needs no workspace: a stream under capture that has none records
+    # it, and the replays equal the eager GEMV bit for bit
+    N, K, M = 96, 512, 9
+    w = sq.load_weight_f32_direct(t, make_kq(t, N, K, 12), N, K)
+    x = torch.from_numpy(make_x(M, K, seed=13)).cuda()
+    y = torch.empty((M, N), device="cuda")
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        sq.matmul_dev(w, x.data_ptr(), M, K, y.data_ptr(), s.cuda_stream)
+    sq.set_param("gemm_min_rows", 1 << 20)
+    want = gemm(w, x.cpu().numpy())
+    for _ in range(3):
+        y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
