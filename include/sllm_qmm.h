@@ -414,8 +414,8 @@ sllm_status sllm_debug_block_dots(const sllm_weight *w, const float *x, int x_ro
                                   int32_t *out);
 
 /*
- * The prefill GEMM's own block dots: runs the int8 matrix-core GEMM (the
- * kernel sllm_matmul uses from gemm_min_rows activation rows on) on x_rows
+ * The prefill GEMM's own block dots: runs the tiled int8 matrix-core GEMM (the
+ * kernel the matmuls use for prompts of more than 32 rows) on x_rows
  * (>= 1) rows against weight rows [row0, row0 + n_rows), and writes every
  * int32 block dot its MFMA instructions returned, from the registers its
  * epilogue scales: out int32 [x_rows][n_rows][groups] (x2 for Q5K1: low,
@@ -448,7 +448,9 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  call path)
  *   gemm_min_rows       >= 0       activation rows from which the GEMM is used (0: 8 for
  *                                  weights of 2^24 elements or more, 16 for smaller ones;
- *                                  Q5_0, Q2K and Q3K: 5 from 2^25 elements, else 8;
+ *                                  Q5_0, Q2K and Q3K: 5 from 2^25 elements, else 8; the
+ *                                  int8 formats 5 where the short-prompt GEMM takes them:
+ *                                  up to 32 rows and 8192 columns (a multiple of 256);
  *                                  the GEMM and GEMV sum a row's blocks in different
  *                                  orders, so a row's last bits can change with it)
  *   gemm_shape          0..5       GEMM workgroups: 1 = 64 x 128 tiles, 2 = 64 x 64 tiles with

@@ -477,11 +477,24 @@ sllm_status with_upload(const void *host, size_t bytes, size_t extra, F fn) {
     return st;
 }
 
-// bf: whether the bf16 GEMM of the fp32-activation formats may run; false on a
-// stream under capture whose workspace cannot hold what it needs (those calls
-// take the GEMV, which needs none).
-bool uses_gemm(const sllm_weight *w, int x_rows, bool bf) {
-    if (act_f32(w->fmt) && !bf) return false;
+// How the matmuls of one call may run. ws: the bf16 GEMM of the fp32-activation
+// formats and the short-prompt GEMM may; false on a stream under capture whose
+// workspace cannot hold what they need (those calls take the GEMV, which needs
+// none, or the tiled GEMM). rows: output rows of all the call's weights (the
+// short-prompt GEMM's launch).
+struct Route {
+    bool ws = true;
+    int64_t rows = 0;
+};
+
+// The short-prompt GEMM takes a weight's rows (an explicit tile shape or K split
+// asks for the tiled GEMM).
+bool sgemm_route(const sllm_weight *w, int x_rows, const Route &r) {
+    return r.ws && sgemm_supported(w->fmt, w->groups, x_rows, r.rows) && !tuning().gemm_shape && !tuning().gemm_splits;
+}
+
+bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
+    if (act_f32(w->fmt) && !r.ws) return false;
     // 0 (the default): the GEMM from 8 activation rows for weights of at least
     // 2^24 elements, from 16 for smaller ones. The GEMV takes up to 4 rows per
     // launch and streams the weight once per launch; the GEMM streams it once.
@@ -496,6 +509,10 @@ bool uses_gemm(const sllm_weight *w, int x_rows, bool bf) {
     // M = 8 27.2 / 25; Q5_0 1536x768 at M = 8 11.2 / 11.5, M = 12 16.4 / 11.8.
     int min_rows = tuning().gemm_min_rows;
     if (min_rows == 0 && act_f32(w->fmt)) min_rows = (int64_t)w->rows * w->cols >= ((int64_t)1 << 25) ? 5 : 8;
+    // The short-prompt GEMM from 5 rows, where the GEMV takes a second launch
+    // (GEMV / GEMM: Q4_1 14336x4096 at M = 4 17.6 / 21.4, M = 5 25.0 / 20.9, Q8_0
+    // 1536x768 5.5 / 8.0 and 8.0 / 8.1, Q5K1 4096x4096 9.9 / 14.9 and 15.1 / 14.9).
+    if (min_rows == 0 && sgemm_route(w, x_rows, r)) min_rows = 5;
     if (min_rows == 0) min_rows = (int64_t)w->rows * w->cols >= ((int64_t)1 << 24) ? 8 : 16;
     if (kq_native(w->fmt) && !w->kq_gemm) return false;
     return x_rows >= min_rows && gemm_supported(w->fmt, w->groups);
@@ -513,50 +530,93 @@ int gemv_fmt(const sllm_weight *w) {
 // 16 times its low ones runs as one MFMA per block (SLLM_Q5K1F).
 int gemm_fmt(const sllm_weight *w) { return w->fmt == SLLM_Q5K1 && w->q5_one_mfma ? SLLM_Q5K1F : w->fmt; }
 
+bool uses_sgemm(const sllm_weight *w, int x_rows, const Route &r) {
+    return sgemm_route(w, x_rows, r) && uses_gemm(w, x_rows, r);
+}
+int64_t total_rows(const sllm_weight *const *ws, int count) {
+    int64_t n = 0;
+    for (int i = 0; i < count; i++) n += ws[i]->rows;
+    return n;
+}
+bool all_sgemm(const sllm_weight *const *ws, int count, int x_rows, const Route &r) {
+    for (int i = 0; i < count; i++)
+        if (!uses_sgemm(ws[i], x_rows, r)) return false;
+    return true;
+}
+
 // One weight's matmul on device buffers: the GEMV, or the GEMM with the given
 // activation workspace (at least gemm_workspace_bytes).
 sllm_status run_matmul(const sllm_weight *w, const float *x, int x_rows, float *dst, hipStream_t s, void *ws,
-                       size_t cap, bool bf) {
+                       size_t cap, const Route &r) {
     const Planes P = as_const(w->planes);
-    if (!uses_gemm(w, x_rows, bf)) return launch_gemv(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
+    if (!uses_gemm(w, x_rows, r)) return launch_gemv(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
+    if (uses_sgemm(w, x_rows, r)) {
+        const sllm_status st = launch_sact(x, nullptr, 0.0f, x_rows, w->groups, ws, s);
+        if (st != SLLM_OK) return st;
+        return launch_sgemm(gemm_fmt(w), &P, &dst, &w->rows, 1, 0, w->groups, x_rows, ws, s);
+    }
     return launch_gemm(gemm_fmt(w), P, x, dst, w->rows, w->groups, x_rows, ws, cap, s);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// The workspace bytes of a call, need(bf), and bf: true unless the stream is being
-// captured and its workspace is too small for the bf16 GEMM's share.
+// The workspace bytes of a call, need(); r.ws is cleared where the stream is being
+// captured and its workspace is too small.
 template <class F>
-size_t fit_workspace(hipStream_t s, bool &bf, F need) {
-    const size_t n = need(true);
-    bf = n == 0 || workspace_at_hand(s, n);
-    return bf ? n : need(false);
+size_t fit_workspace(hipStream_t s, Route &r, F need) {
+    const size_t n = need();
+    r.ws = n == 0 || workspace_at_hand(s, n);
+    return r.ws ? n : need();
 }
 
 // GEMM activation workspace the GEMM-bound weights of a set need (the largest).
-size_t multi_gemm_ws(const sllm_weight *const *ws, int count, int x_rows, bool bf) {
+size_t multi_gemm_ws(const sllm_weight *const *ws, int count, int x_rows, const Route &r) {
     size_t need = 0;
     for (int i = 0; i < count; i++)
-        if (uses_gemm(ws[i], x_rows, bf)) {
-            const size_t b = gemm_workspace_bytes(gemm_fmt(ws[i]), ws[i]->rows, ws[i]->groups, x_rows);
+        if (uses_gemm(ws[i], x_rows, r)) {
+            const size_t b = uses_sgemm(ws[i], x_rows, r)
+                                 ? sgemm_act_bytes(ws[i]->groups)
+                                 : gemm_workspace_bytes(gemm_fmt(ws[i]), ws[i]->rows, ws[i]->groups, x_rows);
             need = b > need ? b : need;
         }
     return align256(need);
 }
 
 // Weights sharing the activation rows x. GEMV weights are grouped by format,
-// up to kMaxSegs per launch (with the RMSNorm prologue when nw is given);
-// GEMM-bound weights run one by one with the workspace [gws, gws + gcap).
+// up to kMaxSegs per launch (with the RMSNorm prologue when nw is given), and so
+// are the short-prompt GEMM's, whose activations are quantized once (nw is only
+// given when every weight is one of these two); other GEMM-bound weights run one
+// by one with the workspace [gws, gws + gcap).
 sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, int x_rows, float *const *dst,
-                       hipStream_t s, void *gws, size_t gcap, const float *nw, float eps, bool bf) {
+                       hipStream_t s, void *gws, size_t gcap, const float *nw, float eps, const Route &r) {
     sllm_status st = SLLM_OK;
     std::vector<char> done((size_t)count, 0);
+    bool quantized = false;
+    for (int i = 0; i < count; i++) {
+        if (done[(size_t)i] || !uses_sgemm(ws[i], x_rows, r)) continue;
+        const sllm_weight *w = ws[i];
+        if (!quantized && (st = launch_sact(x, nw, eps, x_rows, w->groups, gws, s)) != SLLM_OK) return st;
+        quantized = true;
+        Planes P[kMaxSegs];
+        float *D[kMaxSegs];
+        int N[kMaxSegs];
+        int n = 0;
+        for (int j = i; j < count && n < kMaxSegs; j++) {
+            if (done[(size_t)j] || !uses_sgemm(ws[j], x_rows, r) || gemm_fmt(ws[j]) != gemm_fmt(w)) continue;
+            P[n] = as_const(ws[j]->planes);
+            D[n] = dst[j];
+            N[n] = ws[j]->rows;
+            n++;
+            done[(size_t)j] = 1;
+        }
+        if ((st = launch_sgemm(gemm_fmt(w), P, D, N, n, 0, w->groups, x_rows, gws, s)) != SLLM_OK) return st;
+    }
     for (int i = 0; i < count; i++) {
         if (done[(size_t)i]) continue;
         const sllm_weight *w = ws[i];
-        if (uses_gemm(w, x_rows, bf)) {
+        if (uses_gemm(w, x_rows, r)) {
             done[(size_t)i] = 1;
-            if ((st = run_matmul(w, x, x_rows, dst[i], s, gws, gcap, bf)) != SLLM_OK) return st;
+            if ((st = run_matmul(w, x, x_rows, dst[i], s, gws, gcap, r)) != SLLM_OK) return st;
             continue;
         }
         Planes P[kMaxSegs];
@@ -564,7 +624,7 @@ sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, 
         int N[kMaxSegs];
         int n = 0;
         for (int j = i; j < count && n < kMaxSegs; j++) {
-            if (done[(size_t)j] || gemv_fmt(ws[j]) != gemv_fmt(w) || uses_gemm(ws[j], x_rows, bf)) continue;
+            if (done[(size_t)j] || gemv_fmt(ws[j]) != gemv_fmt(w) || uses_gemm(ws[j], x_rows, r)) continue;
             P[n] = as_const(ws[j]->planes);
             D[n] = dst[j];
             N[n] = ws[j]->rows;
@@ -577,37 +637,49 @@ sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, 
 }
 
 // Whether gate / up fit the one paired GEMV launch.
-bool swiglu_paired(const sllm_weight *wg, const sllm_weight *wu, int x_rows, bool bf) {
-    return !uses_gemm(wg, x_rows, bf) && !uses_gemm(wu, x_rows, bf) && gemv_fmt(wg) == gemv_fmt(wu);
+bool swiglu_paired(const sllm_weight *wg, const sllm_weight *wu, int x_rows, const Route &r) {
+    return !uses_gemm(wg, x_rows, r) && !uses_gemm(wu, x_rows, r) && gemv_fmt(wg) == gemv_fmt(wu);
 }
 
 // Workspace the unpaired SwiGLU path needs: the GEMM workspace, then gate / up
 // buffers the caller did not provide.
+bool swiglu_sgemm(const sllm_weight *wg, const sllm_weight *wu, int x_rows, const Route &r) {
+    return uses_sgemm(wg, x_rows, r) && uses_sgemm(wu, x_rows, r) && gemm_fmt(wg) == gemm_fmt(wu);
+}
 size_t swiglu_ws_bytes(const sllm_weight *wg, const sllm_weight *wu, int x_rows, const float *gate,
-                       const float *up, bool bf) {
-    if (swiglu_paired(wg, wu, x_rows, bf)) return 0;
+                       const float *up, const Route &r) {
+    if (swiglu_paired(wg, wu, x_rows, r)) return 0;
+    if (swiglu_sgemm(wg, wu, x_rows, r)) return sgemm_act_bytes(wg->groups);
     const sllm_weight *pair[2] = {wg, wu};
     const size_t mm = align256((size_t)x_rows * wg->rows * sizeof(float));
-    return multi_gemm_ws(pair, 2, x_rows, bf) + (gate ? 0 : mm) + (up ? 0 : mm);
+    return multi_gemm_ws(pair, 2, x_rows, r) + (gate ? 0 : mm) + (up ? 0 : mm);
 }
 
 sllm_status swiglu_impl(const sllm_weight *wg, const sllm_weight *wu, const float *x, int x_rows, float *h,
-                        float *gate, float *up, hipStream_t s, void *ws, const float *nw, float eps, bool bf) {
+                        float *gate, float *up, hipStream_t s, void *ws, const float *nw, float eps, const Route &r) {
     const int N = wg->rows;
-    if (swiglu_paired(wg, wu, x_rows, bf))
+    if (swiglu_paired(wg, wu, x_rows, r))
         return launch_gemv_swiglu(gemv_fmt(wg), as_const(wg->planes), as_const(wu->planes), x, h, gate, up, N,
                                   wg->groups, x_rows, s, nw, eps);
+    if (swiglu_sgemm(wg, wu, x_rows, r)) {
+        const sllm_status st = launch_sact(x, nw, eps, x_rows, wg->groups, ws, s);
+        if (st != SLLM_OK) return st;
+        const Planes P[2] = {as_const(wg->planes), as_const(wu->planes)};
+        float *const D[3] = {h, gate, up};
+        const int Ns[2] = {N, N};
+        return launch_sgemm(gemm_fmt(wg), P, D, Ns, 2, 2, wg->groups, x_rows, ws, s);
+    }
     // Prefill or mixed formats: the two matmuls, then the elementwise SwiGLU;
-    // x is already normed here (nw is only passed for the paired launch).
+    // x is already normed here (nw is only passed for the one-launch forms).
     const sllm_weight *pair[2] = {wg, wu};
-    const size_t gw = multi_gemm_ws(pair, 2, x_rows, bf);
+    const size_t gw = multi_gemm_ws(pair, 2, x_rows, r);
     const size_t mm = align256((size_t)x_rows * N * sizeof(float));
     char *tail = (char *)ws + gw;
     float *g = gate ? gate : (float *)tail;
     float *u = up ? up : (float *)(tail + (gate ? 0 : mm));
     sllm_status st;
-    if ((st = run_matmul(wg, x, x_rows, g, s, ws, gw, bf)) != SLLM_OK) return st;
-    if ((st = run_matmul(wu, x, x_rows, u, s, ws, gw, bf)) != SLLM_OK) return st;
+    if ((st = run_matmul(wg, x, x_rows, g, s, ws, gw, r)) != SLLM_OK) return st;
+    if ((st = run_matmul(wu, x, x_rows, u, s, ws, gw, r)) != SLLM_OK) return st;
     return launch_swiglu(g, u, h, (size_t)x_rows * N, s);
 }
 
@@ -1020,10 +1092,10 @@ sllm_status sllm_matmul_dev(const sllm_weight *w, const float *x, int x_rows, in
     hipStream_t s = (hipStream_t)stream;
     void *ws = nullptr;
     size_t cap = 0;
-    bool bf = true;
-    const size_t need = fit_workspace(s, bf, [&](bool b) { return multi_gemm_ws(&w, 1, x_rows, b); });
+    Route r{true, w->rows};
+    const size_t need = fit_workspace(s, r, [&] { return multi_gemm_ws(&w, 1, x_rows, r); });
     if (need && (st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
-    return run_matmul(w, x, x_rows, dst, s, ws, cap, bf);
+    return run_matmul(w, x, x_rows, dst, s, ws, cap, r);
 }
 
 sllm_status sllm_matmul_argmax_dev(const sllm_weight *w, const float *x, int x_cols, float *logits, int *argmax,
@@ -1068,10 +1140,10 @@ sllm_status sllm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_weight *wu,
     hipStream_t s = (hipStream_t)stream;
     void *ws = nullptr;
     size_t cap = 0;
-    bool bf = true;
-    const size_t need = fit_workspace(s, bf, [&](bool b) { return swiglu_ws_bytes(wg, wu, x_rows, gate, up, b); });
+    Route r{true, 2 * (int64_t)wg->rows};
+    const size_t need = fit_workspace(s, r, [&] { return swiglu_ws_bytes(wg, wu, x_rows, gate, up, r); });
     if (need && (st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
-    return swiglu_impl(wg, wu, x, x_rows, h, gate, up, s, ws, nullptr, 0.0f, bf);
+    return swiglu_impl(wg, wu, x, x_rows, h, gate, up, s, ws, nullptr, 0.0f, r);
 }
 
 sllm_status sllm_rmsnorm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_weight *wu, const float *x,
@@ -1085,19 +1157,22 @@ sllm_status sllm_rmsnorm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_wei
     if ((st = ensure_init()) != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     // one row (decode) with a paired gate / up: the norm is the GEMV's prologue
-    if (x_rows == 1 && swiglu_paired(wg, wu, x_rows, true))
-        return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, nullptr, norm_w, eps, true);
+    if (x_rows == 1 && swiglu_paired(wg, wu, x_rows, Route{}))
+        return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, nullptr, norm_w, eps, Route{});
     // several rows / mixed formats: normed rows into the workspace first
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
     void *ws = nullptr;
     size_t cap = 0;
-    bool bf = true;
-    const size_t need =
-        fit_workspace(s, bf, [&](bool b) { return nb + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, b); });
+    Route r{true, 2 * (int64_t)wg->rows};
+    const size_t need = fit_workspace(s, r, [&] {
+        return (swiglu_sgemm(wg, wu, x_rows, r) ? 0 : nb) + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, r);
+    });
     if ((st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
+    if (swiglu_sgemm(wg, wu, x_rows, r))  // normed as they are quantized
+        return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, ws, norm_w, eps, r);
     float *normed = (float *)ws;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
-    return swiglu_impl(wg, wu, normed, x_rows, h, nullptr, nullptr, s, (char *)ws + nb, nullptr, 0.0f, bf);
+    return swiglu_impl(wg, wu, normed, x_rows, h, nullptr, nullptr, s, (char *)ws + nb, nullptr, 0.0f, r);
 }
 
 sllm_status sllm_matmul_swiglu_into_f32(const sllm_weight *wg, const sllm_weight *wu, const float *x, int x_rows,
@@ -1156,10 +1231,10 @@ sllm_status sllm_matmul_multi_dev(const sllm_weight *const *ws, int count, const
     hipStream_t s = (hipStream_t)stream;
     void *gws = nullptr;
     size_t cap = 0;
-    bool bf = true;
-    const size_t need = fit_workspace(s, bf, [&](bool b) { return multi_gemm_ws(ws, count, x_rows, b); });
+    Route r{true, total_rows(ws, count)};
+    const size_t need = fit_workspace(s, r, [&] { return multi_gemm_ws(ws, count, x_rows, r); });
     if (need && (st = workspace(s, need, &gws, &cap)) != SLLM_OK) return st;
-    return multi_impl(ws, count, x, x_rows, dst, s, gws, need, nullptr, 0.0f, bf);
+    return multi_impl(ws, count, x, x_rows, dst, s, gws, need, nullptr, 0.0f, r);
 }
 
 sllm_status sllm_rmsnorm_matmul_multi_dev(const sllm_weight *const *ws, int count, const float *x,
@@ -1173,19 +1248,23 @@ sllm_status sllm_rmsnorm_matmul_multi_dev(const sllm_weight *const *ws, int coun
     if ((st = ensure_init()) != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     // one row (decode): the norm is the GEMV's prologue
-    if (x_rows == 1 && multi_gemm_ws(ws, count, x_rows, true) == 0)
-        return multi_impl(ws, count, x, x_rows, dst, s, nullptr, 0, norm_w, eps, true);
+    if (x_rows == 1 && multi_gemm_ws(ws, count, x_rows, Route{}) == 0)
+        return multi_impl(ws, count, x, x_rows, dst, s, nullptr, 0, norm_w, eps, Route{});
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
-    bool bf = true;
-    const size_t gneed = fit_workspace(s, bf, [&](bool b) { return nb + multi_gemm_ws(ws, count, x_rows, b); }) - nb;
+    Route r{true, total_rows(ws, count)};
+    const size_t need = fit_workspace(s, r, [&] {
+        return (all_sgemm(ws, count, x_rows, r) ? 0 : nb) + multi_gemm_ws(ws, count, x_rows, r);
+    });
     // several rows: normed rows into the workspace first, then every weight
     // reads them (GEMV and GEMM alike)
     void *ws_ = nullptr;
     size_t cap = 0;
-    if ((st = workspace(s, nb + gneed, &ws_, &cap)) != SLLM_OK) return st;
+    if ((st = workspace(s, need, &ws_, &cap)) != SLLM_OK) return st;
+    if (all_sgemm(ws, count, x_rows, r))  // normed as they are quantized
+        return multi_impl(ws, count, x, x_rows, dst, s, ws_, need, norm_w, eps, r);
     float *normed = (float *)ws_;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
-    return multi_impl(ws, count, normed, x_rows, dst, s, (char *)ws_ + nb, gneed, nullptr, 0.0f, bf);
+    return multi_impl(ws, count, normed, x_rows, dst, s, (char *)ws_ + nb, need - nb, nullptr, 0.0f, r);
 }
 
 sllm_status sllm_rmsnorm_matmul_argmax_dev(const sllm_weight *w, const float *x, const float *norm_w, float eps,
@@ -1368,15 +1447,22 @@ sllm_status sllm_matmul_add_dev(const sllm_weight *w, const float *x, int x_rows
     const Planes P = as_const(w->planes);
     // GEMM: the product into the workspace behind the GEMM's own, then dst += it
     const size_t n = (size_t)x_rows * w->rows;
-    bool bf = true;
-    const size_t need = fit_workspace(s, bf, [&](bool b) {
-        return uses_gemm(w, x_rows, b) ? multi_gemm_ws(&w, 1, x_rows, b) + n * sizeof(float) : (size_t)0;
+    // (its epilogue saves the tiled GEMM's add pass: worth it for few rows too)
+    Route r{true, w->rows > 2048 ? w->rows : 2048};
+    const size_t need = fit_workspace(s, r, [&] {
+        return uses_gemm(w, x_rows, r)
+                   ? multi_gemm_ws(&w, 1, x_rows, r) + (uses_sgemm(w, x_rows, r) ? 0 : n * sizeof(float))
+                   : (size_t)0;
     });
     if (!need) return launch_gemv_add(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
-    const size_t gb = need - n * sizeof(float);
     void *ws = nullptr;
     size_t cap = 0;
     if ((st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
+    if (uses_sgemm(w, x_rows, r)) {  // adds in its epilogue
+        if ((st = launch_sact(x, nullptr, 0.0f, x_rows, w->groups, ws, s)) != SLLM_OK) return st;
+        return launch_sgemm(gemm_fmt(w), &P, &dst, &w->rows, 1, 1, w->groups, x_rows, ws, s);
+    }
+    const size_t gb = need - n * sizeof(float);
     float *tmp = (float *)((char *)ws + gb);
     if ((st = launch_gemm(gemm_fmt(w), P, x, tmp, w->rows, w->groups, x_rows, ws, gb, s)) != SLLM_OK) return st;
     return launch_add(dst, tmp, n, s);

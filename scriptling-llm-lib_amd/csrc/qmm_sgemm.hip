@@ -1,0 +1,497 @@
+// Short-prompt GEMM (up to 32 activation rows) of the int8 formats: Q8_0, Q4_0,
+// Q4_1, Q5K1 on the int8 matrix cores, several weights that share their input in
+// one launch, the residual add or the SwiGLU in its epilogue.
+//
+// What bounds a short prompt: the weight stream (each weight is read once), and
+// before that the launches around it. The tiled GEMM (qmm_gemm.hip) staged
+// weights through LDS with a barrier per 128 columns of K and needed a quantize
+// pass per weight, a split reduction per weight and an elementwise pass after.
+// Here
+// * sact_kernel norms (optionally) and quantizes the rows once per input, with
+//   the GEMV prologue's routines, into MFMA lane order;
+// * a wave streams 32 weight rows over its share of K, eight blocks (one 128-byte
+//   line of a row's codes) at a time: eight lanes load a row's line, a wave-private
+//   LDS image hands every lane its own row, the next eight blocks in flight, no
+//   barrier. (Each lane loading its own row's line read it in pieces: 14336x4096
+//   Q4_1 at M = 32 25.3 us, 34.9 with non-temporal loads, which fetch the line
+//   again for every piece.)
+// * the W waves of a workgroup split K between them and meet in LDS once, in
+//   wave order, where the epilogue is applied: one launch, no partials in memory.
+// The per-block arithmetic is the tiled GEMM's: v_mfma_i32_32x32x32_i8 gives a
+// block's exact dots on top of 1.5 * 2^23, t = fma(F, d, -1.5 * 2^23 d), acc =
+// fma(t, xs, acc), min terms two blocks at a time through v_mfma_f32_32x32x2_f32;
+// eight blocks that hold a non-finite scale, or an activation scale from 2^90,
+// are computed in the reference's operation order (qmm_gemm.hip has the reasons).
+#include <hip/hip_runtime.h>
+
+#include "qmm_device.hpp"
+#include "qmm_internal.hpp"
+
+namespace sllm {
+
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kMagicBits = 0x4B400000;  // 1.5 * 2^23
+constexpr float kMagic = 12582912.0f;
+constexpr float kHugeXs = 0x1p90f;
+constexpr int kCh = 8;  // blocks per chunk
+
+__host__ __device__ constexpr bool has_min(int f) { return f == SLLM_Q4_1 || f == SLLM_Q5K1 || f == SLLM_Q5K1F; }
+__host__ __device__ constexpr bool dual(int f) { return f == SLLM_Q5K1; }
+__host__ __device__ constexpr bool has_hb(int f) { return f == SLLM_Q5K1 || f == SLLM_Q5K1F; }
+
+// Quantized activations, 32 rows (rows past M: zeros):
+//   xq [g][lane][16]  codes: lane r + 32 h, elements 16 h .. of row r
+//   xs, xm, sx [g][32]  scale, float(Σxq) * scale, Σxq
+struct SAct {
+    int8_t *xq;
+    float *xs, *xm;
+    int *sx;
+};
+
+__host__ inline size_t sact_bytes(int G) { return (size_t)G * (1024 + 3 * 128); }
+__host__ inline SAct carve_sact(void *ws, int G) {
+    const size_t n = (size_t)G;
+    SAct a;
+    a.xq = (int8_t *)ws;
+    a.xs = (float *)(a.xq + n * 1024);
+    a.xm = a.xs + n * 32;
+    a.sx = (int *)(a.xm + n * 32);
+    return a;
+}
+
+// Statistics of rmsNormFlatF32 as the GEMV prologue forms them (qmm_gemv_kernel.hpp
+// rms_load / rms_finish): 256 slots, slot s adds v * v over x[s], x[s + 256], ... in
+// order, wave sums of 64 slots, added left to right.
+__device__ __forceinline__ float row_inv(const float *xr, int K, float eps, float *red) {
+    const int t = threadIdx.x;
+    float p = 0.0f;
+    for (int i = t; i < K; i += 16 * 256) {
+        float v[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) v[k] = i + k * 256 < K ? xr[i + k * 256] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; k++) p = p + v[k] * v[k];
+    }
+    const float w = wave_sum(p);
+    if ((t & 63) == 0) red[t >> 6] = w;
+    __syncthreads();
+    const float ss = ((red[0] + red[1]) + red[2]) + red[3];
+    const double q = (K & (K - 1)) == 0 ? (double)ss * (1.0 / (double)K) : (double)ss / (double)K;
+    return 1.0f / (float)sqrt(q + (double)eps);
+}
+
+// One workgroup of 256 threads per row (grid: 32); eight lanes per
+// block. The first four blocks of a lane's group are loaded before the row's
+// statistics are waited for (one memory round trip up to K = 4096).
+__global__ void __launch_bounds__(256) sact_kernel(const float *__restrict__ x, const float *__restrict__ nw,
+                                                   float eps, int M, int G, SAct a) {
+    __shared__ float red[4];
+    const int r = blockIdx.x;
+    const bool live = r < M;
+    const float *xr = x + (size_t)(live ? r : M - 1) * G * 32;
+    const int sub = threadIdx.x & 7, b0 = threadIdx.x >> 3;
+    float4 v[4], w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int g = min(b0 + 32 * i, G - 1);
+        v[i] = ((const float4 *)(xr + (size_t)g * 32))[sub];
+        if (nw) w[i] = ((const float4 *)(nw + (size_t)g * 32))[sub];
+    }
+    const float inv = nw ? row_inv(xr, G * 32, eps, red) : 0.0f;
+    auto put = [&](int g, float4 u, const float4 &c) {
+        if (nw) u = make_float4((u.x * inv) * c.x, (u.y * inv) * c.y, (u.z * inv) * c.z, (u.w * inv) * c.w);
+        if (!live) u = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        int q[1];
+        float s;
+        int sm;
+        quantize_part<8>(&u, q, s, sm);
+        const size_t t = (size_t)g;
+        // word sub of the block: lane half sub / 4, word sub % 4 of its 16 bytes
+        ((int *)(a.xq + t * 1024 + (r + 32 * (sub >> 2)) * 16))[sub & 3] = q[0];
+        if (sub == 0) {
+            a.xs[t * 32 + r] = s;
+            a.xm[t * 32 + r] = (float)sm * s;
+            a.sx[t * 32 + r] = sm;
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (b0 + 32 * i < G) put(b0 + 32 * i, v[i], w[i]);
+    for (int g = b0 + 128; g < G; g += 32) {
+        const float4 u = ((const float4 *)(xr + (size_t)g * 32))[sub];
+        const float4 c = nw ? ((const float4 *)(nw + (size_t)g * 32))[sub] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        put(g, u, c);
+    }
+}
+
+// The weights of one launch: segment s owns the column tiles [tile0[s], tile0[s +
+// 1]). Mode kPair: P[0] / P[1] are gate / up of one FFN, dst[0] receives the SwiGLU,
+// dst[1] / dst[2] (optional) the two products.
+enum SMode { kStore = 0, kAdd = 1, kPair = 2 };
+struct SegG {
+    Planes P[kMaxSegs];
+    float *dst[kMaxSegs];
+    int N[kMaxSegs];
+    int tile0[kMaxSegs + 1];
+    int n, mode;
+};
+
+// One chunk (kCh blocks x 32 weight rows) as a wave loads it: codes, lane l block
+// l % 8 of rows 8 i + l / 8; high bits, lane l words 4 (l % 2) .. of row l / 2;
+// scales, lanes 0..31 d and 32..63 m of row l % 32.
+template <int FMT>
+struct Chunk {
+    static constexpr bool Q8 = FMT == SLLM_Q8_0;
+    v4i q[Q8 ? 8 : 4];
+    v4i sc, dh, hb;
+};
+// Its wave-private LDS image; rows padded so that lanes reading their own rows hit
+// distinct banks.
+template <int FMT>
+struct alignas(16) Image {
+    static constexpr int PL = FMT == SLLM_Q8_0 ? 2 : 1;
+    v4i q[PL][32][kCh + 1];
+    v4i sc[2][32];
+    v4i dh[dual(FMT) ? 32 : 1];
+    v4i hb[has_hb(FMT) ? 32 : 1][3];
+    v4i a[kCh][64];  // the activation codes, lane's own
+    float xs[kCh][32];
+};
+
+template <int FMT>
+__device__ __forceinline__ void load_chunk(Chunk<FMT> &c, const Planes &P, int n0, int N, int G, int g, int lane) {
+    const int b = lane & 7;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const size_t at = (size_t)min(n0 + 8 * i + (lane >> 3), N - 1) * G + g + b;
+        c.q[i] = *(const v4i *)(P.qs + at);
+        if (FMT == SLLM_Q8_0) c.q[FMT == SLLM_Q8_0 ? 4 + i : 0] = *(const v4i *)(P.qs2 + at);
+    }
+    const size_t row = (size_t)min(n0 + (lane & 31), N - 1) * G + g;
+    c.sc = *(const v4i *)((has_min(FMT) && lane >= 32 ? P.m : P.d) + row);
+    if (dual(FMT)) c.dh = *(const v4i *)(P.dh + row);
+    if (has_hb(FMT)) c.hb = *(const v4i *)(P.qh + (size_t)min(n0 + (lane >> 1), N - 1) * G + g + 4 * (lane & 1));
+}
+
+template <int FMT>
+__device__ __forceinline__ void put_chunk(const Chunk<FMT> &c, Image<FMT> &I, int lane) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        I.q[0][8 * i + (lane >> 3)][lane & 7] = c.q[i];
+        if (FMT == SLLM_Q8_0) I.q[FMT == SLLM_Q8_0 ? 1 : 0][8 * i + (lane >> 3)][lane & 7] = c.q[FMT == SLLM_Q8_0 ? 4 + i : 0];
+    }
+    I.sc[lane >> 5][lane & 31] = c.sc;
+    if (dual(FMT)) I.dh[dual(FMT) ? lane & 31 : 0] = c.dh;
+    if (has_hb(FMT)) I.hb[has_hb(FMT) ? lane >> 1 : 0][lane & 1] = c.hb;
+}
+
+__device__ __forceinline__ uint16_t half_of(const v2u &v, int b) { return (uint16_t)(v[b >> 1] >> (16 * (b & 1))); }
+// any of the eight f16 values not finite
+__device__ __forceinline__ bool any_nonfinite(const v4i &v) {
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t u = (uint32_t)v[i];
+        bad |= (u & 0x7c00u) == 0x7c00u || (u & 0x7c000000u) == 0x7c000000u;
+    }
+    return bad;
+}
+
+// Block b's codes as the MFMA's B operand (lane half h: elements 16 h ..).
+template <int FMT>
+__device__ __forceinline__ void operand(const Image<FMT> &I, int b, int r32, int h, v4i &q, v4i &qh) {
+    if (FMT == SLLM_Q8_0) {
+        q = I.q[FMT == SLLM_Q8_0 ? h : 0][r32][b];
+        return;
+    }
+    const v4i w = I.q[0][r32][b];
+    const int sh = 4 * h;
+    const uint32_t hb = has_hb(FMT) ? (uint32_t)((const int *)I.hb[has_hb(FMT) ? r32 : 0])[b] >> sh : 0u;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        int t = (int)((uint32_t)w[k] >> sh) & 0x0f0f0f0f;
+        if (FMT == SLLM_Q4_0) t = ((t | (int)0x80808080) - 0x08080808) ^ (int)0x80808080;  // nib - 8 per byte
+        if (has_hb(FMT)) {
+            // high bits in group order: (hb >> k) & 0x01010101 are elements 4 k ..
+            const int bits = (int)((hb >> k) & 0x01010101u);
+            if (FMT == SLLM_Q5K1F) t |= bits << 4;
+            else qh[k] = bits;
+        }
+        q[k] = t;
+    }
+}
+
+// The activation scales of a lane's 16 rows of block b.
+template <int FMT>
+__device__ __forceinline__ void read_xs(const Image<FMT> &I, int b, int h, float (&xv)[16]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const v4f u = *(const v4f *)(I.xs[b] + 8 * i + 4 * h);
+#pragma unroll
+        for (int k = 0; k < 4; k++) xv[4 * i + k] = u[k];
+    }
+}
+
+// Grid: column tiles of 32; W waves.
+// LDS: every wave's image of its current chunk, then (after a barrier) the waves'
+// sums.
+template <int FMT, int W>
+__global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, int G) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool pair = S.mode == kPair;
+    const int KW = pair ? W / 2 : W;              // waves that split K
+    const int kw = pair ? wave % (W / 2) : wave;  // this wave's place among them
+    // the workgroup's segment (uniform)
+    int seg = 0;
+#pragma unroll
+    for (int s = 1; s < kMaxSegs; s++)
+        if (s < S.n && (int)blockIdx.x >= S.tile0[s]) seg = s;
+    Planes P = S.P[0];
+    int N = S.N[0];
+#pragma unroll
+    for (int s = 1; s < kMaxSegs; s++)
+        if (s == (pair ? wave / (W / 2) : seg)) {
+            P = S.P[s];
+            N = S.N[s];
+        }
+    const int n0 = ((int)blockIdx.x - S.tile0[seg]) * 32;
+    // this wave's chunks [c0, c1)
+    const int nch = G / kCh;
+    const int c0 = nch * kw / KW, c1 = nch * (kw + 1) / KW;
+
+    v16f acc;
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+    v16i cmag;
+#pragma unroll
+    for (int v = 0; v < 16; v++) cmag[v] = kMagicBits;
+
+    if (c0 < c1) {
+        Image<FMT> &I = ((Image<FMT> *)lds)[wave];
+        Chunk<FMT> ck;
+        v4f xr;
+        // Everything a chunk needs is requested a whole chunk ahead, the weights
+        // last: loads return in order, so a load issued behind the next weights and
+        // needed before them would wait for memory in every chunk.
+        v4i a[kCh];
+        float xm[4], xmn[4];  // the min terms' activation parts, two blocks (one per lane half) at a time
+        auto load = [&](int c) {
+#pragma unroll
+            for (int i = 0; i < kCh; i++) a[i] = *(const v4i *)(A.xq + ((size_t)c * kCh + i) * 1024 + lane * 16);
+            // kCh x 32 scales are contiguous, four per lane
+            xr = *(const v4f *)(A.xs + (size_t)c * kCh * 32 + 4 * lane);
+#pragma unroll
+            for (int i = 0; i < 4; i++) xmn[i] = has_min(FMT) ? A.xm[((size_t)c * kCh + 2 * i + h) * 32 + r32] : 0.0f;
+            load_chunk<FMT>(ck, P, n0, N, G, c * kCh, lane);
+        };
+        load(c0);
+        for (int c = c0; c < c1; c++) {
+            const int cnx = min(c + 1, c1 - 1);
+            bool slow = any_nonfinite(ck.sc);
+            if (dual(FMT)) slow |= any_nonfinite(ck.dh);
+            put_chunk<FMT>(ck, I, lane);
+#pragma unroll
+            for (int i = 0; i < kCh; i++) I.a[i][lane] = a[i];
+#pragma unroll
+            for (int i = 0; i < 4; i++) xm[i] = xmn[i];
+            *(v4f *)((float *)I.xs + 4 * lane) = xr;
+#pragma unroll
+            for (int k = 0; k < 4; k++) slow |= !(xr[k] < kHugeXs);
+            const bool exact = __ballot(slow) != 0;
+            load(cnx);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (!exact) {
+#pragma unroll
+                for (int b0 = 0; b0 < kCh; b0 += 4) {
+                    const v2u du = *(const v2u *)((const uint16_t *)&I.sc[0][r32] + b0);
+                    const v2u mu = *(const v2u *)((const uint16_t *)&I.sc[1][r32] + b0);
+                    v2u hu = {};
+                    if (dual(FMT)) hu = *(const v2u *)((const uint16_t *)&I.dh[dual(FMT) ? r32 : 0] + b0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int b = b0 + i;
+                        v4i q, qh;
+                        operand<FMT>(I, b, r32, h, q, qh);
+                        const float wd = FMT == SLLM_Q8_0 ? f16_lut(half_of(du, i)) : f16_exact(half_of(du, i));
+                        const float wdh = dual(FMT) ? f16_exact(half_of(hu, i)) : 0.0f;
+                        const float cd = -kMagic * wd, cdh = -kMagic * wdh;  // exact
+                        float xv[16];
+                        read_xs<FMT>(I, b, h, xv);
+                        const v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(I.a[b][lane], q, cmag, 0, 0, 0);
+                        v16i Dh = {};
+                        if (dual(FMT)) Dh = __builtin_amdgcn_mfma_i32_32x32x32_i8(I.a[b][lane], qh, cmag, 0, 0, 0);
+#pragma unroll
+                        for (int v = 0; v < 16; v++) {
+                            float f = __builtin_fmaf(__int_as_float(D[v]), wd, cd);
+                            if (dual(FMT)) f = f + __builtin_fmaf(__int_as_float(Dh[v]), wdh, cdh);
+                            acc[v] = __builtin_fmaf(f, xv[v], acc[v]);
+                        }
+                        if (has_min(FMT) && (i & 1)) {
+                            const float mn = h ? f16_exact(half_of(mu, i)) : f16_exact(half_of(mu, i - 1));
+                            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xm[b >> 1], mn, acc, 0, 0, 0);
+                        }
+                    }
+                }
+            } else {
+                // the reference's operation order (no contraction)
+#pragma unroll 1
+                for (int b = 0; b < kCh; b++) {
+                    v4i q, qh, hq = {};
+                    operand<FMT>(I, b, r32, h, q, qh);
+                    if (FMT == SLLM_Q5K1F) {
+                        // the two halves apart: low nibbles and high bits of the 5-bit codes
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            hq[k] = (q[k] >> 4) & 0x01010101;
+                            q[k] = q[k] & 0x0f0f0f0f;
+                        }
+                    } else if (dual(FMT)) {
+                        hq = qh;
+                    }
+                    const uint16_t db = ((const uint16_t *)&I.sc[0][r32])[b];
+                    const float wd = FMT == SLLM_Q8_0 ? f16_lut(db) : f16_exact(db);
+                    const float wm = has_min(FMT) ? f16_exact(((const uint16_t *)&I.sc[1][r32])[b]) : 0.0f;
+                    const float wdh = dual(FMT) ? f16_exact(((const uint16_t *)&I.dh[dual(FMT) ? r32 : 0])[b]) : 16.0f * wd;
+                    const v4i av = I.a[b][lane];
+                    const int *sx = A.sx + ((size_t)c * kCh + b) * 32;
+                    float xv[16];
+                    read_xs<FMT>(I, b, h, xv);
+                    const v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, q, cmag, 0, 0, 0);
+                    v16i Dh = {};
+                    if (has_hb(FMT)) Dh = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, hq, cmag, 0, 0, 0);
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const float dot = __int_as_float(D[v]) - kMagic;  // exact
+                        if (!has_min(FMT)) {
+                            // q8q8.go:193-195 + vnni_amd64.s:70-73; q4q8.go:37-43
+                            const float cmb = wd * xv[v];
+                            const float term = cmb * dot;
+                            acc[v] = acc[v] + term;
+                        } else {
+                            // q41q8_row_amd64.s:65-71; the high half of Q5K1 has min +0
+                            const float t1 = dot * wd;
+                            const float t2 = (float)sx[8 * (v >> 2) + 4 * h + (v & 3)] * wm;
+                            float tt = t1 + t2;
+                            tt = tt * xv[v];
+                            acc[v] = acc[v] + tt;
+                            if (has_hb(FMT)) {
+                                const float h1 = (__int_as_float(Dh[v]) - kMagic) * wdh;
+                                const float hh = h1 * xv[v];
+                                acc[v] = acc[v] + hh;
+                            }
+                        }
+                    }
+                }
+            }
+            // the image is read before the next chunk is written into it
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+
+    // the waves' sums meet in LDS: [wave][16][64], added in wave order
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 16; v++) lds[(wave * 16 + v) * 64 + lane] = acc[v];
+    __syncthreads();
+    constexpr int E = 16 * 64;  // elements of the tile
+    float *dst = S.dst[0];
+#pragma unroll
+    for (int s = 1; s < kMaxSegs; s++)
+        if (s == seg) dst = S.dst[s];
+    const int Ns = pair ? S.N[0] : N;
+#pragma unroll
+    for (int i = 0; i < E / (64 * W); i++) {
+        const int e = threadIdx.x + 64 * W * i;
+        const int l = e & 63, v = e >> 6;
+        const int m = 8 * (v >> 2) + 4 * (l >> 5) + (v & 3), col = n0 + (l & 31);
+        float s = lds[e];
+        for (int w = 1; w < KW; w++) s = s + lds[w * E + e];
+        if (m >= M || col >= Ns) continue;
+        const size_t o = (size_t)m * Ns + col;
+        if (pair) {
+            float u = lds[KW * E + e];
+            for (int w = 1; w < KW; w++) u = u + lds[(KW + w) * E + e];
+            dst[o] = swiglu(s, u);
+            if (S.dst[1]) S.dst[1][o] = s;
+            if (S.dst[2]) S.dst[2][o] = u;
+        } else {
+            dst[o] = S.mode == kAdd ? dst[o] + s : s;
+        }
+    }
+}
+
+template <int FMT, int W>
+sllm_status launch_w(const SegG &S, const SAct &A, int M, int G, hipStream_t s) {
+    constexpr size_t img = W * sizeof(Image<FMT>), red = (size_t)W * 1024 * sizeof(float);
+    static_assert((img > red ? img : red) <= 160 * 1024, "LDS");
+    hipLaunchKernelGGL((sgemm_kernel<FMT, W>), dim3(S.tile0[S.n]), dim3(64 * W), img > red ? img : red, s, S, A, M, G);
+    SLLM_HIP(hipGetLastError());
+    return SLLM_OK;
+}
+
+// Eight waves per tile, one tile per CU; with more tiles than CUs four, two
+// tiles per CU (14336x4096 at M = 30: eight waves run in two rounds, 21.4 against
+// 19.6 us).
+template <int FMT>
+sllm_status launch_f(const SegG &S, const SAct &A, int M, int G, hipStream_t s) {
+    return S.tile0[S.n] > 256 ? launch_w<FMT, 4>(S, A, M, G, s) : launch_w<FMT, 8>(S, A, M, G, s);
+}
+
+}  // namespace
+
+// Up to 32 rows and 8192 columns, for launches of 2048 output rows or more and,
+// with up to 2048 columns, of any. Measured (us, with the quantize pass; this /
+// the tiled GEMM, M = 16 and 32): Q4_1 14336x4096 20.6 / 27.6 and 20.9 / 28.6, Q8_0
+// 4096x4096 13.6 / 16.0 and 13.7 / 18.4, Q5K1 4096x4096 14.8 / 14.6 and 14.8 /
+// 16.3, Q4_0 8192x2048 10.4 / 12.7 and 10.5 / 13.6, Q8_0 1536x768 8.2 / 11.4 and
+// 8.6 / 11.8; but Q5K1 1024x4096 14.6 / 11.5 (few tiles: a wave's two chunks of K
+// in turn), Q8_0 4096x14336 37.2 / 26.2 (seven), and with two row tiles (33 to 64
+// rows) Q4_1 14336x4096 39.4 / 28.8.
+bool sgemm_supported(int fmt, int G, int M, int64_t rows) {
+    return !act_f32(fmt) && G % kCh == 0 && M <= 32 && G <= 256 && (rows >= 2048 || G <= 64);
+}
+
+size_t sgemm_act_bytes(int G) { return (sact_bytes(G) + 255) & ~(size_t)255; }
+
+sllm_status launch_sact(const float *x, const float *norm_w, float eps, int M, int G, void *act, hipStream_t s) {
+    hipLaunchKernelGGL(sact_kernel, dim3(32), dim3(256), 0, s, x, norm_w, eps, M, G, carve_sact(act, G));
+    SLLM_HIP(hipGetLastError());
+    return SLLM_OK;
+}
+
+sllm_status launch_sgemm(int fmt, const Planes *P, float *const *dst, const int *N, int nseg, int mode, int G, int M,
+                         const void *act, hipStream_t s) {
+    SegG S{};
+    S.mode = mode;
+    const bool pair = mode == kPair;
+    S.n = pair ? 1 : nseg;
+    S.tile0[0] = 0;
+    for (int i = 0; i < nseg; i++) {
+        S.P[i] = P[i];
+        S.N[i] = N[i];
+    }
+    for (int i = 0; i < (pair ? 3 : nseg); i++) S.dst[i] = dst[i];
+    for (int i = 0; i < S.n; i++) S.tile0[i + 1] = S.tile0[i] + (N[i] + 31) / 32;
+    const SAct A = carve_sact((void *)act, G);
+    switch (fmt) {
+    case SLLM_Q8_0: return launch_f<SLLM_Q8_0>(S, A, M, G, s);
+    case SLLM_Q4_0: return launch_f<SLLM_Q4_0>(S, A, M, G, s);
+    case SLLM_Q4_1: return launch_f<SLLM_Q4_1>(S, A, M, G, s);
+    case SLLM_Q5K1: return launch_f<SLLM_Q5K1>(S, A, M, G, s);
+    case SLLM_Q5K1F: return launch_f<SLLM_Q5K1F>(S, A, M, G, s);
+    }
+    return set_error(SLLM_ERR_QTYPE, "short-prompt gemm: format has no int8 MFMA path");
+}
+
+}  // namespace sllm

@@ -1,0 +1,122 @@
+"""GPU tests of the short-prompt GEMM (int8 formats, up to 32 activation rows):
+edges of its 32 x 32 tiles, of the K split over a workgroup's waves
+(fewer, as many and more chunks than waves), shared-input launches, the residual
+add, the SwiGLU epilogue and the fused norm. Bound: 1e-5 of sum |terms|, as for
+the tiled GEMM (its rounding is the same, its order another)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import sllm_qmm as sq
+
+from _helpers import REL_TOL, make_raw, make_x, term_abs_sum
+
+pytestmark = pytest.mark.gpu
+QTYPES = ["q8", "q4", "q4_1", "q5k1"]
+
+
+@pytest.fixture(autouse=True)
+def _params():
+    sq.set_param("gemm_min_rows", 1)
+    yield
+    sq.set_param("gemm_min_rows", 0)
+
+
+def weight(qtype, N, K, seed):
+    raw = make_raw(qtype, N, K, seed=seed)
+    return raw, sq.DeviceWeight.from_quant(sq.QuantWeight(qtype, raw, K // 32, N, K))
+
+
+def run(w, x):
+    M, K = x.shape
+    xd = torch.from_numpy(x).cuda()
+    y = torch.full((M, w.rows), float("nan"), device="cuda")
+    sq.matmul_dev(w, xd.data_ptr(), M, K, y.data_ptr())
+    torch.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("qtype", QTYPES)
+@pytest.mark.parametrize("N,K,M", [(1, 256, 1), (31, 256, 7), (33, 512, 32), (2100, 2304, 31), (2048, 8192, 5),
+                                   (257, 2048, 16), (8230, 256, 3), (96, 1792, 2)])
+def test_against_the_oracle(qtype, N, K, M):
+    raw, w = weight(qtype, N, K, N + M)
+    x = make_x(M, K, seed=K + M)
+    err = np.abs(run(w, x).astype(np.float64) - oracle.matmul(qtype, raw, N, x))
+    assert np.all(err <= REL_TOL * term_abs_sum(qtype, raw, N, x) + 1e-30)
+
+
+def test_q5k_weights_in_one_and_two_mfmas():
+    from sllm_qmm import synth
+    N, K, M = 70, 1024, 30
+    raw = synth.q5k_blocks(3, N, K)
+    w = sq.load_weight_f32_direct(synth.GGML_Q5_K, raw, N, K)
+    assert w.q5k1_one_mfma
+    qt, ref = oracle.load_weight(synth.GGML_Q5_K, raw, N, K)
+    x = make_x(M, K, seed=4)
+    err = np.abs(run(w, x).astype(np.float64) - oracle.matmul(qt, ref, N, x))
+    assert np.all(err <= REL_TOL * term_abs_sum(qt, ref, N, x) + 1e-30)
+
+
+@pytest.mark.parametrize("M", [3, 32])
+def test_shared_input_add_swiglu_and_norm_equal_the_single_calls(M):
+    # bit for bit: the same kernel on the same codes in the same order
+    K = 1024
+    _, a = weight("q4_1", 300, K, 1)
+    _, b = weight("q8", 65, K, 2)
+    _, c = weight("q4_1", 300, K, 3)
+    ws = [a, b, c]
+    x = make_x(M, K, seed=5)
+    single = [run(w, x) for w in ws]
+    xd = torch.from_numpy(x).cuda()
+    outs = [torch.full((M, w.rows), float("nan"), device="cuda") for w in ws]
+    sq.matmul_multi_dev(ws, xd.data_ptr(), M, K, [o.data_ptr() for o in outs])
+    h, g, u = (torch.full((M, 300), float("nan"), device="cuda") for _ in range(3))
+    sq.matmul_swiglu_dev(a, c, xd.data_ptr(), M, K, h.data_ptr(), g.data_ptr(), u.data_ptr())
+    base = np.random.default_rng(6).normal(size=(M, 300)).astype(np.float32)
+    dst = torch.from_numpy(base).cuda()
+    sq.matmul_add_dev(a, xd.data_ptr(), M, K, dst.data_ptr())
+    nw = np.random.default_rng(7).normal(1, 0.2, K).astype(np.float32)
+    nwd = torch.from_numpy(nw).cuda()
+    nouts = [torch.full((M, w.rows), float("nan"), device="cuda") for w in ws]
+    sq.rmsnorm_matmul_multi_dev(ws, xd.data_ptr(), nwd.data_ptr(), 1e-5, M, K, [o.data_ptr() for o in nouts])
+    torch.cuda.synchronize()
+    bits = lambda t: (t.cpu().numpy() if isinstance(t, torch.Tensor) else t).view(np.uint32)
+    for o, s in zip(outs, single):
+        assert np.array_equal(bits(o), bits(s))
+    assert np.array_equal(bits(dst), bits(base + single[0]))
+    # the paired launch splits K over half as many waves: another order
+    for o, s in ((g, single[0]), (u, single[2])):
+        assert np.abs(o.cpu().numpy() - s).max() <= 1e-5 * np.abs(s).max()
+    want = oracle.swiglu(g.cpu().numpy(), u.cpu().numpy())
+    assert np.all(np.abs(h.cpu().numpy() - want) <= 2.0 ** -21 * np.abs(want) + 1e-30)
+    normed = np.stack([oracle.rmsnorm(x[i:i + 1], nw, 1e-5, lib_order=True)[0] for i in range(M)])
+    for o, w in zip(nouts, ws):
+        assert np.array_equal(bits(o), bits(run(w, normed)))
+
+
+@pytest.mark.parametrize("qtype", QTYPES)
+def test_nonfinite_scales_and_huge_activations_follow_the_reference(qtype):
+    # chunks with such a scale are computed in the reference's operation order
+    N, K, M = 40, 2048, 9
+    raw, _ = weight(qtype, N, K, 8)
+    raw = raw.copy()
+    per = {"q8": 34, "q4": 18, "q4_1": 20, "q5k1": 20}[qtype]
+    blocks = raw.reshape(-1, per)
+    for i, bits in ((5, 0x7C00), (70, 0xFC00), (400, 0x7E00)):
+        blocks[i, 0:2] = [bits & 0xFF, bits >> 8]
+    w = sq.DeviceWeight.from_quant(sq.QuantWeight(qtype, raw, K // 32, N, K))
+    x = make_x(M, K, seed=9)
+    x[2, 300:400] *= np.float32(2.0 ** 98)
+    got = run(w, x)
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref = oracle.matmul(qtype, raw, N, x)
+        bound = REL_TOL * term_abs_sum(qtype, raw, N, x)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert inf.any() and np.array_equal(got[inf], ref[inf])
+    fin = np.isfinite(ref) & np.isfinite(bound)
+    assert np.all(np.abs(got[fin].astype(np.float64) - ref[fin]) <= bound[fin])
