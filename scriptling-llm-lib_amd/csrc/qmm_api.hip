@@ -538,9 +538,10 @@ int64_t total_rows(const sllm_weight *const *ws, int count) {
     for (int i = 0; i < count; i++) n += ws[i]->rows;
     return n;
 }
-bool all_sgemm(const sllm_weight *const *ws, int count, int x_rows, const Route &r) {
+// Every weight takes an int8 GEMM: the rows can be normed as they are quantized.
+bool all_int8_gemm(const sllm_weight *const *ws, int count, int x_rows, const Route &r) {
     for (int i = 0; i < count; i++)
-        if (!uses_sgemm(ws[i], x_rows, r)) return false;
+        if (act_f32(ws[i]->fmt) || !uses_gemm(ws[i], x_rows, r)) return false;
     return true;
 }
 
@@ -555,7 +556,7 @@ sllm_status run_matmul(const sllm_weight *w, const float *x, int x_rows, float *
         if (st != SLLM_OK) return st;
         return launch_sgemm(gemm_fmt(w), &P, &dst, &w->rows, 1, 0, w->groups, x_rows, ws, s);
     }
-    return launch_gemm(gemm_fmt(w), P, x, dst, w->rows, w->groups, x_rows, ws, cap, s);
+    return launch_gemm(gemm_fmt(w), P, x, dst, w->rows, w->groups, x_rows, ws, cap, false, false, s);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -584,9 +585,9 @@ size_t multi_gemm_ws(const sllm_weight *const *ws, int count, int x_rows, const 
 
 // Weights sharing the activation rows x. GEMV weights are grouped by format,
 // up to kMaxSegs per launch (with the RMSNorm prologue when nw is given), and so
-// are the short-prompt GEMM's, whose activations are quantized once (nw is only
-// given when every weight is one of these two); other GEMM-bound weights run one
-// by one with the workspace [gws, gws + gcap).
+// are the short-prompt GEMM's; other GEMM-bound weights run one by one with the
+// workspace [gws, gws + gcap). Either GEMM's activations are quantized once (nw is
+// only given when every weight is a GEMV or an int8 GEMM).
 sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, int x_rows, float *const *dst,
                        hipStream_t s, void *gws, size_t gcap, const float *nw, float eps, const Route &r) {
     sllm_status st = SLLM_OK;
@@ -611,12 +612,19 @@ sllm_status multi_impl(const sllm_weight *const *ws, int count, const float *x, 
         }
         if ((st = launch_sgemm(gemm_fmt(w), P, D, N, n, 0, w->groups, x_rows, gws, s)) != SLLM_OK) return st;
     }
+    quantized = false;  // the tiled GEMM's codes, in a layout of their own
     for (int i = 0; i < count; i++) {
         if (done[(size_t)i]) continue;
         const sllm_weight *w = ws[i];
         if (uses_gemm(w, x_rows, r)) {
             done[(size_t)i] = 1;
-            if ((st = run_matmul(w, x, x_rows, dst[i], s, gws, gcap, r)) != SLLM_OK) return st;
+            const bool int8 = !act_f32(w->fmt);
+            if (int8 && !quantized && (st = launch_gemm_act(x, nw, eps, x_rows, w->groups, gws, s)) != SLLM_OK)
+                return st;
+            if ((st = launch_gemm(gemm_fmt(w), as_const(w->planes), x, dst[i], w->rows, w->groups, x_rows, gws, gcap,
+                                  int8, false, s)) != SLLM_OK)
+                return st;
+            quantized = int8;  // the bf16 GEMM's fragments lie over the codes
             continue;
         }
         Planes P[kMaxSegs];
@@ -669,8 +677,8 @@ sllm_status swiglu_impl(const sllm_weight *wg, const sllm_weight *wu, const floa
         const int Ns[2] = {N, N};
         return launch_sgemm(gemm_fmt(wg), P, D, Ns, 2, 2, wg->groups, x_rows, ws, s);
     }
-    // Prefill or mixed formats: the two matmuls, then the elementwise SwiGLU;
-    // x is already normed here (nw is only passed for the one-launch forms).
+    // Prefill or mixed formats: the two matmuls, then the elementwise SwiGLU (nw is
+    // only given when both are int8 GEMMs).
     const sllm_weight *pair[2] = {wg, wu};
     const size_t gw = multi_gemm_ws(pair, 2, x_rows, r);
     const size_t mm = align256((size_t)x_rows * N * sizeof(float));
@@ -678,8 +686,8 @@ sllm_status swiglu_impl(const sllm_weight *wg, const sllm_weight *wu, const floa
     float *g = gate ? gate : (float *)tail;
     float *u = up ? up : (float *)(tail + (gate ? 0 : mm));
     sllm_status st;
-    if ((st = run_matmul(wg, x, x_rows, g, s, ws, gw, r)) != SLLM_OK) return st;
-    if ((st = run_matmul(wu, x, x_rows, u, s, ws, gw, r)) != SLLM_OK) return st;
+    float *const D[2] = {g, u};
+    if ((st = multi_impl(pair, 2, x, x_rows, D, s, ws, gw, nw, eps, r)) != SLLM_OK) return st;
     return launch_swiglu(g, u, h, (size_t)x_rows * N, s);
 }
 
@@ -1163,12 +1171,13 @@ sllm_status sllm_rmsnorm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_wei
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
     void *ws = nullptr;
     size_t cap = 0;
+    const sllm_weight *const both[2] = {wg, wu};
     Route r{true, 2 * (int64_t)wg->rows};
     const size_t need = fit_workspace(s, r, [&] {
-        return (swiglu_sgemm(wg, wu, x_rows, r) ? 0 : nb) + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, r);
+        return (all_int8_gemm(both, 2, x_rows, r) ? 0 : nb) + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, r);
     });
     if ((st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
-    if (swiglu_sgemm(wg, wu, x_rows, r))  // normed as they are quantized
+    if (all_int8_gemm(both, 2, x_rows, r))  // normed as they are quantized
         return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, ws, norm_w, eps, r);
     float *normed = (float *)ws;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
@@ -1253,14 +1262,14 @@ sllm_status sllm_rmsnorm_matmul_multi_dev(const sllm_weight *const *ws, int coun
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
     Route r{true, total_rows(ws, count)};
     const size_t need = fit_workspace(s, r, [&] {
-        return (all_sgemm(ws, count, x_rows, r) ? 0 : nb) + multi_gemm_ws(ws, count, x_rows, r);
+        return (all_int8_gemm(ws, count, x_rows, r) ? 0 : nb) + multi_gemm_ws(ws, count, x_rows, r);
     });
     // several rows: normed rows into the workspace first, then every weight
     // reads them (GEMV and GEMM alike)
     void *ws_ = nullptr;
     size_t cap = 0;
     if ((st = workspace(s, need, &ws_, &cap)) != SLLM_OK) return st;
-    if (all_sgemm(ws, count, x_rows, r))  // normed as they are quantized
+    if (all_int8_gemm(ws, count, x_rows, r))  // normed as they are quantized
         return multi_impl(ws, count, x, x_rows, dst, s, ws_, need, norm_w, eps, r);
     float *normed = (float *)ws_;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
@@ -1445,15 +1454,8 @@ sllm_status sllm_matmul_add_dev(const sllm_weight *w, const float *x, int x_rows
     if (st != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     const Planes P = as_const(w->planes);
-    // GEMM: the product into the workspace behind the GEMM's own, then dst += it
-    const size_t n = (size_t)x_rows * w->rows;
-    // (its epilogue saves the tiled GEMM's add pass: worth it for few rows too)
-    Route r{true, w->rows > 2048 ? w->rows : 2048};
-    const size_t need = fit_workspace(s, r, [&] {
-        return uses_gemm(w, x_rows, r)
-                   ? multi_gemm_ws(&w, 1, x_rows, r) + (uses_sgemm(w, x_rows, r) ? 0 : n * sizeof(float))
-                   : (size_t)0;
-    });
+    Route r{true, w->rows};
+    const size_t need = fit_workspace(s, r, [&] { return multi_gemm_ws(&w, 1, x_rows, r); });
     if (!need) return launch_gemv_add(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
     void *ws = nullptr;
     size_t cap = 0;
@@ -1462,10 +1464,7 @@ sllm_status sllm_matmul_add_dev(const sllm_weight *w, const float *x, int x_rows
         if ((st = launch_sact(x, nullptr, 0.0f, x_rows, w->groups, ws, s)) != SLLM_OK) return st;
         return launch_sgemm(gemm_fmt(w), &P, &dst, &w->rows, 1, 1, w->groups, x_rows, ws, s);
     }
-    const size_t gb = need - n * sizeof(float);
-    float *tmp = (float *)((char *)ws + gb);
-    if ((st = launch_gemm(gemm_fmt(w), P, x, tmp, w->rows, w->groups, x_rows, ws, gb, s)) != SLLM_OK) return st;
-    return launch_add(dst, tmp, n, s);
+    return launch_gemm(gemm_fmt(w), P, x, dst, w->rows, w->groups, x_rows, ws, need, false, true, s);
 }
 
 sllm_status sllm_kv_cache_create(int n_layers, int n_kv_heads, int d_k, int max_seq, sllm_kv_cache **out) {

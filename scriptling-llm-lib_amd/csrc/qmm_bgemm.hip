@@ -299,7 +299,7 @@ template <int FMT, int WM, int WN, int CT, int KB, int RA, int WA>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)))
 bgemm_kernel(Planes P, const uint16_t *__restrict__ frag, const float *__restrict__ xsum,
              const uint8_t *__restrict__ flag, const float *__restrict__ x, float *__restrict__ out, int M, int N,
-             int G, int mtiles, int ntiles, int splits, int sps) {
+             int G, int mtiles, int ntiles, int splits, int sps, int add) {
     constexpr int BN = 32 * CT * WN, T = 64 * WM * WN;
     constexpr int UNITS = BN * KB, PER = UNITS / T;
     constexpr int HPB = PER * 2 / KB;  // half units decoded beside each block
@@ -480,7 +480,11 @@ bgemm_kernel(Planes P, const uint16_t *__restrict__ frag, const float *__restric
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int m = rt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (m < M && n < N) o[(size_t)m * N + n] = RUN ? tot[RUN ? j : 0][v] : acc[j][v];
+            if (m < M && n < N) {
+                float &d = o[(size_t)m * N + n];
+                const float r = RUN ? tot[RUN ? j : 0][v] : acc[j][v];
+                d = add ? d + r : r;  // add: the residual add, one float32 add
+            }
         }
     }
 }
@@ -549,20 +553,21 @@ BWs layout(int fmt, int M, int N, int G, const BPlan &p) {
 
 template <int FMT, int WM, int WN, int CT, int KB, int RA, int WA>
 sllm_status launch_shape(const Planes &P, const uint16_t *frag, const float *xsum, const uint8_t *flag,
-                         const float *x, float *out, int M, int N, int G, const BPlan &p, hipStream_t s) {
+                         const float *x, float *out, int M, int N, int G, const BPlan &p, int add, hipStream_t s) {
     const int total = p.mtiles * p.ntiles * p.splits;
     constexpr size_t lds = 2 * sizeof(BStage<FMT, KB, 32 * CT * WN>);
     static_assert(lds <= 160 * 1024, "LDS");
     static_assert(32 * CT * WN == kBn, "columns per workgroup");
     hipLaunchKernelGGL((bgemm_kernel<FMT, WM, WN, CT, KB, RA, WA>), dim3((total + 7) / 8 * 8), dim3(64 * WM * WN), lds, s, P,
-                       frag, xsum, flag, x, out, M, N, G, p.mtiles, p.ntiles, p.splits, p.sps);
+                       frag, xsum, flag, x, out, M, N, G, p.mtiles, p.ntiles, p.splits, p.sps, add);
     SLLM_HIP(hipGetLastError());
     return SLLM_OK;
 }
 
 template <int FMT>
 sllm_status launch_fmt(const Planes &P, const float *x, float *dst, int M, int N, int G, const BPlan &p, char *ws,
-                       hipStream_t s) {
+                       bool add, hipStream_t s) {
+    const int ea = add && p.splits == 1;  // the add in the kernel's epilogue, else in the reduction
     const BWs L = layout(FMT, M, N, G, p);
     uint16_t *frag = (uint16_t *)ws;
     float *xsum = (float *)(ws + L.frag);
@@ -574,9 +579,9 @@ sllm_status launch_fmt(const Planes &P, const float *x, float *dst, int M, int N
                        flag);
     SLLM_HIP(hipGetLastError());
     switch (p.shape) {
-    case kRows32: return launch_shape<FMT, 1, 4, 2, 2, 2, 2>(P, frag, xsum, flag, x, out, M, N, G, p, s);
-    case kRows64: return launch_shape<FMT, 2, 4, 2, 2, 4, 2>(P, frag, xsum, flag, x, out, M, N, G, p, s);
-    default: return launch_shape<FMT, 4, 2, 4, kKb128(FMT), 2, 2>(P, frag, xsum, flag, x, out, M, N, G, p, s);
+    case kRows32: return launch_shape<FMT, 1, 4, 2, 2, 2, 2>(P, frag, xsum, flag, x, out, M, N, G, p, ea, s);
+    case kRows64: return launch_shape<FMT, 2, 4, 2, 2, 4, 2>(P, frag, xsum, flag, x, out, M, N, G, p, ea, s);
+    default: return launch_shape<FMT, 4, 2, 4, kKb128(FMT), 2, 2>(P, frag, xsum, flag, x, out, M, N, G, p, ea, s);
     }
 }
 
@@ -587,20 +592,20 @@ size_t bgemm_workspace_bytes(int fmt, int N, int G, int M) {
     return L.frag + L.xsum + L.flag + L.part;
 }
 
-sllm_status launch_bgemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws,
+sllm_status launch_bgemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws, bool add,
                          hipStream_t s) {
     const BPlan p = plan(fmt, M, N, G);
     sllm_status st;
     switch (fmt) {
-    case SLLM_Q5_0: st = launch_fmt<SLLM_Q5_0>(P, x, dst, M, N, G, p, (char *)ws, s); break;
-    case SLLM_Q2K: st = launch_fmt<SLLM_Q2K>(P, x, dst, M, N, G, p, (char *)ws, s); break;
-    case SLLM_Q3K: st = launch_fmt<SLLM_Q3K>(P, x, dst, M, N, G, p, (char *)ws, s); break;
+    case SLLM_Q5_0: st = launch_fmt<SLLM_Q5_0>(P, x, dst, M, N, G, p, (char *)ws, add, s); break;
+    case SLLM_Q2K: st = launch_fmt<SLLM_Q2K>(P, x, dst, M, N, G, p, (char *)ws, add, s); break;
+    case SLLM_Q3K: st = launch_fmt<SLLM_Q3K>(P, x, dst, M, N, G, p, (char *)ws, add, s); break;
     default: return set_error(SLLM_ERR_QTYPE, "gemm: format has no bf16 MFMA path");
     }
     if (st != SLLM_OK || p.splits == 1) return st;
     const BWs L = layout(fmt, M, N, G, p);
     return launch_reduce_splits((const float *)((char *)ws + L.frag + L.xsum + L.flag), dst, (size_t)M * N, p.splits,
-                                s);
+                                add, s);
 }
 
 }  // namespace sllm

@@ -517,7 +517,7 @@ __device__ __forceinline__ void stage_slow(const Stage<FMT, KB, BM, BN> &S, int 
 template <int FMT, int WM, int WN, int CF, int WK, int KB, bool PIPE, int PF, bool DBG>
 __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(2))) gemm_kernel(
     Planes P, const int8_t *__restrict__ xq, const float *__restrict__ xs, const int *__restrict__ sx,
-    float *__restrict__ out, int M, int N, int G, int mtiles, int ntiles, int splits, int sps,
+    float *__restrict__ out, int M, int N, int G, int mtiles, int ntiles, int splits, int sps, int add,
     int *__restrict__ dots) {
     constexpr int BM = 32 * WM, BN = 32 * CF * WN, T = 64 * WM * WN * WK;
     static_assert(KB % WK == 0, "every wave takes the same number of blocks per stage");
@@ -671,7 +671,11 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int m = m0 + wm * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (m < M && n < N) o[(size_t)m * N + n] = acc[j][v];
+            if (m < M && n < N) {
+                // model_f32.go:472-474 / 495-497: x[i] += o[i], one float32 add
+                float &d = o[(size_t)m * N + n];
+                d = add ? d + acc[j][v] : acc[j][v];
+            }
         }
     }
 }
@@ -681,7 +685,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
 // aligned); the loads of up to eight splits are issued before their adds (a
 // load-add chain waited for every split's load in turn).
 template <int V>
-__global__ void reduce_splits_kernel(const float *__restrict__ part, float *__restrict__ dst, size_t n, int S) {
+__global__ void reduce_splits_kernel(const float *__restrict__ part, float *__restrict__ dst, size_t n, int S, int add) {
     typedef float vec __attribute__((ext_vector_type(V)));
     const size_t nv = n / V;
     const vec *pv = (const vec *)part;
@@ -696,7 +700,7 @@ __global__ void reduce_splits_kernel(const float *__restrict__ part, float *__re
             for (int k = 0; k < 8; k++)
                 if (s0 + k < S) v = v + p[k];
         }
-        ((vec *)dst)[i] = v;
+        ((vec *)dst)[i] = add ? ((const vec *)dst)[i] + v : v;
     }
 }
 
@@ -761,7 +765,7 @@ GemmPlan plan_gemm(int fmt, int M, int N, int G) {
 
 template <int FMT, int WM, int WN, int CF, int WK, int KB, bool PIPE, int PF, bool DBG>
 sllm_status launch_shape(const Planes &P, const int8_t *xq, const float *xsp, const int *sxp, float *out, int M,
-                         int N, int G, const GemmPlan &p, int *dots, hipStream_t s) {
+                         int N, int G, const GemmPlan &p, int add, int *dots, hipStream_t s) {
     const int total = p.mtiles * p.ntiles * p.splits;
     const int grid = ((total + 7) / 8) * 8;
     constexpr size_t stages = 2 * sizeof(Stage<FMT, KB, 32 * WM, 32 * CF * WN>);
@@ -769,60 +773,69 @@ sllm_status launch_shape(const Planes &P, const int8_t *xq, const float *xsp, co
     constexpr size_t lds = stages > red ? stages : red;
     static_assert(lds <= 160 * 1024, "LDS");
     hipLaunchKernelGGL((gemm_kernel<FMT, WM, WN, CF, WK, KB, PIPE, PF, DBG>), dim3(grid), dim3(64 * WM * WN * WK), lds, s, P, xq,
-                       xsp, sxp, out, M, N, G, p.mtiles, p.ntiles, p.splits, p.sps, dots);
+                       xsp, sxp, out, M, N, G, p.mtiles, p.ntiles, p.splits, p.sps, add, dots);
     SLLM_HIP(hipGetLastError());
     return SLLM_OK;
 }
 
 template <int FMT, bool DBG>
 sllm_status launch_fmt(const Planes &P, const int8_t *xq, const float *xsp, const int *sxp, float *out, int M,
-                       int N, int G, const GemmPlan &p, int *dots, hipStream_t s) {
+                       int N, int G, const GemmPlan &p, int add, int *dots, hipStream_t s) {
     switch (p.shape) {
-    case kDeep: return launch_shape<FMT, 2, 1, 2, 2, 4, true, 1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    case kDeepS: return launch_shape<FMT, 2, 1, 2, 2, 4, false, 2, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    case kDeepS32: return launch_shape<FMT, 1, 1, 2, 4, 4, false, 2, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    case kWide2: return launch_shape<FMT, 2, 2, 2, 1, 4, true, 2, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    default: return launch_shape<FMT, 2, 2, 2, 1, 4, true, 1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
+    case kDeep: return launch_shape<FMT, 2, 1, 2, 2, 4, true, 1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    case kDeepS: return launch_shape<FMT, 2, 1, 2, 2, 4, false, 2, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    case kDeepS32: return launch_shape<FMT, 1, 1, 2, 4, 4, false, 2, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    case kWide2: return launch_shape<FMT, 2, 2, 2, 1, 4, true, 2, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    default: return launch_shape<FMT, 2, 2, 2, 1, 4, true, 1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
     }
 }
 
 template <bool DBG>
 sllm_status launch_int8(int fmt, const Planes &P, const int8_t *xq, const float *xsp, const int *sxp, float *out,
-                        int M, int N, int G, const GemmPlan &p, int *dots, hipStream_t s) {
+                        int M, int N, int G, const GemmPlan &p, int add, int *dots, hipStream_t s) {
     switch (fmt) {
-    case SLLM_Q8_0: return launch_fmt<SLLM_Q8_0, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    case SLLM_Q4_0: return launch_fmt<SLLM_Q4_0, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    case SLLM_Q4_1: return launch_fmt<SLLM_Q4_1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    case SLLM_Q5K1: return launch_fmt<SLLM_Q5K1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
-    case SLLM_Q5K1F: return launch_fmt<SLLM_Q5K1F, DBG>(P, xq, xsp, sxp, out, M, N, G, p, dots, s);
+    case SLLM_Q8_0: return launch_fmt<SLLM_Q8_0, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    case SLLM_Q4_0: return launch_fmt<SLLM_Q4_0, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    case SLLM_Q4_1: return launch_fmt<SLLM_Q4_1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    case SLLM_Q5K1: return launch_fmt<SLLM_Q5K1, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
+    case SLLM_Q5K1F: return launch_fmt<SLLM_Q5K1F, DBG>(P, xq, xsp, sxp, out, M, N, G, p, add, dots, s);
     }
     return set_error(SLLM_ERR_QTYPE, "gemm: format has no int8 MFMA path");
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// The activation codes at the start of the workspace: xq, xs, Σxq.
+struct ActWs {
+    int8_t *xq;
+    float *xs;
+    int *sx;
+    void *rest;
+};
+ActWs carve_act_ws(void *ws, int M, int G) {
+    const size_t q = align256((size_t)M * G * 32), sb = align256((size_t)M * G * 4);
+    char *b = (char *)ws;
+    return {(int8_t *)b, (float *)(b + q), (int *)(b + q + sb), b + q + 2 * sb};
+}
+
 sllm_status gemm_impl(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws,
-                      size_t ws_bytes, int *dots, hipStream_t s) {
+                      size_t ws_bytes, bool quantized, bool add, int *dots, hipStream_t s) {
     if (ws_bytes < gemm_workspace_bytes(fmt, N, G, M)) return set_error(SLLM_ERR_ARG, "gemm: workspace too small");
     if (!gemm_supported(fmt, G)) return set_error(SLLM_ERR_SHAPE, "gemm: format or cols not supported");
     if (act_f32(fmt)) {
         if (dots) return set_error(SLLM_ERR_QTYPE, "gemm block dots: fp32 activations have no int8 GEMM");
-        return launch_bgemm(fmt, P, x, dst, N, G, M, ws, s);
+        return launch_bgemm(fmt, P, x, dst, N, G, M, ws, add, s);
     }
     const GemmPlan p = plan_gemm(fmt, M, N, G);
     sllm_status st = SLLM_OK;
-    int8_t *xq = (int8_t *)ws;
-    const size_t q = align256((size_t)M * G * 32), sb = align256((size_t)M * G * 4);
-    float *xsp = (float *)((char *)ws + q);
-    int *sxp = (int *)((char *)ws + q + sb);
-    float *part = (float *)((char *)ws + q + 2 * sb);
-    st = launch_quantize_act(x, M, G, xq, xsp, sxp, s);
-    if (st != SLLM_OK) return st;
-    float *out = p.splits > 1 ? part : dst;
-    st = dots ? launch_int8<true>(fmt, P, xq, xsp, sxp, out, M, N, G, p, dots, s)
-              : launch_int8<false>(fmt, P, xq, xsp, sxp, out, M, N, G, p, nullptr, s);
+    if (!quantized && (st = launch_gemm_act(x, nullptr, 0.0f, M, G, ws, s)) != SLLM_OK) return st;
+    const ActWs A = carve_act_ws(ws, M, G);
+    float *out = p.splits > 1 ? (float *)A.rest : dst;
+    const int ea = add && p.splits == 1;  // the add in the kernel's epilogue, else in the reduction
+    st = dots ? launch_int8<true>(fmt, P, A.xq, A.xs, A.sx, out, M, N, G, p, ea, dots, s)
+              : launch_int8<false>(fmt, P, A.xq, A.xs, A.sx, out, M, N, G, p, ea, nullptr, s);
     if (st != SLLM_OK || p.splits == 1) return st;
-    return launch_reduce_splits(part, dst, (size_t)M * N, p.splits, s);
+    return launch_reduce_splits(out, dst, (size_t)M * N, p.splits, add, s);
 }
 
 }  // namespace
@@ -838,27 +851,33 @@ size_t gemm_workspace_bytes(int fmt, int N, int G, int M) {
     return align256((size_t)M * G * 32) + 2 * align256((size_t)M * G * 4) + align256(parts);
 }
 
-sllm_status launch_reduce_splits(const float *part, float *dst, size_t n, int S, hipStream_t s) {
+sllm_status launch_reduce_splits(const float *part, float *dst, size_t n, int S, bool add, hipStream_t s) {
     const bool v4 = n % 4 == 0 && ((uintptr_t)dst & 15) == 0;
     int grid = (int)((n / (v4 ? 4 : 1) + 255) / 256);
     if (grid > 4096) grid = 4096;
     if (v4)
-        hipLaunchKernelGGL(reduce_splits_kernel<4>, dim3(grid), dim3(256), 0, s, part, dst, n, S);
+        hipLaunchKernelGGL(reduce_splits_kernel<4>, dim3(grid), dim3(256), 0, s, part, dst, n, S, add ? 1 : 0);
     else
-        hipLaunchKernelGGL(reduce_splits_kernel<1>, dim3(grid), dim3(256), 0, s, part, dst, n, S);
+        hipLaunchKernelGGL(reduce_splits_kernel<1>, dim3(grid), dim3(256), 0, s, part, dst, n, S, add ? 1 : 0);
     SLLM_HIP(hipGetLastError());
     return SLLM_OK;
 }
 
+sllm_status launch_gemm_act(const float *x, const float *norm_w, float eps, int M, int G, void *ws, hipStream_t s) {
+    const ActWs A = carve_act_ws(ws, M, G);
+    return norm_w ? launch_norm_quant(x, norm_w, eps, M, G, A.xq, A.xs, A.sx, s)
+                  : launch_quantize_act(x, M, G, A.xq, A.xs, A.sx, s);
+}
+
 sllm_status launch_gemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws,
-                        size_t ws_bytes, hipStream_t s) {
-    return gemm_impl(fmt, P, x, dst, N, G, M, ws, ws_bytes, nullptr, s);
+                        size_t ws_bytes, bool quantized, bool add, hipStream_t s) {
+    return gemm_impl(fmt, P, x, dst, N, G, M, ws, ws_bytes, quantized, add, nullptr, s);
 }
 
 sllm_status launch_gemm_dots(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws,
                              size_t ws_bytes, int32_t *dots, hipStream_t s) {
     if (!dots) return set_error(SLLM_ERR_ARG, "gemm block dots: null output");
-    return gemm_impl(fmt, P, x, dst, N, G, M, ws, ws_bytes, dots, s);
+    return gemm_impl(fmt, P, x, dst, N, G, M, ws, ws_bytes, false, false, dots, s);
 }
 
 }  // namespace sllm

@@ -198,16 +198,22 @@ sllm_status launch_gemv_argmax(int fmt, const Planes &P, const float *x, float *
 // down matmuls (model_f32.go:472-474, 495-497), in the GEMV epilogue.
 sllm_status launch_gemv_add(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M,
                             hipStream_t s);
-// dst[i] += src[i] for n elements (the GEMM path of the residual add).
-sllm_status launch_add(float *dst, const float *src, size_t n, hipStream_t s);
 // rmsNormFlatF32 of rows x K into out (the prefill path of the fused-norm
 // entry points; same statistics as the GEMV prologue).
 sllm_status launch_rmsnorm(const float *x, const float *norm_w, float eps, int rows, int K, float *out,
                            hipStream_t s);
 // h[i] = SwiGLU(gate[i], up[i]) for n elements (the prefill path and mixed formats).
 sllm_status launch_swiglu(const float *gate, const float *up, float *h, size_t n, hipStream_t s);
-sllm_status launch_gemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M,
-                        void *ws, size_t ws_bytes, hipStream_t s);
+// The GEMM of one weight. int8 formats: the activation codes are in ws already where
+// quantized is set (launch_gemm_act, or an earlier weight's GEMM on the same rows).
+// add: dst += product.
+sllm_status launch_gemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws,
+                        size_t ws_bytes, bool quantized, bool add, hipStream_t s);
+// The tiled int8 GEMM's activation codes (at the start of its workspace) of the rows
+// x, RMSNormed first where norm_w is given.
+sllm_status launch_gemm_act(const float *x, const float *norm_w, float eps, int M, int G, void *ws, hipStream_t s);
+sllm_status launch_norm_quant(const float *x, const float *norm_w, float eps, int rows, int G, int8_t *xq, float *xs,
+                              int32_t *sx, hipStream_t s);
 // The same GEMM that also writes every int32 block dot its matrix cores
 // produce to dots [M][N][G] (x2 for Q5K1: low, high); int8 formats only.
 sllm_status launch_gemm_dots(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M,
@@ -227,11 +233,12 @@ sllm_status launch_sgemm(int fmt, const Planes *P, float *const *dst, const int 
                          const void *act, hipStream_t s);
 // Formats with fp32 activations (Q5_0, Q2_K, Q3_K): the same products on the bf16
 // matrix cores; ws holds at least bgemm_workspace_bytes.
-sllm_status launch_bgemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws,
+sllm_status launch_bgemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws, bool add,
                          hipStream_t s);
 size_t bgemm_workspace_bytes(int fmt, int N, int G, int M);
-// dst = part[0] + part[1] + ... + part[S - 1] (n floats each), in split order.
-sllm_status launch_reduce_splits(const float *part, float *dst, size_t n, int S, hipStream_t s);
+// dst = part[0] + part[1] + ... + part[S - 1] (n floats each), in split order; add:
+// dst += that sum.
+sllm_status launch_reduce_splits(const float *part, float *dst, size_t n, int S, bool add, hipStream_t s);
 sllm_status launch_quantize_act(const float *x, int rows, int G, int8_t *xq, float *xs, int32_t *sx,
                                 hipStream_t s);
 sllm_status launch_block_dots(int fmt, const Planes &P, const float *x, int N, int G, int M,
