@@ -12,8 +12,10 @@
 //   state goes to the workspace. Scores are the reference's sequential
 //   float32 dots. For one query row (decode) it also does the bias / norm /
 //   RoPE / append work itself.
-// attn_prep_kernel (several rows): that work, one wave per (row, head).
-// attn_combine_kernel (more than one split): one wave per (row, head) merges
+// attn_prep_kernel (several rows): that work, a workgroup of eight waves over a
+//   row's heads.
+// attn_flash_kernel / attn_flash_combine_kernel (prompts): below.
+// attn_combine_kernel (more than one split): one workgroup per (row, head) merges
 //   the splits. Separate launches instead of a last-workgroup combine: on
 //   this multi-XCD part a device-scope fence writes back and invalidates the
 //   L2, which costs more than the launch.
@@ -478,76 +480,86 @@ __global__ void __launch_bounds__(kMaxWaves * 64) attn_split_kernel(AttnArgs a) 
     }
 }
 
-// The splits of one (row, head), one wave each: M = max of the split maxima,
-// weights w_t = float32(exp(float64(m_t - M))), L = sum of l_t * w_t (fixed
-// lane order), out[d] = (sum over t of o_t[d] * w_t) * (1 / L), written in
-// mergeHeadsDataF32's layout (float32_ops.go:262-273).
-__global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int pair = blockIdx.x * 4 + (threadIdx.x >> 6);  // qi * n_heads + h
-    if (pair >= a.seq * a.n_heads) return;                 // wave-uniform
+// The splits of one (row, head), one workgroup of a wave per eight splits (at most
+// kCombineWaves): M = max of the split maxima, weights w_t = float32(exp(float64(m_t - M))), L = sum of l_t *
+// w_t, out[d] = (sum over t of o_t[d] * w_t) * (1 / L), written in
+// mergeHeadsDataF32's layout (float32_ops.go:262-273). Every wave takes a
+// consecutive share of the splits, eight at a time with all their loads issued
+// together, and the waves' sums are added in wave order. (One wave per head left
+// 32 waves on the device for a decode step, each with up to four rounds of memory
+// in turn: 9.0 us at 63 splits. One decode step, whole call, 32/8/128: 8000 cached
+// 32.1 -> 27.1 us, 4000 16.9 -> 15.6; 8/1/256: 8000 40.7 -> 29.7; up to 16 splits
+// the same.)
+constexpr int kCombineWaves = 8;
+__global__ void __launch_bounds__(64 * kCombineWaves) attn_combine_kernel(AttnArgs a) {
+    __shared__ float Ls[kCombineWaves], Os[kCombineWaves][kMaxDk];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int pair = blockIdx.x;  // qi * n_heads + h
     const int dk = a.d_k;
     const size_t stride = (size_t)dk + 2;
     const float *pb = a.part + (size_t)pair * a.splits * stride;
-    // splits in groups of 16: lane t holds m_t and l_t of its group, every
-    // lane the values of its d for the whole group - all loaded together
-    // (a group's missing splits weigh 0 and add exact zeros). With at most 16
-    // splits the maximum comes from the same loads (one memory round);
-    // otherwise from a first pass over the maxima.
-    const bool one = a.splits <= 16;
-    float M = -INFINITY;
-    if (!one) {
-        for (int t = lane; t < a.splits; t += 64) M = fmaxf(M, pb[t * stride]);
+    const int waves = blockDim.x >> 6;
+    const int s0 = a.splits * wave / waves, s1 = a.splits * (wave + 1) / waves;
+    float ov[8][4], ml[8], ll[8];
+    auto load8 = [&](int t0) {
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-    }
-    float Lp = 0.0f;
-    float O[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int t0 = 0; t0 < a.splits; t0 += 16) {
-        const int nt = min(16, a.splits - t0);
-        const int tl = t0 + (lane & 15);
-        const bool mine = lane < 16 && tl < a.splits;
-        const float ml = mine ? pb[tl * stride] : -INFINITY;
-        const float ll = mine ? pb[tl * stride + 1] : 0.0f;
-        float ov[16][4];
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const float *ob = pb + (size_t)(t0 + u) * stride + 2;
+        for (int u = 0; u < 8; u++) {
+            const float *ob = pb + (size_t)min(t0 + u, a.splits - 1) * stride;
+            ml[u] = ob[0];
+            ll[u] = ob[1];
 #pragma unroll
             for (int jj = 0; jj < 4; jj++) {
                 const int d = lane + 64 * jj;
-                ov[u][jj] = (u < nt && d < dk) ? ob[d] : 0.0f;
+                ov[u][jj] = d < dk ? ob[2 + d] : 0.0f;
             }
         }
-        if (one) {
-            M = ml;
+    };
+    load8(s0);
+    float M = -INFINITY;
+    for (int t = lane; t < a.splits; t += 64) M = fmaxf(M, pb[t * stride]);
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-        }
-        // a split without positions (-inf) weighs 0
-        const float wl = (mine && ml != -INFINITY) ? (float)exp((double)(ml - M)) : 0.0f;
-        Lp = Lp + ll * wl;
+    for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    float L = 0.0f;
+    float O[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t0 = s0; t0 < s1; t0 += 8) {
+        if (t0 > s0) load8(t0);
+        // lane u forms the weight of split t0 + u; a split without positions (-inf)
+        // weighs 0, and so does one past the share (its values are not added)
+        float mu = ml[0];
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const float w = lane_bcast(wl, u);  // 0 past the group's end
+        for (int u = 1; u < 8; u++) mu = (lane & 7) == u ? ml[u] : mu;
+        const float wl = mu != -INFINITY ? (float)exp((double)(mu - M)) : 0.0f;
 #pragma unroll
-            for (int jj = 0; jj < 4; jj++) O[jj] = O[jj] + ov[u][jj] * w;
+        for (int u = 0; u < 8; u++) {
+            if (t0 + u < s1) {
+                const float w = lane_bcast(wl, u);
+                L = L + ll[u] * w;
+#pragma unroll
+                for (int jj = 0; jj < 4; jj++) O[jj] = O[jj] + ov[u][jj] * w;
+            }
         }
     }
-    const float L = wave_sum(Lp);
-    const float inv = 1.0f / L;
-    float *dst = a.out + (size_t)pair * dk;  // mergeHeadsDataF32 layout
+    if (lane == 0) Ls[wave] = L;
 #pragma unroll
     for (int jj = 0; jj < 4; jj++) {
         const int d = lane + 64 * jj;
-        if (d < dk) dst[d] = O[jj] * inv;
+        if (d < dk) Os[wave][d] = O[jj];
+    }
+    __syncthreads();
+    float Lt = 0.0f;
+    for (int w = 0; w < waves; w++) Lt = Lt + Ls[w];
+    const float inv = 1.0f / Lt;
+    for (int d = threadIdx.x; d < dk; d += blockDim.x) {
+        float o = 0.0f;
+        for (int w = 0; w < waves; w++) o = o + Os[w][d];
+        a.out[(size_t)pair * dk + d] = o * inv;  // mergeHeadsDataF32 layout
     }
 }
 
 // ---------------------------------------------------------- prompts ----
 //
-// attn_flash_kernel: several query rows (from kFlashRows on, d_k up to 128) on
-// the fp32 matrix cores. A wave owns 32 query rows of one q head; the four
+// attn_flash_kernel: several query rows (more than kFlashPairs pairs of row and kv
+// head, d_k up to 128) on the fp32 matrix cores. A wave owns 32 query rows of one q head; the four
 // waves of a workgroup share one kv head's K and V tiles of 32 positions in LDS
 // (GQA: the q heads of the group; otherwise further row blocks). Both products
 // are taken transposed, so that a lane is a query row throughout:
@@ -560,12 +572,13 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a) {
 //     B operand of a two-deep MFMA it pairs positions p and p + 4: P goes from
 //     accumulator to operand without leaving its registers, V is read to match.
 // Scores are fp32 dots of the same products as the reference's (in two halves,
-// added by the MFMA), the exponentials float32(exp(float64(score - running
-// max))), the sums fp32: as the split kernel, in another association.
+// added by the MFMA), the exponentials exp_neg's (fp32, the argument's
+// reduction compensated: rms error 0.290 ulp where float32(exp(float64(x))) has
+// 0.289), the sums fp32, in another association than the split kernel's.
 //
 // What bounds it: the fp32 matrix cores (64 cycles per 32 x 32 x 2; 2 DK of
 // them per tile); the split kernel spent 64-lane VALU dots and one pass over K
-// and V per query row (1024 rows of 32 / 8 heads, d_k 128: 896 us).
+// and V per query row (1024 rows of 32 / 8 heads, d_k 128: 882 us, now 139).
 // Causal rows differ in length: a row block's tiles are cut into chunks of C
 // tiles (workgroups of their own; heaviest first) whose states
 // attn_flash_combine_kernel merges; C is about the tiles one workgroup slot gets
@@ -1110,7 +1123,8 @@ sllm_status launch_attention(const AttnArgs &a, hipStream_t s) {
         }
     }
     if (a.splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3((a.seq * a.n_heads + 3) / 4), dim3(256), 0, s, a);
+        const int waves = (a.splits + 7) / 8 < kCombineWaves ? (a.splits + 7) / 8 : kCombineWaves;
+        hipLaunchKernelGGL(attn_combine_kernel, dim3(a.seq * a.n_heads), dim3(64 * waves), 0, s, a);
         SLLM_HIP(hipGetLastError());
     }
     return SLLM_OK;

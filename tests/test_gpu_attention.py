@@ -171,6 +171,15 @@ def test_tile_groups_and_splits(groups, target, cache_len):
         sq.set_param("attn_target_blocks", 512)
 
 
+@pytest.mark.parametrize("splits,last", [(2, 1), (8, 128), (9, 1), (16, 64), (17, 65), (63, 128), (65, 1), (131, 7)])
+@pytest.mark.parametrize("dk", [64, 100])
+def test_merged_splits_of_a_long_context(splits, last, dk):
+    # 128 positions a split: one to eight waves of the merge, with equal and
+    # unequal shares, within the float32 bound of the whole sum
+    rng = np.random.default_rng(splits + dk)
+    run_case(Model(2, 1, dk, dk // 2, rng), 1, 128 * (splits - 1) + last - 1, rng)
+
+
 @pytest.mark.parametrize("H,KV,dk,half,seq,cache_len", [
     (8, 2, 128, 64, 1, 0), (8, 2, 128, 64, 1, 130), (8, 2, 128, 64, 1, 2047), (8, 2, 128, 64, 3, 70),
     (32, 8, 128, 64, 1, 128), (16, 2, 64, 32, 1, 300), (6, 3, 96, 48, 1, 65), (4, 2, 64, 32, 5, 40)])
