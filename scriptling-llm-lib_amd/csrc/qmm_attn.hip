@@ -113,21 +113,33 @@ __global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_kernel(AttnArgs a) 
     __shared__ float rc[kMaxDk / 2], rs[kMaxDk / 2];
     const int s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int dk = a.d_k;
-    for (int i = threadIdx.x; i < a.half_dim; i += 64 * kPrepWaves) {
-        const float ang = a.freqs[i] * (float)(a.start_pos + s);
-        double sd, cd;
-        sincos((double)ang, &sd, &cd);
-        rc[i] = (float)cd;
-        rs[i] = (float)sd;
-    }
-    __syncthreads();
     float *row = rows[wave];
-    for (int t = blockIdx.y * kPrepWaves + wave; t < a.n_heads + a.n_kv; t += gridDim.y * kPrepWaves) {
+    auto prep = [&](int t) {
         const bool isq = t < a.n_heads;
         const int h = isq ? t : t - a.n_heads;
         const int cols = (isq ? a.n_heads : a.n_kv) * dk;
         prep_row(row, (isq ? a.q : a.k) + (size_t)s * cols + (size_t)h * dk, dk, isq ? a.q_bias : a.k_bias, h * dk,
                  isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, nullptr, 0, 0, lane);
+    };
+    // the first head's row is loaded with the frequency (half_dim is below the
+    // workgroup's threads), not behind the rotation's barrier
+    const int first = blockIdx.y * kPrepWaves + wave;
+    const float fr = (int)threadIdx.x < a.half_dim ? a.freqs[threadIdx.x] : 0.0f;
+    if (first < a.n_heads + a.n_kv) prep(first);
+    static_assert(kMaxDk / 2 <= 64 * kPrepWaves, "a thread per frequency");
+    if ((int)threadIdx.x < a.half_dim) {
+        const float ang = fr * (float)(a.start_pos + s);
+        double sd, cd;
+        sincos((double)ang, &sd, &cd);
+        rc[threadIdx.x] = (float)cd;
+        rs[threadIdx.x] = (float)sd;
+    }
+    __syncthreads();
+    for (int t = first; t < a.n_heads + a.n_kv; t += gridDim.y * kPrepWaves) {
+        const bool isq = t < a.n_heads;
+        const int h = isq ? t : t - a.n_heads;
+        const int cols = (isq ? a.n_heads : a.n_kv) * dk;
+        if (t != first) prep(t);
         // RoPE (applyRopeInPlaceF32, float32_ops.go:174-188)
         for (int i = lane; i < a.half_dim; i += 64) {
             const float c = rc[i], sn = rs[i];
