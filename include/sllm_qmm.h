@@ -348,7 +348,9 @@ sllm_status sllm_attention_dev(sllm_kv_cache *kv, int layer, const sllm_attn_par
  * attention as sllm_attention_dev (same kernels, bit-identical outputs), but
  * its scratch - the rotated q rows and the split states - lives in a static
  * 8 MiB device array per GPU, held until the process ends, so the call
- * allocates nothing and never touches the stream's workspace. Calls that
+ * allocates nothing and never touches the stream's workspace. (Prompts whose
+ * matrix-core scratch does not fit there keep the split kernel: the same dots
+ * and weights, the sums in another order.) Calls that
  * need more scratch than that (about seq_len x n_heads x (d_k x 4 bytes) for
  * the q rows, plus the split states of long caches; a decode step of a
  * 64-head model at 8K positions needs about 2 MiB) return SLLM_ERR_SHAPE.
@@ -450,7 +452,8 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  weights of 2^24 elements or more, 16 for smaller ones;
  *                                  Q5_0, Q2K and Q3K: 5 from 2^25 elements, else 8; the
  *                                  int8 formats 5 where the short-prompt GEMM takes them:
- *                                  up to 32 rows and 8192 columns (a multiple of 256);
+ *                                  up to 32 rows and 8192 columns (a multiple of 256;
+ *                                  4096 for at most 2048 weight rows);
  *                                  the GEMM and GEMV sum a row's blocks in different
  *                                  orders, so a row's last bits can change with it)
  *   gemm_shape          0..5       GEMM workgroups: 1 = 64 x 128 tiles, 2 = 64 x 64 tiles with

@@ -134,18 +134,24 @@ sllm_status amax_scratch(hipStream_t stream, void **out) {
 // bytes (to at least twice its size, so retired buffers total less than the
 // live one). The old buffer is retired, not freed (work queued on the stream
 // and graphs captured on it may still use it). A stream under capture cannot
-// grow its workspace: the caller reserves it first (sllm_workspace_reserve).
-sllm_status workspace(hipStream_t stream, size_t need, void **out, size_t *cap) {
+// grow its workspace: the caller reserves it first (sllm_workspace_reserve), or,
+// given `stuck`, is told so there instead of by an error.
+sllm_status workspace(hipStream_t stream, size_t need, void **out, size_t *cap, bool *stuck = nullptr) {
     int dev = 0;
     SLLM_HIP(hipGetDevice(&dev));
     const uint64_t key = ((uint64_t)(uintptr_t)stream << 8) ^ (uint64_t)dev;
     std::lock_guard<std::mutex> lk(g_mu);
     Ws &w = g_ws[key];
     if (w.cap < need) {
-        if (capturing(stream))
+        if (capturing(stream)) {
+            if (stuck) {
+                *stuck = true;
+                return SLLM_OK;
+            }
             return set_error(SLLM_ERR_ARG, "the stream's workspace must grow to " + std::to_string(need) +
                                                " bytes while the stream is capturing; call "
                                                "sllm_workspace_reserve on it before the capture");
+        }
         size_t want = need < ((size_t)4 << 20) ? ((size_t)4 << 20) : need;
         want = want < 2 * w.cap ? 2 * w.cap : want;
         void *p = nullptr;
@@ -480,17 +486,15 @@ sllm_status with_upload(const void *host, size_t bytes, size_t extra, F fn) {
 // How the matmuls of one call may run. ws: the bf16 GEMM of the fp32-activation
 // formats and the short-prompt GEMM may; false on a stream under capture whose
 // workspace cannot hold what they need (those calls take the GEMV, which needs
-// none, or the tiled GEMM). rows: output rows of all the call's weights (the
-// short-prompt GEMM's launch).
+// none, or the tiled GEMM).
 struct Route {
     bool ws = true;
-    int64_t rows = 0;
 };
 
 // The short-prompt GEMM takes a weight's rows (an explicit tile shape or K split
 // asks for the tiled GEMM).
 bool sgemm_route(const sllm_weight *w, int x_rows, const Route &r) {
-    return r.ws && sgemm_supported(w->fmt, w->groups, x_rows, r.rows) && !tuning().gemm_shape && !tuning().gemm_splits;
+    return r.ws && sgemm_supported(w->fmt, w->groups, x_rows, w->rows) && !tuning().gemm_shape && !tuning().gemm_splits;
 }
 
 bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
@@ -512,6 +516,8 @@ bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
     // The short-prompt GEMM from 5 rows, where the GEMV takes a second launch
     // (GEMV / GEMM: Q4_1 14336x4096 at M = 4 17.6 / 21.4, M = 5 25.0 / 20.9, Q8_0
     // 1536x768 5.5 / 8.0 and 8.0 / 8.1, Q5K1 4096x4096 9.9 / 14.9 and 15.1 / 14.9).
+    // Narrow weights too (Q5K1 1024x4096 at M = 5 11.1 / 11.1, Q8_0 10.0 / 10.5): beside
+    // a wide one in a GEMV of their own, a q / k / v call at M = 6 took 33.8 us.
     if (min_rows == 0 && sgemm_route(w, x_rows, r)) min_rows = 5;
     if (min_rows == 0) min_rows = (int64_t)w->rows * w->cols >= ((int64_t)1 << 24) ? 8 : 16;
     if (kq_native(w->fmt) && !w->kq_gemm) return false;
@@ -532,11 +538,6 @@ int gemm_fmt(const sllm_weight *w) { return w->fmt == SLLM_Q5K1 && w->q5_one_mfm
 
 bool uses_sgemm(const sllm_weight *w, int x_rows, const Route &r) {
     return sgemm_route(w, x_rows, r) && uses_gemm(w, x_rows, r);
-}
-int64_t total_rows(const sllm_weight *const *ws, int count) {
-    int64_t n = 0;
-    for (int i = 0; i < count; i++) n += ws[i]->rows;
-    return n;
 }
 // Every weight takes an int8 GEMM: the rows can be normed as they are quantized.
 bool all_int8_gemm(const sllm_weight *const *ws, int count, int x_rows, const Route &r) {
@@ -561,13 +562,19 @@ sllm_status run_matmul(const sllm_weight *w, const float *x, int x_rows, float *
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// The workspace bytes of a call, need(); r.ws is cleared where the stream is being
-// captured and its workspace is too small.
+// The workspace of a call that needs need() bytes, written to *bytes; r.ws is
+// cleared where the stream is being captured and its workspace is too small.
 template <class F>
-size_t fit_workspace(hipStream_t s, Route &r, F need) {
-    const size_t n = need();
-    r.ws = n == 0 || workspace_at_hand(s, n);
-    return r.ws ? n : need();
+sllm_status fit_workspace(hipStream_t s, Route &r, F need, void **ws, size_t *bytes) {
+    size_t cap = 0;
+    *ws = nullptr;
+    if ((*bytes = need()) == 0) return SLLM_OK;
+    bool stuck = false;
+    const sllm_status st = workspace(s, *bytes, ws, &cap, &stuck);
+    if (!stuck) return st;
+    r.ws = false;
+    if ((*bytes = need()) == 0) return SLLM_OK;
+    return workspace(s, *bytes, ws, &cap);
 }
 
 // GEMM activation workspace the GEMM-bound weights of a set need (the largest).
@@ -576,7 +583,7 @@ size_t multi_gemm_ws(const sllm_weight *const *ws, int count, int x_rows, const 
     for (int i = 0; i < count; i++)
         if (uses_gemm(ws[i], x_rows, r)) {
             const size_t b = uses_sgemm(ws[i], x_rows, r)
-                                 ? sgemm_act_bytes(ws[i]->groups)
+                                 ? sgemm_ws_bytes(ws[i]->groups, x_rows, ws[i]->rows)
                                  : gemm_workspace_bytes(gemm_fmt(ws[i]), ws[i]->rows, ws[i]->groups, x_rows);
             need = b > need ? b : need;
         }
@@ -657,7 +664,7 @@ bool swiglu_sgemm(const sllm_weight *wg, const sllm_weight *wu, int x_rows, cons
 size_t swiglu_ws_bytes(const sllm_weight *wg, const sllm_weight *wu, int x_rows, const float *gate,
                        const float *up, const Route &r) {
     if (swiglu_paired(wg, wu, x_rows, r)) return 0;
-    if (swiglu_sgemm(wg, wu, x_rows, r)) return sgemm_act_bytes(wg->groups);
+    if (swiglu_sgemm(wg, wu, x_rows, r)) return sgemm_ws_bytes(wg->groups, x_rows, wg->rows);
     const sllm_weight *pair[2] = {wg, wu};
     const size_t mm = align256((size_t)x_rows * wg->rows * sizeof(float));
     return multi_gemm_ws(pair, 2, x_rows, r) + (gate ? 0 : mm) + (up ? 0 : mm);
@@ -1099,11 +1106,11 @@ sllm_status sllm_matmul_dev(const sllm_weight *w, const float *x, int x_rows, in
     if (st != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     void *ws = nullptr;
-    size_t cap = 0;
-    Route r{true, w->rows};
-    const size_t need = fit_workspace(s, r, [&] { return multi_gemm_ws(&w, 1, x_rows, r); });
-    if (need && (st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
-    return run_matmul(w, x, x_rows, dst, s, ws, cap, r);
+    size_t need = 0;
+    Route r;
+    st = fit_workspace(s, r, [&] { return multi_gemm_ws(&w, 1, x_rows, r); }, &ws, &need);
+    if (st != SLLM_OK) return st;
+    return run_matmul(w, x, x_rows, dst, s, ws, need, r);
 }
 
 sllm_status sllm_matmul_argmax_dev(const sllm_weight *w, const float *x, int x_cols, float *logits, int *argmax,
@@ -1147,10 +1154,10 @@ sllm_status sllm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_weight *wu,
     if ((st = ensure_init()) != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     void *ws = nullptr;
-    size_t cap = 0;
-    Route r{true, 2 * (int64_t)wg->rows};
-    const size_t need = fit_workspace(s, r, [&] { return swiglu_ws_bytes(wg, wu, x_rows, gate, up, r); });
-    if (need && (st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
+    size_t need = 0;
+    Route r;
+    st = fit_workspace(s, r, [&] { return swiglu_ws_bytes(wg, wu, x_rows, gate, up, r); }, &ws, &need);
+    if (st != SLLM_OK) return st;
     return swiglu_impl(wg, wu, x, x_rows, h, gate, up, s, ws, nullptr, 0.0f, r);
 }
 
@@ -1170,13 +1177,13 @@ sllm_status sllm_rmsnorm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_wei
     // several rows / mixed formats: normed rows into the workspace first
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
     void *ws = nullptr;
-    size_t cap = 0;
+    size_t need = 0;
     const sllm_weight *const both[2] = {wg, wu};
-    Route r{true, 2 * (int64_t)wg->rows};
-    const size_t need = fit_workspace(s, r, [&] {
+    Route r;
+    auto bytes = [&] {
         return (all_int8_gemm(both, 2, x_rows, r) ? 0 : nb) + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, r);
-    });
-    if ((st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
+    };
+    if ((st = fit_workspace(s, r, bytes, &ws, &need)) != SLLM_OK) return st;
     if (all_int8_gemm(both, 2, x_rows, r))  // normed as they are quantized
         return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, ws, norm_w, eps, r);
     float *normed = (float *)ws;
@@ -1239,10 +1246,10 @@ sllm_status sllm_matmul_multi_dev(const sllm_weight *const *ws, int count, const
     if ((st = ensure_init()) != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     void *gws = nullptr;
-    size_t cap = 0;
-    Route r{true, total_rows(ws, count)};
-    const size_t need = fit_workspace(s, r, [&] { return multi_gemm_ws(ws, count, x_rows, r); });
-    if (need && (st = workspace(s, need, &gws, &cap)) != SLLM_OK) return st;
+    size_t need = 0;
+    Route r;
+    st = fit_workspace(s, r, [&] { return multi_gemm_ws(ws, count, x_rows, r); }, &gws, &need);
+    if (st != SLLM_OK) return st;
     return multi_impl(ws, count, x, x_rows, dst, s, gws, need, nullptr, 0.0f, r);
 }
 
@@ -1260,15 +1267,13 @@ sllm_status sllm_rmsnorm_matmul_multi_dev(const sllm_weight *const *ws, int coun
     if (x_rows == 1 && multi_gemm_ws(ws, count, x_rows, Route{}) == 0)
         return multi_impl(ws, count, x, x_rows, dst, s, nullptr, 0, norm_w, eps, Route{});
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
-    Route r{true, total_rows(ws, count)};
-    const size_t need = fit_workspace(s, r, [&] {
-        return (all_int8_gemm(ws, count, x_rows, r) ? 0 : nb) + multi_gemm_ws(ws, count, x_rows, r);
-    });
+    Route r;
+    auto bytes = [&] { return (all_int8_gemm(ws, count, x_rows, r) ? 0 : nb) + multi_gemm_ws(ws, count, x_rows, r); };
     // several rows: normed rows into the workspace first, then every weight
     // reads them (GEMV and GEMM alike)
     void *ws_ = nullptr;
-    size_t cap = 0;
-    if ((st = workspace(s, need, &ws_, &cap)) != SLLM_OK) return st;
+    size_t need = 0;
+    if ((st = fit_workspace(s, r, bytes, &ws_, &need)) != SLLM_OK) return st;
     if (all_int8_gemm(ws, count, x_rows, r))  // normed as they are quantized
         return multi_impl(ws, count, x, x_rows, dst, s, ws_, need, norm_w, eps, r);
     float *normed = (float *)ws_;
@@ -1454,12 +1459,12 @@ sllm_status sllm_matmul_add_dev(const sllm_weight *w, const float *x, int x_rows
     if (st != SLLM_OK) return st;
     hipStream_t s = (hipStream_t)stream;
     const Planes P = as_const(w->planes);
-    Route r{true, w->rows};
-    const size_t need = fit_workspace(s, r, [&] { return multi_gemm_ws(&w, 1, x_rows, r); });
-    if (!need) return launch_gemv_add(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
+    Route r;
     void *ws = nullptr;
-    size_t cap = 0;
-    if ((st = workspace(s, need, &ws, &cap)) != SLLM_OK) return st;
+    size_t need = 0;
+    st = fit_workspace(s, r, [&] { return multi_gemm_ws(&w, 1, x_rows, r); }, &ws, &need);
+    if (st != SLLM_OK) return st;
+    if (!need) return launch_gemv_add(gemv_fmt(w), P, x, dst, w->rows, w->groups, x_rows, s);
     if (uses_sgemm(w, x_rows, r)) {  // adds in its epilogue
         if ((st = launch_sact(x, nullptr, 0.0f, x_rows, w->groups, ws, s)) != SLLM_OK) return st;
         return launch_sgemm(gemm_fmt(w), &P, &dst, &w->rows, 1, 1, w->groups, x_rows, ws, s);

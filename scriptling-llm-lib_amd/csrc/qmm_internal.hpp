@@ -221,13 +221,12 @@ sllm_status launch_gemm_dots(int fmt, const Planes &P, const float *x, float *ds
 size_t gemm_workspace_bytes(int fmt, int N, int G, int M);
 bool gemm_supported(int fmt, int G);  // int8 formats: K a multiple of 128 (others stay on the GEMV)
 // Short prompts of the int8 formats (qmm_sgemm.hip): the activation rows normed
-// (norm_w, may be null) and quantized once into act (sgemm_act_bytes), then up to
+// (norm_w, may be null) and quantized once into act (sgemm_ws_bytes), then up to
 // kMaxSegs weights of one format in a launch. mode: 0 dst = product, 1 dst +=
 // product, 2 (two weights, gate and up) dst[0] = SwiGLU, dst[1] / dst[2] (may be
 // null) the products.
-// rows: the output rows of all weights of the call.
 bool sgemm_supported(int fmt, int G, int M, int64_t rows);
-size_t sgemm_act_bytes(int G);
+size_t sgemm_ws_bytes(int G, int M, int64_t rows);
 sllm_status launch_sact(const float *x, const float *norm_w, float eps, int M, int G, void *act, hipStream_t s);
 sllm_status launch_sgemm(int fmt, const Planes *P, float *const *dst, const int *N, int nseg, int mode, int G, int M,
                          const void *act, hipStream_t s);

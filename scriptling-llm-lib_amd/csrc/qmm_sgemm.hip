@@ -15,8 +15,11 @@
 //   barrier. (Each lane loading its own row's line read it in pieces: 14336x4096
 //   Q4_1 at M = 32 25.3 us, 34.9 with non-temporal loads, which fetch the line
 //   again for every piece.)
-// * the W waves of a workgroup split K between them and meet in LDS once, in
-//   wave order, where the epilogue is applied: one launch, no partials in memory.
+// * the W waves of a workgroup split K between them and meet in LDS once, where
+//   the epilogue is applied: one launch, no partials in memory. K is cut into 8 or
+//   16 parts whose sums are added as a binary tree, whichever waves form them:
+//   an output's order depends on K alone, so a weight gives the same bits alone,
+//   beside others and in a gate / up pair.
 // The per-block arithmetic is the tiled GEMM's: v_mfma_i32_32x32x32_i8 gives a
 // block's exact dots on top of 1.5 * 2^23, t = fma(F, d, -1.5 * 2^23 d), acc =
 // fma(t, xs, acc), min terms two blocks at a time through v_mfma_f32_32x32x2_f32;
@@ -40,7 +43,11 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int kMagicBits = 0x4B400000;  // 1.5 * 2^23
 constexpr float kMagic = 12582912.0f;
 constexpr float kHugeXs = 0x1p90f;
-constexpr int kCh = 8;  // blocks per chunk
+constexpr int kCh = 8;      // blocks per chunk
+constexpr int kSplits = 8;  // K splits of a narrow weight's launch
+// Parts of K, each summed by itself: a wave's in a narrow weight's launch, one
+// chunk up to 4096 columns.
+__host__ __device__ constexpr int parts_of(int G) { return G > 64 ? 16 : 8; }
 
 __host__ __device__ constexpr bool has_min(int f) { return f == SLLM_Q4_1 || f == SLLM_Q5K1 || f == SLLM_Q5K1F; }
 __host__ __device__ constexpr bool dual(int f) { return f == SLLM_Q5K1; }
@@ -239,11 +246,23 @@ __device__ __forceinline__ void read_xs(const Image<FMT> &I, int b, int h, float
     }
 }
 
-// Grid: column tiles of 32; W waves.
+// The sum of n (1, 2, 4 or 8) values, at(0) .. at(n - 1), as a binary tree.
+template <class F>
+__device__ __forceinline__ float tree_sum(int n, F at) {
+    float s = at(0);
+    if (n >= 2) s = s + at(1);
+    if (n >= 4) s = s + (at(2) + at(3));
+    if (n >= 8) s = s + ((at(4) + at(5)) + (at(6) + at(7)));
+    return s;
+}
+
+// Grid: column tiles of 32, K splits (1, or kSplits with W = 2: one weight, its partial
+// sums to S.dst[0] as [split][M][N]); W waves.
 // LDS: every wave's image of its current chunk, then (after a barrier) the waves'
 // sums.
 template <int FMT, int W>
-__global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, int G) {
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2)))
+sgemm_kernel(SegG S, SAct A, int M, int G) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -264,9 +283,11 @@ __global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, in
             N = S.N[s];
         }
     const int n0 = ((int)blockIdx.x - S.tile0[seg]) * 32;
-    // this wave's chunks [c0, c1)
-    const int nch = G / kCh;
-    const int c0 = nch * kw / KW, c1 = nch * (kw + 1) / KW;
+    // this wave's parts of K: per (1, 2 or 4) of them, chunks [c0, c1)
+    const int nch = G / kCh, parts = parts_of(G);
+    const int per = parts / (KW * (int)gridDim.y);
+    const int p0 = ((int)blockIdx.y * KW + kw) * per;
+    const int c0 = nch * p0 / parts, c1 = nch * (p0 + per) / parts;
 
     v16f acc;
 #pragma unroll
@@ -275,6 +296,25 @@ __global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, in
 #pragma unroll
     for (int v = 0; v < 16; v++) cmag[v] = kMagicBits;
 
+    // acc: the current part's sum; ones, twos: finished parts that wait for their
+    // neighbours in the tree
+    v16f ones, twos;
+    auto close_part = [&](int i) {
+        if (i & 1) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] = ones[v] + acc[v];
+            if (i & 2) {
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[v] = twos[v] + acc[v];
+            }
+        }
+        if (i + 1 < per) {
+            if (i & 1) twos = acc;
+            else ones = acc;
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+        }
+    };
     if (c0 < c1) {
         Image<FMT> &I = ((Image<FMT> *)lds)[wave];
         Chunk<FMT> ck;
@@ -294,7 +334,12 @@ __global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, in
             load_chunk<FMT>(ck, P, n0, N, G, c * kCh, lane);
         };
         load(c0);
+        int part = 0, cend = nch * (p0 + 1) / parts;
         for (int c = c0; c < c1; c++) {
+            while (c == cend) {  // parts may be empty
+                close_part(part++);
+                cend = nch * (p0 + part + 1) / parts;
+            }
             const int cnx = min(c + 1, c1 - 1);
             bool slow = any_nonfinite(ck.sc);
             if (dual(FMT)) slow |= any_nonfinite(ck.dh);
@@ -397,9 +442,10 @@ __global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, in
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
         }
+        for (; part < per; part++) close_part(part);
     }
 
-    // the waves' sums meet in LDS: [wave][16][64], added in wave order
+    // the waves' sums meet in LDS: [wave][16][64]
     __syncthreads();
 #pragma unroll
     for (int v = 0; v < 16; v++) lds[(wave * 16 + v) * 64 + lane] = acc[v];
@@ -410,18 +456,17 @@ __global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, in
     for (int s = 1; s < kMaxSegs; s++)
         if (s == seg) dst = S.dst[s];
     const int Ns = pair ? S.N[0] : N;
+    dst += (size_t)blockIdx.y * M * Ns;
 #pragma unroll
     for (int i = 0; i < E / (64 * W); i++) {
         const int e = threadIdx.x + 64 * W * i;
         const int l = e & 63, v = e >> 6;
         const int m = 8 * (v >> 2) + 4 * (l >> 5) + (v & 3), col = n0 + (l & 31);
-        float s = lds[e];
-        for (int w = 1; w < KW; w++) s = s + lds[w * E + e];
+        const float s = tree_sum(KW, [&](int w) { return lds[w * E + e]; });
         if (m >= M || col >= Ns) continue;
         const size_t o = (size_t)m * Ns + col;
         if (pair) {
-            float u = lds[KW * E + e];
-            for (int w = 1; w < KW; w++) u = u + lds[(KW + w) * E + e];
+            const float u = tree_sum(KW, [&](int w) { return lds[(KW + w) * E + e]; });
             dst[o] = swiglu(s, u);
             if (S.dst[1]) S.dst[1][o] = s;
             if (S.dst[2]) S.dst[2][o] = u;
@@ -431,38 +476,69 @@ __global__ void __launch_bounds__(64 * W) sgemm_kernel(SegG S, SAct A, int M, in
     }
 }
 
+// The upper levels of the tree over a narrow weight's K splits.
+__global__ void __launch_bounds__(256) split_sum_kernel(const float *__restrict__ part, float *__restrict__ dst, int n,
+                                                        int add) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float s = tree_sum(kSplits, [&](int k) { return part[(size_t)k * n + i]; });
+    dst[i] = add ? dst[i] + s : s;
+}
+
+// A weight of 64 tiles or fewer and more than 64 blocks of K: launched by itself it
+// is cut into K splits, one chunk of K to a wave (Q5K1 1024x4096 at M = 32 11.7 us,
+// 13.3 in four splits of two chunks, 14.8 in one launch).
+bool narrow(int64_t rows, int G) { return rows <= 2048 && G > 64; }
+
 template <int FMT, int W>
-sllm_status launch_w(const SegG &S, const SAct &A, int M, int G, hipStream_t s) {
+sllm_status launch_w(const SegG &S, const SAct &A, int M, int G, hipStream_t s, int splits = 1) {
     constexpr size_t img = W * sizeof(Image<FMT>), red = (size_t)W * 1024 * sizeof(float);
     static_assert((img > red ? img : red) <= 160 * 1024, "LDS");
-    hipLaunchKernelGGL((sgemm_kernel<FMT, W>), dim3(S.tile0[S.n]), dim3(64 * W), img > red ? img : red, s, S, A, M, G);
+    hipLaunchKernelGGL((sgemm_kernel<FMT, W>), dim3(S.tile0[S.n], splits), dim3(64 * W), img > red ? img : red, s, S, A, M, G);
     SLLM_HIP(hipGetLastError());
     return SLLM_OK;
 }
 
 // Eight waves per tile, one tile per CU; with more tiles than CUs four, two
 // tiles per CU (14336x4096 at M = 30: eight waves run in two rounds, 21.4 against
-// 19.6 us).
+// 19.6 us), but not for a pair of more than 64 blocks of K, where a wave would have
+// eight parts to hold sums of.
 template <int FMT>
 sllm_status launch_f(const SegG &S, const SAct &A, int M, int G, hipStream_t s) {
-    return S.tile0[S.n] > 256 ? launch_w<FMT, 4>(S, A, M, G, s) : launch_w<FMT, 8>(S, A, M, G, s);
+    if (S.n == 1 && S.mode != kPair && narrow(S.N[0], G)) {
+        SegG T = S;
+        T.mode = kStore;
+        T.dst[0] = (float *)((char *)A.xq + ((sact_bytes(G) + 255) & ~(size_t)255));
+        const sllm_status st = launch_w<FMT, 2>(T, A, M, G, s, kSplits);
+        if (st != SLLM_OK) return st;
+        const int n = M * S.N[0];
+        hipLaunchKernelGGL(split_sum_kernel, dim3((n + 255) / 256), dim3(256), 0, s, T.dst[0], S.dst[0], n, S.mode == kAdd);
+        SLLM_HIP(hipGetLastError());
+        return SLLM_OK;
+    }
+    return S.tile0[S.n] > 256 && (S.mode != kPair || G <= 64) ? launch_w<FMT, 4>(S, A, M, G, s) : launch_w<FMT, 8>(S, A, M, G, s);
 }
 
 }  // namespace
 
-// Up to 32 rows and 8192 columns, for launches of 2048 output rows or more and,
-// with up to 2048 columns, of any. Measured (us, with the quantize pass; this /
-// the tiled GEMM, M = 16 and 32): Q4_1 14336x4096 20.6 / 27.6 and 20.9 / 28.6, Q8_0
+// Up to 32 rows and 8192 columns (4096 where the weight is narrow), whatever else the
+// call holds: a weight's bits do not depend on its company. Measured (us, with the quantize pass; this / the
+// tiled GEMM, M = 16 and 32): Q4_1 14336x4096 20.6 / 27.6 and 20.9 / 28.6, Q8_0
 // 4096x4096 13.6 / 16.0 and 13.7 / 18.4, Q5K1 4096x4096 14.8 / 14.6 and 14.8 /
 // 16.3, Q4_0 8192x2048 10.4 / 12.7 and 10.5 / 13.6, Q8_0 1536x768 8.2 / 11.4 and
-// 8.6 / 11.8; but Q5K1 1024x4096 14.6 / 11.5 (few tiles: a wave's two chunks of K
-// in turn), Q8_0 4096x14336 37.2 / 26.2 (seven), and with two row tiles (33 to 64
-// rows) Q4_1 14336x4096 39.4 / 28.8.
+// 8.6 / 11.8, narrow Q5K1 1024x4096 11.2 / 11.1 and 11.7 / 11.8; but Q4_0 512x8192
+// 13.7 / 12.4 and 14.1 / 13.0, Q8_0 4096x14336 37.2 / 26.2 (a wave's seven chunks of K in
+// turn), and with two row tiles (33 to 64 rows) Q4_1 14336x4096 39.4 / 28.8.
 bool sgemm_supported(int fmt, int G, int M, int64_t rows) {
-    return !act_f32(fmt) && G % kCh == 0 && M <= 32 && G <= 256 && (rows >= 2048 || G <= 64);
+    return !act_f32(fmt) && G % kCh == 0 && M <= 32 && G <= (rows <= 2048 ? 128 : 256);
 }
 
-size_t sgemm_act_bytes(int G) { return (sact_bytes(G) + 255) & ~(size_t)255; }
+// The codes, and the partial sums of a weight of so many rows that is launched by
+// itself.
+size_t sgemm_ws_bytes(int G, int M, int64_t rows) {
+    const size_t act = (sact_bytes(G) + 255) & ~(size_t)255;
+    return act + (narrow(rows, G) ? (size_t)kSplits * M * rows * sizeof(float) : 0);
+}
 
 sllm_status launch_sact(const float *x, const float *norm_w, float eps, int M, int G, void *act, hipStream_t s) {
     hipLaunchKernelGGL(sact_kernel, dim3(32), dim3(256), 0, s, x, norm_w, eps, M, G, carve_sact(act, G));
