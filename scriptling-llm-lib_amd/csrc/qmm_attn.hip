@@ -15,8 +15,8 @@
 // attn_prep_kernel (several rows): that work, a workgroup of eight waves over a
 //   row's heads.
 // attn_flash_kernel / attn_flash_combine_kernel (prompts): below.
-// attn_combine_kernel (more than one split): one workgroup per (row, head) merges
-//   the splits. Separate launches instead of a last-workgroup combine: on
+// attn_combine_kernel (more than one split), attn_combine_long_kernel (more than
+//   kShortSplits): merge the splits of every (row, head). Separate launches instead of a last-workgroup combine: on
 //   this multi-XCD part a device-scope fence writes back and invalidates the
 //   L2, which costs more than the launch.
 #include <hip/hip_runtime.h>
@@ -492,80 +492,131 @@ __global__ void __launch_bounds__(kMaxWaves * 64) attn_split_kernel(AttnArgs a) 
     }
 }
 
-// The splits of one (row, head), one workgroup of a wave per eight splits (at most
-// kCombineWaves): M = max of the split maxima, weights w_t = float32(exp(float64(m_t - M))), L = sum of l_t *
-// w_t, out[d] = (sum over t of o_t[d] * w_t) * (1 / L), written in
-// mergeHeadsDataF32's layout (float32_ops.go:262-273). Every wave takes a
-// consecutive share of the splits, eight at a time with all their loads issued
-// together, and the waves' sums are added in wave order. (One wave per head left
-// 32 waves on the device for a decode step, each with up to four rounds of memory
-// in turn: 9.0 us at 63 splits. One decode step, whole call, 32/8/128: 8000 cached
-// 32.1 -> 27.1 us, 4000 16.9 -> 15.6; 8/1/256: 8000 40.7 -> 29.7; up to 16 splits
-// the same.)
-constexpr int kCombineWaves = 8;
-__global__ void __launch_bounds__(64 * kCombineWaves) attn_combine_kernel(AttnArgs a) {
-    __shared__ float Ls[kCombineWaves], Os[kCombineWaves][kMaxDk];
+// The merge of the splits of one (row, head): M = max of the split maxima, weights
+// w_t = float32(exp(float64(m_t - M))), L = sum of l_t * w_t (lane t % 16 adds its
+// splits' terms in order, then the wave's tree), out[d] = (sum over t, in order, of
+// o_t[d] * w_t) * (1 / L), written in mergeHeadsDataF32's layout
+// (float32_ops.go:262-273). A split without positions (max -inf) weighs 0. Both
+// kernels below form every output in that one order.
+
+// Up to kShortSplits splits: one wave per (row, head), everything loaded together.
+constexpr int kShortSplits = 16;
+__global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int pair = blockIdx.x * 4 + (threadIdx.x >> 6);  // qi * n_heads + h
+    if (pair >= a.seq * a.n_heads) return;                 // wave-uniform
+    const int dk = a.d_k, nt = a.splits;
+    const size_t stride = (size_t)dk + 2;
+    const float *pb = a.part + (size_t)pair * nt * stride;
+    const bool mine = lane < nt;  // lane t holds m_t and l_t
+    const float ml = mine ? pb[lane * stride] : -INFINITY;
+    const float ll = mine ? pb[lane * stride + 1] : 0.0f;
+    float ov[kShortSplits][4];
+#pragma unroll
+    for (int u = 0; u < kShortSplits; u++) {
+        const float *ob = pb + (size_t)u * stride + 2;
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) {
+            const int d = lane + 64 * jj;
+            ov[u][jj] = (u < nt && d < dk) ? ob[d] : 0.0f;
+        }
+    }
+    float M = ml;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    const float wl = (mine && ml != -INFINITY) ? (float)exp((double)(ml - M)) : 0.0f;
+    float O[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < kShortSplits; u++) {
+        const float w = lane_bcast(wl, u);  // 0 past the last split, where the values are zeros
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) O[jj] = O[jj] + ov[u][jj] * w;
+    }
+    const float inv = 1.0f / wave_sum(0.0f + ll * wl);
+    float *dst = a.out + (size_t)pair * dk;  // mergeHeadsDataF32 layout
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) {
+        const int d = lane + 64 * jj;
+        if (d < dk) dst[d] = O[jj] * inv;
+    }
+}
+
+// More splits: one workgroup of eight waves per (row, head). In a round a wave takes
+// up to eight splits, all its loads issued together, and leaves their weighted values
+// in LDS; a thread per dimension then adds the round's in split order. (One wave per
+// head left 32 waves on the device for a decode step, each with a round of memory
+// per 16 splits: 9.0 us at 63 splits. One decode step, whole call, one wave / this:
+// 32/8/128 at 8000 cached 31.2 / 27.5 us, 4000 18.3 / 16.5; 8/1/256 at 8000 40.1 /
+// 32.0. Sums by wave, in another order, would take 26.1 at 8000.)
+constexpr int kLongWaves = 8, kRound = 8 * kLongWaves;
+__global__ void __launch_bounds__(64 * kLongWaves) attn_combine_long_kernel(AttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int pair = blockIdx.x;  // qi * n_heads + h
     const int dk = a.d_k;
+    float *P = lds, *T = lds + kRound * dk;  // [split of the round][d]; l_t * w_t
     const size_t stride = (size_t)dk + 2;
     const float *pb = a.part + (size_t)pair * a.splits * stride;
-    const int waves = blockDim.x >> 6;
-    const int s0 = a.splits * wave / waves, s1 = a.splits * (wave + 1) / waves;
-    float ov[8][4], ml[8], ll[8];
-    auto load8 = [&](int t0) {
+    // this wave's splits of the round from t0: u0 .. u0 + nu - 1 (none if nu <= 0);
+    // lane u holds split u0 + u's max and sum
+    int n, u0, nu;
+    float ov[8][4], ml, ll;
+    auto load = [&](int t0) {
+        n = min(kRound, a.splits - t0);
+        const int per = (n + kLongWaves - 1) / kLongWaves;
+        u0 = wave * per;
+        nu = min(per, n - u0);
+        const float *rb = pb + (size_t)(t0 + min(u0, n - 1)) * stride;
+        const int last = max(nu, 1) - 1;
+        ml = rb[min(lane, last) * stride];
+        ll = rb[min(lane, last) * stride + 1];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            const float *ob = pb + (size_t)min(t0 + u, a.splits - 1) * stride;
-            ml[u] = ob[0];
-            ll[u] = ob[1];
+            const float *ob = rb + min(u, last) * stride + 2;
 #pragma unroll
             for (int jj = 0; jj < 4; jj++) {
                 const int d = lane + 64 * jj;
-                ov[u][jj] = d < dk ? ob[2 + d] : 0.0f;
+                ov[u][jj] = d < dk ? ob[d] : 0.0f;
             }
         }
     };
-    load8(s0);
+    load(0);  // before the maxima are waited for
     float M = -INFINITY;
     for (int t = lane; t < a.splits; t += 64) M = fmaxf(M, pb[t * stride]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-    float L = 0.0f;
-    float O[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int t0 = s0; t0 < s1; t0 += 8) {
-        if (t0 > s0) load8(t0);
-        // lane u forms the weight of split t0 + u; a split without positions (-inf)
-        // weighs 0, and so does one past the share (its values are not added)
-        float mu = ml[0];
-#pragma unroll
-        for (int u = 1; u < 8; u++) mu = (lane & 7) == u ? ml[u] : mu;
-        const float wl = mu != -INFINITY ? (float)exp((double)(mu - M)) : 0.0f;
+    static_assert(kMaxDk <= 64 * kLongWaves, "a thread per dimension");
+    float O = 0.0f, Lp = 0.0f;
+    for (int t0 = 0; t0 < a.splits; t0 += kRound) {
+        if (t0 > 0) load(t0);
+        const float wl = ml != -INFINITY ? (float)exp((double)(ml - M)) : 0.0f;
+        if (lane < nu) T[u0 + lane] = ll * wl;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            if (t0 + u < s1) {
-                const float w = lane_bcast(wl, u);
-                L = L + ll[u] * w;
+            const float w = lane_bcast(wl, u);
 #pragma unroll
-                for (int jj = 0; jj < 4; jj++) O[jj] = O[jj] + ov[u][jj] * w;
+            for (int jj = 0; jj < 4; jj++) {
+                const int d = lane + 64 * jj;
+                if (u < nu && d < dk) P[(u0 + u) * dk + d] = ov[u][jj] * w;
             }
         }
-    }
-    if (lane == 0) Ls[wave] = L;
+        __syncthreads();
+        for (int t = lane & 15; t < n; t += 16) Lp = Lp + T[t];
+        if ((int)threadIdx.x < dk) {
+            int t = 0;
+            for (; t + 16 <= n; t += 16) {
+                float v[16];
 #pragma unroll
-    for (int jj = 0; jj < 4; jj++) {
-        const int d = lane + 64 * jj;
-        if (d < dk) Os[wave][d] = O[jj];
+                for (int u = 0; u < 16; u++) v[u] = P[(t + u) * dk + threadIdx.x];
+#pragma unroll
+                for (int u = 0; u < 16; u++) O = O + v[u];
+            }
+            for (; t < n; t++) O = O + P[t * dk + threadIdx.x];
+        }
+        if (t0 + kRound < a.splits) __syncthreads();  // read before the next round is written
     }
-    __syncthreads();
-    float Lt = 0.0f;
-    for (int w = 0; w < waves; w++) Lt = Lt + Ls[w];
-    const float inv = 1.0f / Lt;
-    for (int d = threadIdx.x; d < dk; d += blockDim.x) {
-        float o = 0.0f;
-        for (int w = 0; w < waves; w++) o = o + Os[w][d];
-        a.out[(size_t)pair * dk + d] = o * inv;  // mergeHeadsDataF32 layout
-    }
+    const float inv = 1.0f / wave_sum(lane < 16 ? Lp : 0.0f);
+    if ((int)threadIdx.x < dk) a.out[(size_t)pair * dk + threadIdx.x] = O * inv;  // mergeHeadsDataF32 layout
 }
 
 // ---------------------------------------------------------- prompts ----
@@ -1135,8 +1186,12 @@ sllm_status launch_attention(const AttnArgs &a, hipStream_t s) {
         }
     }
     if (a.splits > 1) {
-        const int waves = (a.splits + 7) / 8 < kCombineWaves ? (a.splits + 7) / 8 : kCombineWaves;
-        hipLaunchKernelGGL(attn_combine_kernel, dim3(a.seq * a.n_heads), dim3(64 * waves), 0, s, a);
+        const int pairs = a.seq * a.n_heads;
+        if (a.splits <= kShortSplits)
+            hipLaunchKernelGGL(attn_combine_kernel, dim3((pairs + 3) / 4), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL(attn_combine_long_kernel, dim3(pairs), dim3(64 * kLongWaves),
+                               (size_t)kRound * (a.d_k + 1) * sizeof(float), s, a);
         SLLM_HIP(hipGetLastError());
     }
     return SLLM_OK;

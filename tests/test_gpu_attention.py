@@ -295,6 +295,41 @@ def test_matmul_add_is_matmul_then_one_add(qtype, M):
     assert np.array_equal(dst.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("splits", [2, 8, 9, 16, 17, 63, 65, 131])
+def test_the_merge_adds_in_split_order(splits):
+    # every position of a split (128 of them) has one score and an integer value
+    # times a power of two, so the splits' states are exact and only the merge
+    # rounds: values in split order, the sums of weights by lane (split mod 16) and
+    # then in the wave's tree. Equal bits.
+    rng = np.random.default_rng(splits)
+    m = Model(2, 1, 4, 0, rng)
+    n = 128 * splits
+    c = (rng.integers(-40, 1, splits) / 8).astype(np.float32)
+    vals = (rng.integers(-500, 500, (splits, 128, 4)) * 2.0 ** rng.integers(-12, 1, (splits, 1, 4))).astype(np.float32)
+    K = np.zeros((n, 4), np.float32)
+    K[:, 0] = np.repeat(c, 128)
+    V = vals.reshape(n, 4)
+    kv = sq.KVCache(1, 1, 4, n)
+    for ptr, src in zip(kv.data(0), (K, V)):
+        dev_view(ptr, src.size).copy_(torch.from_numpy(src.reshape(-1)))
+    kv.set_length(n - 1)
+    q, k, v = (torch.from_numpy(a).cuda() for a in (np.tile(np.eye(1, 4, dtype=np.float32), 2), K[-1:], V[-1:]))
+    out = torch.full((8,), float("nan"), device="cuda")
+    sq.attention_dev(kv, 0, m.params, q.data_ptr(), k.data_ptr(), v.data_ptr(), 1, n - 1, out.data_ptr())
+    torch.cuda.synchronize()
+    f = np.float32
+    sc = c * f(0.5)
+    w = np.exp((sc - sc.max()).astype(np.float64)).astype(f)
+    L, O = np.zeros(16, f), np.zeros(4, f)
+    for t in range(splits):
+        L[t % 16] = L[t % 16] + f(128) * w[t]
+        O = O + vals[t].astype(np.float64).sum(0).astype(f) * w[t]
+    while L.size > 1:
+        L = L[::2] + L[1::2]
+    want = np.tile(O * (f(1) / L[0]), 2)
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.slow
 def test_prefill_rows_beyond_the_grid_limit():
     # seq_len x n_kv_heads above 65535 (the split kernel's grid y): the rows
