@@ -635,9 +635,8 @@ __global__ void __launch_bounds__(64 * kLongWaves) attn_combine_long_kernel(Attn
 //     B operand of a two-deep MFMA it pairs positions p and p + 4: P goes from
 //     accumulator to operand without leaving its registers, V is read to match.
 // Scores are fp32 dots of the same products as the reference's (in two halves,
-// added by the MFMA), the exponentials exp_neg's (fp32, the argument's
-// reduction compensated: rms error 0.290 ulp where float32(exp(float64(x))) has
-// 0.289), the sums fp32, in another association than the split kernel's.
+// added by the MFMA), the exponentials float32(exp(float64(x))) as the reference's
+// (exp_neg), the sums fp32, in another association than the split kernel's.
 //
 // What bounds it: the fp32 matrix cores (64 cycles per 32 x 32 x 2; 2 DK of
 // them per tile); the split kernel spent 64-lane VALU dots and one pass over K
@@ -664,28 +663,28 @@ __host__ __device__ inline int flash_chunk(const FlashPlan &f, int tiles) {
     return (tiles + n - 1) / n;
 }
 
-// exp(x) for x <= 0 (or NaN) to float32, in float32 operations: r = x - n ln 2 in
-// two parts (the first exact: n has at most 8 bits, the first constant 16), the
-// Taylor polynomial of exp(r) - 1 - r to r^8 (remainder 2^-32), and 1 + r added
-// with its rounding error carried along (Fast2Sum). Over [-80, 0] its rms error
-// is 0.2897 ulp (the rounded fp64 exp 0.2886), one argument in 67 differs from
-// that by an ulp; attention outputs are as far from 64 bits with either.
+// float32(exp(float64(x))) for a float32 x <= 0 (or NaN): the exponential in 64 bits,
+// rounded to float32 once. r = x - n ln 2 in two parts (the first product exact: n
+// has at most 8 bits, the first constant 42), |r| <= 0.35, the Taylor polynomial of
+// exp(r) to r^11 (remainder below 2^-46 of the value). Below -104 the float32 is 0.
 __device__ __forceinline__ float exp_neg(float x) {
-    const float n = __builtin_rintf(x * 1.44269504f);
-    const float rh = __builtin_fmaf(n, -0.693145752f, x);  // 0x3f317200: 16 bits of ln 2
-    const float rl = n * -1.42860677e-6f;
-    const float r = rh + rl;
-    float p = 2.48015873e-5f;  // 1 / 8!
-    p = __builtin_fmaf(p, r, 1.98412698e-4f);
-    p = __builtin_fmaf(p, r, 1.38888889e-3f);
-    p = __builtin_fmaf(p, r, 8.33333333e-3f);
-    p = __builtin_fmaf(p, r, 4.16666667e-2f);
-    p = __builtin_fmaf(p, r, 1.66666667e-1f);
-    p = __builtin_fmaf(p, r, 0.5f);
-    const float t = __builtin_fmaf(r * r, p, rl);
-    const float s = 1.0f + rh;
-    const float e = rh - (s - 1.0f);
-    const float y = __builtin_ldexpf(s + (e + t), (int)n);
+    const double xd = (double)x;
+    const double n = __builtin_rint(xd * 1.4426950408889634);
+    double r = __builtin_fma(n, -0x1.62e42fefa38p-1, xd);
+    r = __builtin_fma(n, -0x1.ef35793c7673p-45, r);
+    double p = 1.0 / 39916800.0;
+    p = __builtin_fma(p, r, 1.0 / 3628800.0);
+    p = __builtin_fma(p, r, 1.0 / 362880.0);
+    p = __builtin_fma(p, r, 1.0 / 40320.0);
+    p = __builtin_fma(p, r, 1.0 / 5040.0);
+    p = __builtin_fma(p, r, 1.0 / 720.0);
+    p = __builtin_fma(p, r, 1.0 / 120.0);
+    p = __builtin_fma(p, r, 1.0 / 24.0);
+    p = __builtin_fma(p, r, 1.0 / 6.0);
+    p = __builtin_fma(p, r, 0.5);
+    p = __builtin_fma(p, r, 1.0);
+    p = __builtin_fma(p, r, 1.0);
+    const float y = (float)__builtin_ldexp(p, (int)n);
     return x < -104.0f ? 0.0f : y;
 }
 

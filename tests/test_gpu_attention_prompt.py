@@ -66,3 +66,24 @@ def test_an_output_off_16_bytes_is_taken_as_before():
     a = _run(m, q, k, v, ck, cv, seq, cl)
     b = _run(m, q, k, v, ck, cv, seq, cl, offset=1)
     assert np.abs(a - b).max() <= 1e-5 * np.abs(a).max()  # two associations of the same float32 sums
+
+
+def test_weights_are_the_rounded_64_bit_exponential():
+    # two cached positions, scores 0 and x <= -18 with values 0 and 1 (the rows' own
+    # positions weigh 0): the sum of weights is 1 in float32, so the output is the
+    # weight itself, float32(exp(float64(x)))
+    rng = np.random.default_rng(8)
+    m = Model(8, 8, 4, 0, rng)
+    seq, cl = 600, 2
+    x = np.float32(-18) - rng.uniform(0, 86, size=(seq, 8)).astype(np.float32)
+    q = np.zeros((seq, 8, 4), np.float32)
+    q[..., 0], q[..., 1] = 2 * x, 1  # scale 1 / sqrt(4)
+    k = np.zeros((seq, 8, 4), np.float32)
+    k[..., 1] = -1e6
+    ck = np.zeros((8, cl + seq, 4), np.float32)
+    ck[:, 1, 0] = 1
+    cv = np.zeros_like(ck)
+    cv[:, 1] = 1
+    out = _run(m, q, k, np.ones_like(k), ck, cv, seq, cl)
+    want = np.exp(x.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(out.view(np.uint32), np.repeat(want, 4, -1).reshape(out.shape).view(np.uint32))
