@@ -834,11 +834,13 @@ attn_flash_kernel(AttnArgs a, FlashPlan f) {
             // the first positions a row meets: exp(-inf) = 0 exactly
             float alpha = 1.0f;
             if (any && !(m == mn)) alpha = (m == -INFINITY && mn < INFINITY) ? 0.0f : (float)exp((double)(m - mn));
+            // while every score so far is -inf a position weighs exp(-inf) = 0 (not exp(-inf + inf))
+            const float ref = mn == -INFINITY ? 0.0f : mn;
             float es = 0.0f;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const bool in = 8 * (v >> 2) + (v & 3) < left;
-                const float e = exp_neg(s[v] - mn);
+                const float e = exp_neg(s[v] - ref);
                 s[v] = in ? e : 0.0f;
                 es = es + s[v];
             }

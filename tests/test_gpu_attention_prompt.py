@@ -87,3 +87,22 @@ def test_weights_are_the_rounded_64_bit_exponential():
     out = _run(m, q, k, np.ones_like(k), ck, cv, seq, cl)
     want = np.exp(x.astype(np.float64)).astype(np.float32)
     assert np.array_equal(out.view(np.uint32), np.repeat(want, 4, -1).reshape(out.shape).view(np.uint32))
+
+
+def test_a_whole_tile_of_infinitely_low_scores():
+    # positions 0 .. 31 overflow to -inf and weigh 0, the others weigh the same
+    rng = np.random.default_rng(9)
+    m = Model(8, 8, 4, 0, rng)
+    seq, cl = 600, 40
+    q = np.full((seq, 8, 4), 1e20, np.float32)
+    ck = np.zeros((8, cl + seq, 4), np.float32)
+    ck[:, :32] = -1e20
+    cv = rng.normal(size=(8, cl + seq, 4)).astype(np.float32)
+    v = rng.normal(size=(seq, 8, 4)).astype(np.float32)
+    out = _run(m, q, np.zeros((seq, 8, 4), np.float32), v, ck, cv, seq, cl)
+    seen = np.concatenate([cv[:, 32:cl].transpose(1, 0, 2), v]).astype(np.float64)
+    n = 8 + np.arange(1, seq + 1)
+    want = np.cumsum(seen, 0)[8:] / n[:, None, None]
+    # float32 sums of up to 608 terms
+    bound = (2 * 608 + 8) * 2.0 ** -24 * np.cumsum(np.abs(seen), 0)[8:] / n[:, None, None]
+    assert np.all(np.abs(out - want) <= bound)
