@@ -346,14 +346,13 @@ sllm_status sllm_attention_dev(sllm_kv_cache *kv, int layer, const sllm_attn_par
  * memory: code under HIP graph capture (without a warm-up call on the
  * stream), serving loops and harnesses that forbid hipMalloc. The same
  * attention as sllm_attention_dev (same kernels, bit-identical outputs), but
- * its scratch - the rotated q rows and the split states - lives in a static
- * 8 MiB device array per GPU, held until the process ends, so the call
- * allocates nothing and never touches the stream's workspace. (Prompts whose
- * matrix-core scratch does not fit there keep the split kernel: the same dots
- * and weights, the sums in another order.) Calls that
- * need more scratch than that (about seq_len x n_heads x (d_k x 4 bytes) for
- * the q rows, plus the split states of long caches; a decode step of a
- * 64-head model at 8K positions needs about 2 MiB) return SLLM_ERR_SHAPE.
+ * its scratch - the rotated q rows, the split states and a prompt's
+ * matrix-core states - lives in a static 64 MiB device array per GPU, held
+ * until the process ends, so the call allocates nothing and never touches the
+ * stream's workspace. Calls whose q rows and split states need more than 8 MiB
+ * (about seq_len x n_heads x (d_k x 4 bytes) for the q rows, plus the split
+ * states of long caches; a decode step of a 64-head model at 8K positions needs
+ * about 2 MiB) return SLLM_ERR_SHAPE.
  * Every call on one GPU shares that GPU's array: calls that overlap on one
  * GPU (different streams, or graph replays running concurrently) race and
  * give wrong results; serialize them.

@@ -187,7 +187,6 @@ bool workspace_at_hand(hipStream_t stream, size_t need) {
 // each GPU comes from hipGetSymbolAddress, looked up once per device with
 // that device current, and kept in g_scratch. Nothing in it needs to start at
 // zero: every call writes the q rows and split states it reads.
-constexpr size_t kStaticScratchBytes = (size_t)8 << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 std::unordered_map<int, void *> g_scratch;  // device -> address of its scratch
 
@@ -757,18 +756,18 @@ sllm_status attention_impl(sllm_kv_cache *kv, int layer, const sllm_attn_params 
     size_t wsb = 0;
     attention_plan(seq_len, p->n_heads, kv->n_kv, kv->d_k, cl + seq_len, &splits, &tps, &tw, &hs, &wsb);
     // The matrix-core kernel needs more scratch where rows are long: where that
-    // cannot be had (the static scratch, a stream under capture), the split
-    // kernel's plan holds.
+    // cannot be had (a stream under capture), the split kernel's plan holds. (The
+    // static scratch holds it for every call that it takes.)
     size_t fwsb = 0;
     bool flash = attention_flash(seq_len, p->n_heads, kv->n_kv, kv->d_k, cl, out, &fwsb) &&
-                 (noalloc ? fwsb <= kStaticScratchBytes : fwsb <= wsb || workspace_at_hand(s, fwsb));
+                 (noalloc || fwsb <= wsb || workspace_at_hand(s, fwsb));
     void *ws = nullptr;
     size_t cap = 0;
     if (noalloc) {
-        if (wsb > kStaticScratchBytes)
+        if (wsb > kNoallocBytes)
             return set_error(SLLM_ERR_SHAPE, "attention needs " + std::to_string(wsb) +
                                                  " bytes of scratch, more than the static scratch's " +
-                                                 std::to_string(kStaticScratchBytes) +
+                                                 std::to_string(kNoallocBytes) +
                                                  " (fewer rows per call, or sllm_attention_dev)");
         if ((st = static_scratch(&ws)) != SLLM_OK) return st;
     } else if ((st = workspace(s, flash ? fwsb : wsb, &ws, &cap)) != SLLM_OK) {

@@ -1098,6 +1098,10 @@ namespace {
 // / 21.5; 32/4/128 128 23.8 / 28.3, 200 54.7 / 44.8; 16/16/80 64 19.9 / 17.4.
 constexpr int kFlashPairs = 512;
 
+size_t qrot_bytes(int seq, int n_heads, int d_k) {
+    return ((size_t)seq * n_heads * d_k * sizeof(float) + 255) & ~(size_t)255;
+}
+
 FlashPlan flash_plan(int seq, int n_heads, int n_kv, int d_k, int cache_len, size_t *part) {
     const int rep = n_heads / n_kv, U = (seq + 31) / 32 * rep;
     FlashPlan f;
@@ -1118,10 +1122,14 @@ FlashPlan flash_plan(int seq, int n_heads, int n_kv, int d_k, int cache_len, siz
     const int64_t all = total * n_kv, slots = 2 * (int64_t)tuning().attn_target_blocks;
     const int64_t c = (all + slots - 1) / slots, least = all > 1024 ? 3 : (all > 128 ? 2 : 1);
     f.chunk = (int)(c < least ? least : c);
+    // the states' most bytes; calls that the static scratch takes get what it holds
+    // beside the q rows, also on a stream's workspace: both give the same bits
+    const size_t most_part = qrot_bytes(seq, n_heads, d_k) <= kNoallocBytes ? kStaticScratchBytes - kNoallocBytes
+                                                                            : (size_t)256 << 20;
     for (;; f.chunk *= 2) {
         f.chunks = (most + f.chunk - 1) / f.chunk;
         *part = f.chunks > 1 ? (size_t)n_kv * f.groups * f.chunks * kFlashWaves * 32 * (d_k + 2) * sizeof(float) : 0;
-        if (*part <= ((size_t)256 << 20)) return f;
+        if (*part <= most_part) return f;
     }
 }
 
@@ -1139,8 +1147,7 @@ bool attention_flash(int seq, int n_heads, int n_kv, int d_k, int cache_len, con
     size_t part = 0;
     const FlashPlan f = flash_plan(seq, n_heads, n_kv, d_k, cache_len, &part);
     if (f.groups > 65535 || f.chunks > 65535) return false;  // grid y, z
-    const size_t qrot = (size_t)seq * n_heads * d_k * sizeof(float);
-    *ws_bytes = ((qrot + 255) & ~(size_t)255) + part;
+    *ws_bytes = qrot_bytes(seq, n_heads, d_k) + part;
     return true;
 }
 

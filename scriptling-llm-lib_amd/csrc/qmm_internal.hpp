@@ -288,6 +288,10 @@ struct AttnArgs {
 void attention_plan(int seq, int n_heads, int n_kv, int d_k, int kv_len, int *splits, int *tps, int *tw, int *hs,
                     size_t *ws_bytes);
 sllm_status launch_attention(const AttnArgs &a, hipStream_t s);
+// sllm_attention_noalloc_dev takes calls whose q rows and split states (attention_plan)
+// fit kNoallocBytes; its static scratch also holds the matrix-core kernel's states
+// for every one of them.
+constexpr size_t kNoallocBytes = (size_t)8 << 20, kStaticScratchBytes = (size_t)64 << 20;
 // Whether a prompt takes the matrix-core kernel (several rows, d_k up to 128, out
 // 16-byte aligned), and its workspace bytes; cache_len: rows held before the call.
 bool attention_flash(int seq, int n_heads, int n_kv, int d_k, int cache_len, const float *out, size_t *ws_bytes);

@@ -61,6 +61,26 @@ def test_noalloc_equals_attention_dev_on_two_calls():
     b.close()
 
 
+@pytest.mark.parametrize("seq,start", [(130, 0), (300, 37), (512, 0), (70, 900)])
+def test_noalloc_equals_attention_dev_on_prompts(seq, start):
+    # matrix-core prompts up to the most q rows the call takes (512 rows: 8 MiB)
+    rng = np.random.default_rng(seq)
+    m = Model(H, KV, DK, HALF, rng, base=500000.0)
+    cap = start + seq
+    kvs = [sq.KVCache(1, KV, DK, cap) for _ in range(2)]
+    q, k, v = (torch.from_numpy(rng.normal(size=(seq, n * DK)).astype(np.float32)).cuda() for n in (H, KV, KV))
+    outs = [torch.full((seq, H * DK), float("nan"), device="cuda") for _ in range(2)]
+    for kv, o, call in zip(kvs, outs, (sq.attention_dev, sq.attention_noalloc_dev)):
+        _fill(kv, np.random.default_rng(8), cap)
+        kv.set_length(start)
+        call(kv, 0, m.params, q.data_ptr(), k.data_ptr(), v.data_ptr(), seq, start, o.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.isfinite(outs[0]).all()
+    assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+    for kv in kvs:
+        kv.close()
+
+
 def test_noalloc_captures_on_a_fresh_stream():
     rng = np.random.default_rng(9)
     m = Model(H, KV, DK, HALF, rng, base=500000.0)
