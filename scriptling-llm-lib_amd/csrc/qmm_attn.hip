@@ -12,8 +12,7 @@
 //   state goes to the workspace. Scores are the reference's sequential
 //   float32 dots. For one query row (decode) it also does the bias / norm /
 //   RoPE / append work itself.
-// attn_prep_kernel (several rows): that work, a workgroup of eight waves over a
-//   row's heads.
+// attn_prep_kernel / attn_prep_rows_kernel (several rows): that work.
 // attn_flash_kernel / attn_flash_combine_kernel (prompts): below.
 // attn_combine_kernel (more than one split), attn_combine_long_kernel (more than
 //   kShortSplits): merge the splits of every (row, head). Separate launches instead of a last-workgroup combine: on
@@ -100,32 +99,62 @@ __device__ void prep_row(float *row, const float *src, int dk, const float *bias
     wave_lds_sync();
 }
 
-// Several rows (prefill): gridDim.y workgroups per row - q heads into the workspace, kv
-// heads into the cache (k: bias, norm, RoPE; v: bias) at rows cache_len + s
-// (the append, model_f32.go:445-448). The row's rotation (the same for every
-// head) is formed once per workgroup in LDS, then a wave takes every eighth head
-// of the workgroup's: with a workgroup and an fp64 sincos of its own for every
-// head, 1024 rows of 32 + 8 heads took 15.9 us (now 13.0). Few rows get a
-// workgroup for every eight heads, so that no wave takes two in turn.
+// Several rows (prefill): q heads go to the workspace, kv heads into the cache (k:
+// bias, norm, RoPE; v: bias) at rows cache_len + s (the append, model_f32.go:445-448).
+// prep_head: head t of row s (q heads, then kv heads) into row (LDS), rotated by `half`
+// frequencies; put_head: row to where it belongs.
+__device__ __forceinline__ void prep_head(const AttnArgs &a, int s, int t, float *row, int half, int lane) {
+    const int dk = a.d_k;
+    const bool isq = t < a.n_heads;
+    const int h = isq ? t : t - a.n_heads;
+    const int cols = (isq ? a.n_heads : a.n_kv) * dk;
+    prep_row(row, (isq ? a.q : a.k) + (size_t)s * cols + (size_t)h * dk, dk, isq ? a.q_bias : a.k_bias, h * dk,
+             isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, a.freqs, half, a.start_pos + s, lane);
+}
+__device__ __forceinline__ void put_head(const AttnArgs &a, int s, int t, const float *row, int lane) {
+    const int dk = a.d_k;
+    if (t < a.n_heads) {
+        float *dst = a.qrot + ((size_t)s * a.n_heads + t) * dk;
+        for (int d = lane; d < dk; d += 64) dst[d] = row[d];
+        return;
+    }
+    const int h = t - a.n_heads;
+    const size_t at = ((size_t)h * a.cap + (size_t)(a.cache_len + s)) * dk;
+    const float *vs = a.v + ((size_t)s * a.n_kv + h) * dk;
+    for (int d = lane; d < dk; d += 64) {
+        a.cache_k[at + d] = row[d];
+        float x = vs[d];
+        if (a.v_bias && h * dk + d < a.vb_len) x = x + a.v_bias[h * dk + d];
+        a.cache_v[at + d] = x;
+    }
+}
+
+// Few rows before the split kernel: one wave per (row, head).
+__global__ void __launch_bounds__(64) attn_prep_kernel(AttnArgs a) {
+    __shared__ float row[kMaxDk];
+    prep_head(a, blockIdx.x, blockIdx.y, row, a.half_dim, threadIdx.x);
+    put_head(a, blockIdx.x, blockIdx.y, row, threadIdx.x);
+}
+
+// Prompts: gridDim.y workgroups per row. The row's rotation (the same for every head)
+// is formed once per workgroup in LDS, then a wave takes every eighth head of the
+// workgroup's: with a workgroup and an fp64 sincos of its own for every head, 1024
+// rows of 32 + 8 heads took 15.9 us (now 13.0). Below kPrepRows rows a row has a
+// workgroup for every eight heads, so that no wave takes two in turn. (Whole calls,
+// us, one wave per head / one workgroup per row: 32/8/128 20 rows 10.3 / 12.1, 64
+// 10.9 / 13.6, 200 32.0 / 33.7, 512 62.6 / 62.8, 700 96.6 / 95.7.)
+constexpr int kPrepRows = 512;
 constexpr int kPrepWaves = 8;
-__global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_rows_kernel(AttnArgs a) {
     __shared__ float rows[kPrepWaves][kMaxDk];
     __shared__ float rc[kMaxDk / 2], rs[kMaxDk / 2];
     const int s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int dk = a.d_k;
     float *row = rows[wave];
-    auto prep = [&](int t) {
-        const bool isq = t < a.n_heads;
-        const int h = isq ? t : t - a.n_heads;
-        const int cols = (isq ? a.n_heads : a.n_kv) * dk;
-        prep_row(row, (isq ? a.q : a.k) + (size_t)s * cols + (size_t)h * dk, dk, isq ? a.q_bias : a.k_bias, h * dk,
-                 isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, nullptr, 0, 0, lane);
-    };
     // the first head's row is loaded with the frequency (half_dim is below the
     // workgroup's threads), not behind the rotation's barrier
-    const int first = blockIdx.y * kPrepWaves + wave;
     const float fr = (int)threadIdx.x < a.half_dim ? a.freqs[threadIdx.x] : 0.0f;
-    if (first < a.n_heads + a.n_kv) prep(first);
+    const int first = blockIdx.y * kPrepWaves + wave;
+    if (first < a.n_heads + a.n_kv) prep_head(a, s, first, row, 0, lane);
     static_assert(kMaxDk / 2 <= 64 * kPrepWaves, "a thread per frequency");
     if ((int)threadIdx.x < a.half_dim) {
         const float ang = fr * (float)(a.start_pos + s);
@@ -136,10 +165,7 @@ __global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_kernel(AttnArgs a) 
     }
     __syncthreads();
     for (int t = first; t < a.n_heads + a.n_kv; t += gridDim.y * kPrepWaves) {
-        const bool isq = t < a.n_heads;
-        const int h = isq ? t : t - a.n_heads;
-        const int cols = (isq ? a.n_heads : a.n_kv) * dk;
-        if (t != first) prep(t);
+        if (t != first) prep_head(a, s, t, row, 0, lane);
         // RoPE (applyRopeInPlaceF32, float32_ops.go:174-188)
         for (int i = lane; i < a.half_dim; i += 64) {
             const float c = rc[i], sn = rs[i];
@@ -148,19 +174,7 @@ __global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_kernel(AttnArgs a) 
             row[2 * i + 1] = x0 * sn + x1 * c;
         }
         wave_lds_sync();
-        if (isq) {
-            float *dst = a.qrot + ((size_t)s * a.n_heads + h) * dk;
-            for (int d = lane; d < dk; d += 64) dst[d] = row[d];
-        } else {
-            const size_t at = ((size_t)h * a.cap + (size_t)(a.cache_len + s)) * dk;
-            const float *vs = a.v + (size_t)s * cols + (size_t)h * dk;
-            for (int d = lane; d < dk; d += 64) {
-                a.cache_k[at + d] = row[d];
-                float x = vs[d];
-                if (a.v_bias && h * dk + d < a.vb_len) x = x + a.v_bias[h * dk + d];
-                a.cache_v[at + d] = x;
-            }
-        }
+        put_head(a, s, t, row, lane);
         wave_lds_sync();  // the row is read before the next head's is written
     }
 }
@@ -186,7 +200,7 @@ __global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_kernel(AttnArgs a) 
 // PREP (one query row): group 0's waves first build the q heads (bias, norm,
 // RoPE) in LDS, and in the workgroup whose range holds the new position the
 // last wave builds the new k / v row, appends it to the cache and the groups
-// use it from LDS; otherwise attn_prep_kernel has done both. Per tile the K
+// use it from LDS; otherwise the preparation has done both. Per tile the K
 // and V rows are loaded together (K straight to LDS, V to registers while
 // the scores are computed, then to the same LDS buffer): one memory latency
 // per tile, overlapped with the q preparation for the first tile (FULL; the
@@ -1080,10 +1094,14 @@ void launch_split(const AttnArgs &a, dim3 grid, size_t lds, hipStream_t s) {
 }
 
 namespace {
-sllm_status launch_prep(const AttnArgs &a, hipStream_t s) {
-    const int heads = a.n_heads + a.n_kv, most = (heads + kPrepWaves - 1) / kPrepWaves;
-    const int per_row = a.seq >= 2 * cus_per_device() ? 1 : most;
-    hipLaunchKernelGGL(attn_prep_kernel, dim3(a.seq, per_row), dim3(64 * kPrepWaves), 0, s, a);
+sllm_status launch_prep(const AttnArgs &a, bool flash, hipStream_t s) {
+    const int heads = a.n_heads + a.n_kv;
+    if (flash || a.seq >= kPrepRows)
+        hipLaunchKernelGGL(attn_prep_rows_kernel,
+                           dim3(a.seq, a.seq >= kPrepRows ? 1 : (heads + kPrepWaves - 1) / kPrepWaves),
+                           dim3(64 * kPrepWaves), 0, s, a);
+    else
+        hipLaunchKernelGGL(attn_prep_kernel, dim3(a.seq, heads), dim3(64), 0, s, a);
     SLLM_HIP(hipGetLastError());
     return SLLM_OK;
 }
@@ -1154,7 +1172,7 @@ bool attention_flash(int seq, int n_heads, int n_kv, int d_k, int cache_len, con
 sllm_status launch_attention_flash(const AttnArgs &a, hipStream_t s) {
     size_t part = 0;
     const FlashPlan f = flash_plan(a.seq, a.n_heads, a.n_kv, a.d_k, a.cache_len, &part);
-    const sllm_status st = launch_prep(a, s);
+    const sllm_status st = launch_prep(a, true, s);
     if (st != SLLM_OK) return st;
     switch ((a.d_k + 31) / 32) {
     case 1: launch_flash_dt<1>(a, f, s); break;
@@ -1179,7 +1197,7 @@ sllm_status launch_attention(const AttnArgs &a, hipStream_t s) {
         launch_split<true>(b, dim3(a.splits, a.n_kv * a.hs), lds, s);
         SLLM_HIP(hipGetLastError());
     } else {
-        const sllm_status st = launch_prep(a, s);
+        const sllm_status st = launch_prep(a, false, s);
         if (st != SLLM_OK) return st;
         // grid y is (row, kv head, head slice), at most 65535: long prefills
         // run in chunks of rows (every row's k / v is already in the cache)
