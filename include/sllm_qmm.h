@@ -330,7 +330,8 @@ typedef struct sllm_attn_params {
  * fixed order. One row (decode): two launches (the attention over splits of
  * the cached positions, which also prepares the row, then the combine of the
  * splits); several rows: three (the row preparation first). Prompts (more
- * than 512 pairs of row and kv head, d_k up to 128, out_dev 16-byte aligned)
+ * than 512 pairs of row and kv head, up to 1536 where few positions are seen;
+ * d_k up to 128, out_dev 16-byte aligned)
  * run on the fp32 matrix cores, where a score is the dots of the head's two
  * halves added; they use more workspace where it can be had (not on a
  * stream under capture whose workspace is smaller). Asynchronous on

@@ -635,7 +635,7 @@ __global__ void __launch_bounds__(64 * kLongWaves) attn_combine_long_kernel(Attn
 
 // ---------------------------------------------------------- prompts ----
 //
-// attn_flash_kernel: several query rows (more than kFlashPairs pairs of row and kv
+// attn_flash_kernel: several query rows (more than flash_pairs pairs of row and kv
 // head, d_k up to 128) on the fp32 matrix cores. A wave owns 32 query rows of one q head; the four
 // waves of a workgroup share one kv head's K and V tiles of 32 positions in LDS
 // (GQA: the q heads of the group; otherwise further row blocks). Both products
@@ -1109,12 +1109,22 @@ sllm_status launch_prep(const AttnArgs &a, bool flash, hipStream_t s) {
 
 namespace {
 // (query row, kv head) pairs above which a prompt takes attn_flash_kernel: up to
-// there the split kernel's one workgroup per pair all run at once, and its
-// shorter chain wins. Measured (us, split / matrix cores; q heads / kv heads /
-// d_k, rows): 32/8/128 64 13.2 / 21.3, 128 27.7 / 24.7, 1024 884 / 184; 32/32/64
-// 31 26.1 / 18.2 (99 cached), 200 139.5 / 32.5; 9/3/64 128 13.4 / 17.8, 200 23.9
-// / 21.5; 32/4/128 128 23.8 / 28.3, 200 54.7 / 44.8; 16/16/80 64 19.9 / 17.4.
-constexpr int kFlashPairs = 512;
+// there the split kernel's one workgroup per pair all run at once, and its shorter
+// chain wins. The fewer tiles of positions a row sees, the fewer tile groups (waves,
+// LDS) a workgroup has and the more run side by side; q heads above four per kv head
+// make it larger. Head sizes that are no multiple of 64 have the slower form of the
+// split kernel. Measured (us, split / matrix cores; q heads / kv heads / d_k, rows +
+// cached): 32/32/64 40 12.8 / 13.9, 48 13.9 / 14.1, 64 18.4 / 14.6; 16/16/128 48 10.3
+// / 17.5, 64 14.0 / 18.3; 40/40/128 13 + 30 10.3 / 16.9; 32/8/128 72 17.8 / 19.7, 96
+// 19.7 / 20.4, 112 25.4 / 21.2, 65 + 100 26.8 / 27.0; 24/8/128 96 19.2 / 20.9; 64/8/128
+// 65 25.2 / 21.1; 16/16/80 48 13.5 / 16.0, 64 19.2 / 16.6, 33 + 64 28.5 / 17.0;
+// 9/3/64 160 18.8 (split), 171 23.0 / 17.1; 32/4/128 128 22.4 (split), 129 32.8 / 22.6.
+int64_t flash_pairs(int rep, int d_k, int kv_len) {
+    const bool full = d_k % 64 == 0;
+    const int64_t one_tile = full ? 1536 : 768, two = full ? 768 : 512;
+    const int64_t n = (kv_len <= kTile ? one_tile : kv_len <= 2 * kTile ? two : 512) * 4 / (rep > 4 ? rep : 4);
+    return n > 512 ? n : 512;
+}
 
 size_t qrot_bytes(int seq, int n_heads, int d_k) {
     return ((size_t)seq * n_heads * d_k * sizeof(float) + 255) & ~(size_t)255;
@@ -1161,7 +1171,7 @@ void launch_flash_dt(const AttnArgs &a, const FlashPlan &f, hipStream_t s) {
 }  // namespace
 
 bool attention_flash(int seq, int n_heads, int n_kv, int d_k, int cache_len, const float *out, size_t *ws_bytes) {
-    if ((int64_t)seq * n_kv <= kFlashPairs || d_k > 128 || ((uintptr_t)out & 15) != 0) return false;
+    if ((int64_t)seq * n_kv <= flash_pairs(n_heads / n_kv, d_k, cache_len + seq) || d_k > 128 || ((uintptr_t)out & 15) != 0) return false;
     size_t part = 0;
     const FlashPlan f = flash_plan(seq, n_heads, n_kv, d_k, cache_len, &part);
     if (f.groups > 65535 || f.chunks > 65535) return false;  // grid y, z

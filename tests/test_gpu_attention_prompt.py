@@ -106,3 +106,21 @@ def test_a_whole_tile_of_infinitely_low_scores():
     # float32 sums of up to 608 terms
     bound = (2 * 608 + 8) * 2.0 ** -24 * np.cumsum(np.abs(seen), 0)[8:] / n[:, None, None]
     assert np.all(np.abs(out - want) <= bound)
+
+
+@pytest.mark.parametrize("H,KV,dk,seq,cl,flash", [
+    (32, 32, 64, 48, 0, False), (32, 32, 64, 49, 0, True), (40, 40, 128, 13, 30, False), (16, 16, 80, 48, 0, False),
+    (16, 16, 80, 49, 0, True), (32, 8, 128, 96, 0, False), (32, 8, 128, 97, 0, True), (32, 8, 128, 64, 65, False),
+    (32, 8, 128, 65, 64, True), (64, 8, 128, 64, 0, False), (64, 8, 128, 65, 0, True), (9, 3, 64, 170, 0, False),
+    (9, 3, 64, 171, 0, True), (5, 1, 256, 600, 0, False)])
+def test_the_line_between_the_kernels(H, KV, dk, seq, cl, flash):
+    # an output off 16 bytes always takes the split kernel: below the line both
+    # outputs have its bits, above it those of two associations
+    rng = np.random.default_rng(seq)
+    m = Model(H, KV, dk, 0, rng)
+    q, k, v = (rng.normal(size=(seq, n * dk)).astype(np.float32) for n in (H, KV, KV))
+    ck, cv = (rng.normal(size=(KV, cl + seq, dk)).astype(np.float32) for _ in range(2))
+    a = _run(m, q, k, v, ck, cv, seq, cl)
+    b = _run(m, q, k, v, ck, cv, seq, cl, offset=1)
+    assert np.abs(a - b).max() <= 1e-5 * np.abs(a).max()
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32)) is not flash
