@@ -354,3 +354,23 @@ def test_q5k1_one_mfma_nonfinite_scale(scale):
     ref = oracle.matmul("q5k1", raw, N, x)
     assert not np.isfinite(ref).all()
     assert_fp32_parity(got.reshape(M, N), ref, term_abs_sum("q5k1", raw, N, x), f"q5k1 {scale}")
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("N,M", [(64, 33), (301, 100)])
+def test_residual_add_with_and_without_splits(N, M, splits):
+    # in the GEMM's epilogue (one split) or in the reduction: the product of the plain
+    # call, then one float32 add
+    K = 768
+    w = sq.DeviceWeight.from_quant(sq.QuantWeight("q8", make_raw("q8", N, K, seed=3), K // 32, N, K))
+    x = torch.from_numpy(make_x(M, K, seed=4)).cuda()
+    base = np.random.default_rng(5).normal(size=(M, N)).astype(np.float32)
+    dst, plain = torch.from_numpy(base).cuda(), torch.empty(M, N, device="cuda")
+    sq.set_param("gemm_splits", splits)
+    try:
+        sq.matmul_add_dev(w, x.data_ptr(), M, K, dst.data_ptr())
+        sq.matmul_dev(w, x.data_ptr(), M, K, plain.data_ptr())
+    finally:
+        sq.set_param("gemm_splits", 0)
+    torch.cuda.synchronize()
+    assert np.array_equal(dst.cpu().numpy().view(np.uint32), (base + plain.cpu().numpy()).view(np.uint32))
