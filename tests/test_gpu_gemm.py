@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 import sllm_qmm as sq
