@@ -106,7 +106,9 @@ sllm_status sllm_weight_from_quant(const char *qtype, const void *raw, size_t ra
  *      native blocks and multiply fp32 activations by them, so only the order
  *      of the row sums differs (no int8 activation codes for these types);
  *      the prefill GEMM sums a 16-element sub-block's exact code products
- *      first and applies its scale and min to the sums.
+ *      first and applies its scale to the sums (Q2_K: products of the codes
+ *      from the one whose weight is nearest zero, whose own weight then
+ *      multiplies the sub-block's sum of activations).
  * Other types return SLLM_ERR_QTYPE (the reference's dense-fp32 branch).
  */
 sllm_status sllm_weight_from_gguf(uint32_t ggml_type, const void *raw, size_t raw_bytes,

@@ -13,10 +13,13 @@
 //   wants: 1 KB per (32 rows, 16 elements, part), lane l's 16 bytes at 16 l;
 // * v_mfma_f32_32x32x16_bf16 over the three parts forms every product exactly
 //   and sums a 16- or 32-element group in fp32;
-// * the epilogue adds scale * sum with one fused multiply-add. Q2_K's min term,
-//   -dmin m * (sum of the group's x), is a plain product over groups and goes
-//   through v_mfma_f32_32x32x2_f32 into the same accumulator (the group sums
-//   are formed in fp64 and rounded once).
+// * the epilogue adds scale * sum with one fused multiply-add.
+// * a Q2_K weight dl q - ml is taken as dl (q - b) + w_b, b the code whose weight w_b
+//   = dl b - ml is nearest zero (rounded once: the reference's float32): the two
+//   terms are never more than three times the weight, so where dl q and ml nearly
+//   cancel nothing is lost, and a weight of 0 gives 0. The second term, w_b * (sum
+//   of the group's x), goes through v_mfma_f32_32x32x2_f32 into the same accumulator
+//   (the group sums are formed in fp64 and rounded once).
 // Against the reference's per-element order this is reassociation and fewer
 // roundings; measured against 64 bits the error is no larger than the GEMV's
 // (gemm_kquant tests).
@@ -177,8 +180,9 @@ __device__ __forceinline__ uint32_t pack_bf(float a, float b) {
 // go in with codes and scale negated, so that the two halves' drifts cancel
 // (Q2_K over 4096 / 14336 columns 1.9e-7 / 2.9e-7 from the 64-bit result
 // without, Q5_0 1.24e-7 / 1.8e-7).
+// base: Q2_K's b (codes q - b).
 template <int FMT>
-__device__ __forceinline__ void decode_half(const WUnit<FMT> &u, int ks, uint32_t neg, uint4 (&p)[2]) {
+__device__ __forceinline__ void decode_half(const WUnit<FMT> &u, int ks, uint32_t neg, uint32_t base, uint4 (&p)[2]) {
     if constexpr (FMT == SLLM_Q5_0) {
         const uint32_t w[4] = {(uint32_t)u.qs.x, (uint32_t)u.qs.y, (uint32_t)u.qs.z, (uint32_t)u.qs.w};
 #pragma unroll
@@ -198,13 +202,12 @@ __device__ __forceinline__ void decode_half(const WUnit<FMT> &u, int ks, uint32_
             p[h] = make_uint4(o[0], o[1], o[2], o[3]);
         }
     } else {
-        // bf16 high and low bytes of the value of code 0..7 (Q3K: code + 4 *
-        // high bit - 4; Q2K: the code), looked up four at a time with v_perm
-        constexpr uint32_t lo0 = FMT == SLLM_Q3K ? 0x80004080u : 0x40008000u;  // codes 0..3
-        constexpr uint32_t lo1 = 0x40008000u;                                  // Q3K codes 4..7 (0, 1, 2, 3)
+        // bf16 high and low bytes of the values -4 .. 3 at index 0 .. 7 (Q3K: code + 4 *
+        // high bit; Q2K: code + 4 - b), looked up four at a time with v_perm
+        constexpr uint32_t lo0 = 0x80004080u, lo1 = 0x40008000u;
         const uint32_t sgn = neg * 0x01010101u;
-        const uint32_t hi0 = (FMT == SLLM_Q3K ? 0xBFC0C0C0u : 0x40403F00u) ^ sgn;
-        const uint32_t hi1 = 0x40403F00u ^ sgn;
+        const uint32_t hi0 = 0xBFC0C0C0u ^ sgn, hi1 = 0x40403F00u ^ sgn;
+        const uint32_t shift = FMT == SLLM_Q2K ? (4u - base) * 0x01010101u : 0u;
         const uint32_t w = ks ? u.q2.y : u.q2.x;
         uint32_t o[8];
 #pragma unroll
@@ -215,6 +218,8 @@ __device__ __forceinline__ void decode_half(const WUnit<FMT> &u, int ks, uint32_
                 t = (t & 0x0011u) | ((t & 0x1100u) << 8);          // bits 0, 4, 16, 20
                 t = (t & 0x00010001u) | ((t & 0x00100010u) << 4);  // bits 0, 8, 16, 24
                 sel |= t << 2;
+            } else {
+                sel += shift;
             }
             const uint32_t l = __builtin_amdgcn_perm(lo1, lo0, sel), hh = __builtin_amdgcn_perm(hi1, hi0, sel);
             o[2 * j] = __builtin_amdgcn_perm(hh, l, 0x05010400u);
@@ -238,6 +243,13 @@ __device__ __forceinline__ void unit_scale(const WUnit<FMT> &u, int i, float &sc
     } else {
         sc = f16_exact((uint16_t)(u.sb & 0xffffu)) * (float)(int)(int8_t)(((uint32_t)u.d >> (8 * i)) & 0xffu);
     }
+}
+
+// Q2_K: the code whose weight is nearest zero, ml / dl rounded to 0 .. 3 (at dl = 0
+// any: the codes do not matter).
+__device__ __forceinline__ uint32_t q2k_base(float sc, float mn) {
+    const float s = __builtin_fabsf(sc), t = sc < 0.0f ? -mn : mn;
+    return (t > 0.5f * s) + (t > 1.5f * s) + (t > 2.5f * s);
 }
 
 // One LDS stage: KB blocks of BN columns. b: [blk][column tile][ks][lane][16
@@ -384,17 +396,19 @@ bgemm_kernel(Planes P, const uint16_t *__restrict__ frag, const float *__restric
             const int c = e / KB, blk = e % KB;
             uint4 p[2];
             const uint32_t neg = blk & 1 ? 0x80u : 0u;  // odd blocks negated, codes and scale
-            decode_half<FMT>(u[i], ks, neg, p);
+            float sc, mn;
+            unit_scale<FMT>(u[i], ks, sc, mn);
+            const uint32_t base = FMT == SLLM_Q2K ? q2k_base(sc, mn) : 0u;
+            decode_half<FMT>(u[i], ks, neg, base, p);
             unsigned char *b = S.b + blk * St::BLK + (c >> 5) * 2048 + (c & 31) * 16 + ks * 1024;
             *(uint4 *)b = p[0];
             *(uint4 *)(b + 512) = p[1];
             if (kq_native(FMT) || ks == 0) {
-                float sc, mn;
-                unit_scale<FMT>(u[i], ks, sc, mn);
+                const float wb = __builtin_fmaf(sc, (float)base, -mn);
                 sc = __uint_as_float(__float_as_uint(sc) ^ neg << 24);
                 // blocks past the row's end repeat its last one with scale 0 (their activations are zeros)
                 S.sc[blk * St::NG + (kq_native(FMT) ? ks : 0)][c] = kq_native(FMT) || s * KB + blk < G ? sc : 0.0f;
-                if (FMT == SLLM_Q2K) S.mn[FMT == SLLM_Q2K ? blk * St::NG + ks : 0][c] = -mn;
+                if (FMT == SLLM_Q2K) S.mn[FMT == SLLM_Q2K ? blk * St::NG + ks : 0][c] = wb;
             }
         };
         // activation fragments of a block: [ks][part]
@@ -432,7 +446,7 @@ bgemm_kernel(Planes P, const uint16_t *__restrict__ frag, const float *__restric
                     }
                 }
                 if (FMT == SLLM_Q2K) {
-                    // - min * (group sum) of both sub-blocks: k slot = lane / 32
+                    // w_b * (group sum) of both sub-blocks: k slot = lane / 32
                     const float mn = S.mn[FMT == SLLM_Q2K ? blk * St::NG + (lane >> 5) : 0][c0 + 32 * j];
                     acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[r], mn, acc[j], 0, 0, 0);
                 }

@@ -128,3 +128,30 @@ def test_capture_without_workspace_takes_the_gemv(t):
         g.replay()
         torch.cuda.synchronize()
         assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+def test_q2k_weights_that_nearly_cancel():
+    # dl q and ml close together: rows of exact zeros give exact zeros, and the error
+    # is in |w| (dl (q - b) and w_b are within 3 |w|), not in |dl q| + |ml|
+    N, K, M = 96, 1024, 48
+    rng = np.random.default_rng(21)
+    raw = make_kq(10, N, K, 22).reshape(N, K // 256, 84)
+    code = (np.arange(N) % 3 + 1).astype(np.uint8)  # every code of a row
+    sc = rng.integers(1, 6, (N, K // 256, 16)).astype(np.uint8)
+    raw[..., :16] = sc | ((sc * code[:, None, None]) << 4)
+    raw[..., 16:80] = (code * 0x55)[:, None, None]
+    d = np.float16(2.0 ** -6)
+    dm = np.full(N, d)
+    dm[N // 2:] = np.float16(2.0 ** -6 * (1 + 2.0 ** -9))
+    raw[..., 80:82] = np.frombuffer(d.tobytes(), np.uint8)
+    raw[..., 82:84] = dm.view(np.uint8).reshape(N, 1, 2)
+    raw = raw.reshape(-1)
+    W = oracle.dense_weights(10, raw, N, K)
+    assert not W[:N // 2].any() and W[N // 2:].all()
+    w = sq.load_weight_f32_direct(10, raw, N, K)
+    x = make_x(M, K, seed=23)
+    got = gemm(w, x)
+    assert not got[:, :N // 2].any()
+    ref = oracle.matmul_dense(W, x).astype(np.float64)
+    bound = 3 * (K + K // 32 + 64) * U * (np.abs(x).astype(np.float64) @ np.abs(W).T.astype(np.float64))
+    assert np.all(np.abs(got - ref) <= bound)
