@@ -452,7 +452,8 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  call path)
  *   gemm_min_rows       >= 0       activation rows from which the GEMM is used (0: 8 for
  *                                  weights of 2^24 elements or more, 16 for smaller ones;
- *                                  Q5_0, Q2K and Q3K: 5 from 2^25 elements, else 8; the
+ *                                  Q5_0, Q2K and Q3K: 5 from 2^25 elements, 7 for most
+ *                                  above 2^22, else 9; the
  *                                  int8 formats 5 where the short-prompt GEMM takes them:
  *                                  up to 32 rows and 8192 columns (a multiple of 256;
  *                                  4096 for at most 2048 weight rows);
@@ -465,8 +466,8 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  loads in flight (0: 1, above 128 rows 5; for Q5K1 3,
  *                                  and 4 up to 32 rows; for Q5K1 in one MFMA per block,
  *                                  see sllm_weight_q5k1_one_mfma, 4 up to 32 rows, 2 up
- *                                  to 128, else 1); Q5_0, Q2K, Q3K: 256 columns of 1 =
- *                                  32, 2 = 64, 3 = 128 rows (0: by the rows). The shape
+ *                                  to 128, else 1); Q5_0, Q2K, Q3K: 1 = 32 x 256, 2 = 64 x
+ *                                  128, 3 = 128 x 256 (0: by rows and weight). The shape
  *                                  moves the fp32 summation splits
  *   gemm_splits         0..64      GEMM K splits, added in split order (0: by tile count;
  *                                  the split count moves the fp32 summation splits)

@@ -496,6 +496,20 @@ bool sgemm_route(const sllm_weight *w, int x_rows, const Route &r) {
     return r.ws && sgemm_supported(w->fmt, w->groups, x_rows, w->rows) && !tuning().gemm_shape && !tuning().gemm_splits;
 }
 
+// Rows from which the bf16 GEMM is faster than the GEMV's launches of up to four.
+// Measured (GEMV time / GEMM time, Q5_0, Q2_K, Q3_K): 14336x4096 at M = 4 1.01 / 1.50 /
+// 1.06, M = 5 1.30 / 1.74 / 1.43; 8192x4096 at M = 5 1.17 / 1.04 / 1.19; 4096x4096 at M = 6
+// 1.05 / 0.90 / 1.08, M = 7 1.29 / 1.11 / 1.32; 2560x2560 at M = 6 1.00 / 1.11 / 1.02, M = 7
+// 1.28 / 1.36 / 1.34; 1024x4096 at M = 7 1.32 / 1.16 / 1.31; 4096x1024 at M = 6 0.97 / 1.11 /
+// 0.97, M = 8 1.10 / 1.45 / 1.13; 2048x2048 at M = 8 0.89 / 1.03 / 0.84, M = 9 1.14 / 1.24 /
+// 1.06; 512x2048 at M = 8 0.82 / 0.94 / 0.85, M = 9 1.04 / 1.14 / 1.07; 1536x768 at M = 8 0.94 /
+// 1.07 / 0.90, M = 9 1.20 / 1.33 / 1.17.
+int bf16_min_rows(const sllm_weight *w) {
+    const int64_t n = (int64_t)w->rows * w->cols;
+    if (n >= ((int64_t)1 << 25)) return 5;
+    return w->cols >= 4096 || n >= ((int64_t)6 << 20) || (w->rows >= 4096 && n >= ((int64_t)1 << 22)) ? 7 : 9;
+}
+
 bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
     if (act_f32(w->fmt) && !r.ws) return false;
     // 0 (the default): the GEMM from 8 activation rows for weights of at least
@@ -504,14 +518,10 @@ bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
     // Measured (us, GEMV at M = 8 / GEMM at M = 8): Q4_1 14336x4096 36.0 /
     // 28.3, Q8_0 4096x14336 54.6 / 42.4, Q5K1 4096x4096 20.2 / 17.7; Q4_1
     // 1024x4096 at M = 8 13.7 / 20.1 and M = 16 27.2 / 19.1, Q4_0 8192x2048 at
-    // M = 16 30.5 / 17.9. The formats with fp32 activations go through the bf16
-    // GEMM from 5 rows for weights of at least 2^25 elements and from 8 for
-    // smaller ones. Measured (us, GEMV / GEMM): Q5_0 14336x4096 at M = 4 36.7 /
-    // 36.5, M = 5 48.5 / 37; Q3_K 4096x14336 at M = 5 71.6 / 43; Q5_0 4096x4096
-    // at M = 6 22.1 / 21, M = 8 28.6 / 22; Q2_K 4096x4096 at M = 6 20.6 / 25,
-    // M = 8 27.2 / 25; Q5_0 1536x768 at M = 8 11.2 / 11.5, M = 12 16.4 / 11.8.
+    // M = 16 30.5 / 17.9. The formats with fp32 activations have a line of
+    // their own (bf16_min_rows).
     int min_rows = tuning().gemm_min_rows;
-    if (min_rows == 0 && act_f32(w->fmt)) min_rows = (int64_t)w->rows * w->cols >= ((int64_t)1 << 25) ? 5 : 8;
+    if (min_rows == 0 && act_f32(w->fmt)) min_rows = bf16_min_rows(w);
     // The short-prompt GEMM from 5 rows, where the GEMV takes a second launch
     // (GEMV / GEMM: Q4_1 14336x4096 at M = 4 17.6 / 21.4, M = 5 25.0 / 20.9, Q8_0
     // 1536x768 5.5 / 8.0 and 8.0 / 8.1, Q5K1 4096x4096 9.9 / 14.9 and 15.1 / 14.9).

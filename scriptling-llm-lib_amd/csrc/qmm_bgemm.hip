@@ -307,11 +307,11 @@ constexpr int run_of(int fmt, int ct) { return fmt == SLLM_Q5_0 ? (ct == 4 ? 0 :
 // of KB blocks. RA: blocks of activation fragments held in registers (RA - 1
 // of them in flight); WA: stages of weights in flight. Gp: G rounded up to a
 // multiple of 4, the blocks the fragments are laid out for (zeros past G).
-template <int FMT, int WM, int WN, int CT, int KB, int RA, int WA>
+template <int FMT, int WM, int WN, int CT, int KB, int RA, int WA, bool ADD>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)))
 bgemm_kernel(Planes P, const uint16_t *__restrict__ frag, const float *__restrict__ xsum,
              const uint8_t *__restrict__ flag, const float *__restrict__ x, float *__restrict__ out, int M, int N,
-             int G, int mtiles, int ntiles, int splits, int sps, int add) {
+             int G, int mtiles, int ntiles, int splits, int sps) {
     constexpr int BN = 32 * CT * WN, T = 64 * WM * WN;
     constexpr int UNITS = BN * KB, PER = UNITS / T;
     constexpr int HPB = PER * 2 / KB;  // half units decoded beside each block
@@ -497,49 +497,64 @@ bgemm_kernel(Planes P, const uint16_t *__restrict__ frag, const float *__restric
             if (m < M && n < N) {
                 float &d = o[(size_t)m * N + n];
                 const float r = RUN ? tot[RUN ? j : 0][v] : acc[j][v];
-                d = add ? d + r : r;  // add: the residual add, one float32 add
+                d = ADD ? d + r : r;  // ADD: the residual add, one float32 add
             }
         }
     }
 }
 
-// Workgroup shapes: rows 32 WM, 256 columns.
+// Workgroup shapes, rows x columns: 32 x 256, 64 x 128 (both four waves, two workgroups
+// per CU), 128 x 256 (eight waves).
 enum BShape { kRows32 = 0, kRows64 = 1, kRows128 = 2 };
 
 struct BPlan {
-    int shape, wm, kb, mtiles, ntiles, splits, sps;
+    int shape, wm, bn, kb, mtiles, ntiles, splits, sps;
 };
 
-constexpr int kBn = 256;
 // Blocks per stage of the 128-row shape
 constexpr int kKb128(int fmt) { return fmt == SLLM_Q5_0 ? 4 : 2; }
 
 BPlan plan(int fmt, int M, int N, int G) {
     BPlan p{};
     const int RT = (M + 31) / 32;
-    // 128-row tiles decode each weight half as often as 64-row ones; those
-    // where the last tile would be less than three quarters full
-    p.shape = RT == 1 ? kRows32 : (RT == 2 || (RT + 3) / 4 * 4 * 4 > RT * 5 ? kRows64 : kRows128);
+    const int64_t w = (int64_t)N * G * 32;
+    // 32 x 256 up to 32 rows of a weight of 2^25 elements; 128 x 256 above 64 rows of
+    // 1.5e9 products (the k-quants: 3e9, and a last row tile at least three quarters
+    // full or the only one); else 64 x 128, whose many small workgroups fill the device
+    // from a small weight. Best time over the K splits (us, 32 x 256 / 64 x 128 / 128 x
+    // 256): Q5_0 1024x4096 at M = 32 17.9 / 16.1, M = 100 - / 21.1 / 26.5; 4096x4096 M =
+    // 32 23.9 / 22.0, M = 100 - / 31.4 / 29.5; 14336x4096 M = 32 38.3 / 41.8, M = 96 - /
+    // 70.5 / 57.4, M = 512 - / 254 / 171; Q3_K 4096x4096 M = 128 - / 35.5 / 35.4, 8192x4096
+    // M = 160 - / 69.7 / 72.9, M = 256 - / 85.9 / 76.0. (64 x 256, one workgroup per CU:
+    // Q5_0 1024x4096 at M = 64 20.5 against 18.8, 14336x4096 47.2 against 44.8.)
+    const bool kq = kq_native(fmt);
+    const bool wide = RT > 2 && w * M >= (kq ? (int64_t)3000000000 : 1500000000) &&
+                      (!kq || RT <= 4 || (RT + 3) / 4 * 80 <= RT * 23);
+    p.shape = RT == 1 && w >= ((int64_t)1 << 25) ? kRows32 : (wide ? kRows128 : kRows64);
     if (tuning().gemm_shape >= 1 && tuning().gemm_shape <= 3) p.shape = tuning().gemm_shape - 1;
     p.wm = p.shape == kRows32 ? 1 : (p.shape == kRows64 ? 2 : 4);
+    p.bn = p.shape == kRows64 ? 128 : 256;
     p.kb = p.shape == kRows128 ? kKb128(fmt) : 2;
     p.mtiles = (RT + p.wm - 1) / p.wm;
-    p.ntiles = (N + kBn - 1) / kBn;
+    p.ntiles = (N + p.bn - 1) / p.bn;
     const int nst = ((G + 3) & ~3) / p.kb;
-    // K splits: the count that minimises rounds of workgroups x stages each,
-    // plus the partials' write and read
-    const int slots = 256 * (p.shape == kRows32 ? 2 : 1);
-    const double stage = p.kb * (p.shape == kRows128 ? 0.9 : 0.45);  // us per stage of one workgroup
+    // K splits: the count of least cost, in blocks of K that a workgroup alone on its CU
+    // takes the time of: its blocks, times co for each workgroup where the CU has
+    // several, and a fixed part for each; then the reduction's megabytes. Fitted to 477
+    // (format, weight, rows), every split count timed: shape and count together are 1.2 %
+    // above the best on average.
+    static constexpr struct { double co, fix, mb; } kCost[4] = {{0.7, 0.5, 1}, {0.65, 2, 1}, {1, 8, 0.1}, {0.7, 8, 0.1}};
+    const auto &c = kCost[kq && p.shape == kRows32 ? 3 : p.shape];
     int best = 1;
     double bc = 1e30;
     for (int S = 1; S <= 32 && S <= nst; S++) {
         const int sps = (nst + S - 1) / S;
         if ((nst + sps - 1) / sps != S) continue;
-        const int64_t rounds = ((int64_t)p.mtiles * p.ntiles * S + slots - 1) / slots;
-        double c = rounds * (sps * stage + 2.0);
-        if (S > 1) c += 3.0 + 2.0 * S * M * (double)N * 4 / 4.0e6;
-        if (c < bc) {
-            bc = c;
+        const int64_t n = ((int64_t)p.mtiles * p.ntiles * S + 255) / 256;
+        double t = sps * p.kb * (n == 1 ? 1.0 : c.co * n) + c.fix * n;
+        if (S > 1) t += c.mb * S * M * (double)N * 4e-6;
+        if (t < bc) {
+            bc = t;
             best = S;
         }
     }
@@ -571,9 +586,9 @@ sllm_status launch_shape(const Planes &P, const uint16_t *frag, const float *xsu
     const int total = p.mtiles * p.ntiles * p.splits;
     constexpr size_t lds = 2 * sizeof(BStage<FMT, KB, 32 * CT * WN>);
     static_assert(lds <= 160 * 1024, "LDS");
-    static_assert(32 * CT * WN == kBn, "columns per workgroup");
-    hipLaunchKernelGGL((bgemm_kernel<FMT, WM, WN, CT, KB, RA, WA>), dim3((total + 7) / 8 * 8), dim3(64 * WM * WN), lds, s, P,
-                       frag, xsum, flag, x, out, M, N, G, p.mtiles, p.ntiles, p.splits, p.sps, add);
+    const auto kernel = add ? bgemm_kernel<FMT, WM, WN, CT, KB, RA, WA, true> : bgemm_kernel<FMT, WM, WN, CT, KB, RA, WA, false>;
+    hipLaunchKernelGGL(kernel, dim3((total + 7) / 8 * 8), dim3(64 * WM * WN), lds, s, P, frag, xsum, flag, x, out, M, N, G,
+                       p.mtiles, p.ntiles, p.splits, p.sps);
     SLLM_HIP(hipGetLastError());
     return SLLM_OK;
 }
@@ -594,7 +609,7 @@ sllm_status launch_fmt(const Planes &P, const float *x, float *dst, int M, int N
     SLLM_HIP(hipGetLastError());
     switch (p.shape) {
     case kRows32: return launch_shape<FMT, 1, 4, 2, 2, 2, 2>(P, frag, xsum, flag, x, out, M, N, G, p, ea, s);
-    case kRows64: return launch_shape<FMT, 2, 4, 2, 2, 4, 2>(P, frag, xsum, flag, x, out, M, N, G, p, ea, s);
+    case kRows64: return launch_shape<FMT, 2, 2, 2, 2, 4, 2>(P, frag, xsum, flag, x, out, M, N, G, p, ea, s);
     default: return launch_shape<FMT, 4, 2, 4, kKb128(FMT), 2, 2>(P, frag, xsum, flag, x, out, M, N, G, p, ea, s);
     }
 }

@@ -155,3 +155,17 @@ def test_q2k_weights_that_nearly_cancel():
     ref = oracle.matmul_dense(W, x).astype(np.float64)
     bound = 3 * (K + K // 32 + 64) * U * (np.abs(x).astype(np.float64) @ np.abs(W).T.astype(np.float64))
     assert np.all(np.abs(got - ref) <= bound)
+
+
+@pytest.mark.parametrize("t", [10, 11])
+@pytest.mark.parametrize("N,K,M,gemm_from", [(512, 2048, 8, 9), (512, 2048, 9, 9), (64, 4096, 6, 7), (64, 4096, 7, 7),
+                                             (4096, 1024, 6, 7), (4096, 1024, 7, 7)])
+def test_the_line_between_gemv_and_gemm(t, N, K, M, gemm_from):
+    w = sq.load_weight_f32_direct(t, make_kq(t, N, K, 41), N, K)
+    x = make_x(M, K, seed=42)
+    forced = gemm(w, x)
+    sq.set_param("gemm_min_rows", 1 << 20)
+    gemv = gemm(w, x)
+    sq.set_param("gemm_min_rows", 0)
+    assert not np.array_equal(gemv, forced)  # two orders
+    assert np.array_equal(gemm(w, x), forced if M >= gemm_from else gemv)
