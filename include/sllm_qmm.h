@@ -454,9 +454,10 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  weights of 2^24 elements or more, 16 for smaller ones;
  *                                  Q5_0, Q2K and Q3K: 5 from 2^25 elements, 7 for most
  *                                  above 2^22, else 9; the
- *                                  int8 formats 5 where the short-prompt GEMM takes them:
- *                                  up to 32 rows and 8192 columns (a multiple of 256;
- *                                  4096 for at most 2048 weight rows);
+ *                                  int8 formats where the short-prompt GEMM takes them (up
+ *                                  to 32 rows and 8192 columns, a multiple of 256; 4096
+ *                                  for at most 4096 weight rows): 5 above 4096 weight
+ *                                  rows, else 6 at 4096 columns, else 7;
  *                                  the GEMM and GEMV sum a row's blocks in different
  *                                  orders, so a row's last bits can change with it)
  *   gemm_shape          0..5       GEMM workgroups: 1 = 64 x 128 tiles, 2 = 64 x 64 tiles with

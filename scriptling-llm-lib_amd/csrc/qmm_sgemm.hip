@@ -7,7 +7,7 @@
 // weights through LDS with a barrier per 128 columns of K and needed a quantize
 // pass per weight, a split reduction per weight and an elementwise pass after.
 // Here
-// * sact_kernel norms (optionally) and quantizes the rows once per input, with
+// * sact_kernel (sact_norm_kernel: normed) quantizes the rows once per input, with
 //   the GEMV prologue's routines, into MFMA lane order;
 // * a wave streams 32 weight rows over its share of K, eight blocks (one 128-byte
 //   line of a row's codes) at a time: eight lanes load a row's line, a wave-private
@@ -94,11 +94,36 @@ __device__ __forceinline__ float row_inv(const float *xr, int K, float eps, floa
     return 1.0f / (float)sqrt(q + (double)eps);
 }
 
-// One workgroup of 256 threads per row (grid: 32); eight lanes per
-// block. The first four blocks of a lane's group are loaded before the row's
-// statistics are waited for (one memory round trip up to K = 4096).
-__global__ void __launch_bounds__(256) sact_kernel(const float *__restrict__ x, const float *__restrict__ nw,
-                                                   float eps, int M, int G, SAct a) {
+// Eight lanes quantize a block. Rows past M (of 32) are zeros.
+// A block's part u of row r: quantized into place.
+__device__ __forceinline__ void put_part(const SAct &a, int r, int g, int sub, const float4 &u) {
+    int q[1];
+    float s;
+    int sm;
+    quantize_part<8>(&u, q, s, sm);
+    const size_t t = (size_t)g;
+    // word sub of the block: lane half sub / 4, word sub % 4 of its 16 bytes
+    ((int *)(a.xq + t * 1024 + (r + 32 * (sub >> 2)) * 16))[sub & 3] = q[0];
+    if (sub == 0) {
+        a.xs[t * 32 + r] = s;
+        a.xm[t * 32 + r] = (float)sm * s;
+        a.sx[t * 32 + r] = sm;
+    }
+}
+
+// Without the norm: grid (32 rows, 32 blocks each). (One workgroup per row, its parts in
+// turn: every call 0.8-1 us longer, Q4_1 4096x4096 at M = 16 13.8 against 12.8.)
+__global__ void __launch_bounds__(256) sact_kernel(const float *__restrict__ x, int M, int G, SAct a) {
+    const int r = blockIdx.x, sub = threadIdx.x & 7, g = blockIdx.y * 32 + (threadIdx.x >> 3);
+    if (g >= G) return;  // eight lanes alike
+    put_part(a, r, g, sub, r < M ? ((const float4 *)x)[((size_t)r * G + g) * 8 + sub] : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+}
+
+// RMSNormed rows: one workgroup per row. The first four blocks of a lane's group are
+// loaded before the row's statistics are waited for (one memory round trip up to K =
+// 4096).
+__global__ void __launch_bounds__(256) sact_norm_kernel(const float *__restrict__ x, const float *__restrict__ nw,
+                                                        float eps, int M, int G, SAct a) {
     __shared__ float red[4];
     const int r = blockIdx.x;
     const bool live = r < M;
@@ -109,33 +134,18 @@ __global__ void __launch_bounds__(256) sact_kernel(const float *__restrict__ x, 
     for (int i = 0; i < 4; i++) {
         const int g = min(b0 + 32 * i, G - 1);
         v[i] = ((const float4 *)(xr + (size_t)g * 32))[sub];
-        if (nw) w[i] = ((const float4 *)(nw + (size_t)g * 32))[sub];
+        w[i] = ((const float4 *)(nw + (size_t)g * 32))[sub];
     }
-    const float inv = nw ? row_inv(xr, G * 32, eps, red) : 0.0f;
-    auto put = [&](int g, float4 u, const float4 &c) {
-        if (nw) u = make_float4((u.x * inv) * c.x, (u.y * inv) * c.y, (u.z * inv) * c.z, (u.w * inv) * c.w);
-        if (!live) u = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        int q[1];
-        float s;
-        int sm;
-        quantize_part<8>(&u, q, s, sm);
-        const size_t t = (size_t)g;
-        // word sub of the block: lane half sub / 4, word sub % 4 of its 16 bytes
-        ((int *)(a.xq + t * 1024 + (r + 32 * (sub >> 2)) * 16))[sub & 3] = q[0];
-        if (sub == 0) {
-            a.xs[t * 32 + r] = s;
-            a.xm[t * 32 + r] = (float)sm * s;
-            a.sx[t * 32 + r] = sm;
-        }
+    const float inv = row_inv(xr, G * 32, eps, red);
+    auto put = [&](int g, const float4 &u, const float4 &c) {
+        put_part(a, r, g, sub, live ? make_float4((u.x * inv) * c.x, (u.y * inv) * c.y, (u.z * inv) * c.z, (u.w * inv) * c.w)
+                                    : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     };
 #pragma unroll
     for (int i = 0; i < 4; i++)
         if (b0 + 32 * i < G) put(b0 + 32 * i, v[i], w[i]);
-    for (int g = b0 + 128; g < G; g += 32) {
-        const float4 u = ((const float4 *)(xr + (size_t)g * 32))[sub];
-        const float4 c = nw ? ((const float4 *)(nw + (size_t)g * 32))[sub] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        put(g, u, c);
-    }
+    for (int g = b0 + 128; g < G; g += 32)
+        put(g, ((const float4 *)(xr + (size_t)g * 32))[sub], ((const float4 *)(nw + (size_t)g * 32))[sub]);
 }
 
 // The weights of one launch: segment s owns the column tiles [tile0[s], tile0[s +
@@ -521,16 +531,18 @@ sllm_status launch_f(const SegG &S, const SAct &A, int M, int G, hipStream_t s) 
 
 }  // namespace
 
-// Up to 32 rows and 8192 columns (4096 where the weight is narrow), whatever else the
-// call holds: a weight's bits do not depend on its company. Measured (us, with the quantize pass; this / the
-// tiled GEMM, M = 16 and 32): Q4_1 14336x4096 20.6 / 27.6 and 20.9 / 28.6, Q8_0
-// 4096x4096 13.6 / 16.0 and 13.7 / 18.4, Q5K1 4096x4096 14.8 / 14.6 and 14.8 /
-// 16.3, Q4_0 8192x2048 10.4 / 12.7 and 10.5 / 13.6, Q8_0 1536x768 8.2 / 11.4 and
-// 8.6 / 11.8, narrow Q5K1 1024x4096 11.2 / 11.1 and 11.7 / 11.8; but Q4_0 512x8192
-// 13.7 / 12.4 and 14.1 / 13.0, Q8_0 4096x14336 37.2 / 26.2 (a wave's seven chunks of K in
-// turn), and with two row tiles (33 to 64 rows) Q4_1 14336x4096 39.4 / 28.8.
+// Up to 32 rows, and 8192 columns above 4096 weight rows, else 4096 (fewer tiles than
+// waves' chunks of K in turn), whatever else the call holds: a weight's bits do not
+// depend on its company. Measured (us, with the quantize pass; this / the tiled GEMM, M =
+// 16 and 32): Q4_1 14336x4096 21.5 / 29.6 (M = 16), 4096x4096 12.8 / 15.9 and 13.0 / 18.9,
+// 1024x4096 10.1 / 11.7 and 10.6 / 12.5, 4608x8192 19.5 / 27.3 and 20.0 / 29.3, 1536x768 7.6 /
+// 12.1 (M = 16); Q5K1 4096x4096 14.1 / 15.1 and 14.3 / 16.9, 1024x4096 10.4 / 11.3 and 10.8 /
+// 12.2; but (before the quantize pass lost 0.8 us) Q5K1 4096x8192 24.2 / 20.0 and 24.5 /
+// 21.6, 2304x4608 17.4 / 14.5 and 17.5 / 15.9, Q4_1 4096x8192 22.1 / 21.5, Q8_0 4096x14336
+// 37.2 / 26.2 (a wave's seven chunks of K in turn), and with two row tiles (33 to 64 rows)
+// Q4_1 14336x4096 39.4 / 28.8.
 bool sgemm_supported(int fmt, int G, int M, int64_t rows) {
-    return !act_f32(fmt) && G % kCh == 0 && M <= 32 && G <= (rows <= 2048 ? 128 : 256);
+    return !act_f32(fmt) && G % kCh == 0 && M <= 32 && G <= (rows <= 4096 ? 128 : 256);
 }
 
 // The codes, and the partial sums of a weight of so many rows that is launched by
@@ -541,7 +553,9 @@ size_t sgemm_ws_bytes(int G, int M, int64_t rows) {
 }
 
 sllm_status launch_sact(const float *x, const float *norm_w, float eps, int M, int G, void *act, hipStream_t s) {
-    hipLaunchKernelGGL(sact_kernel, dim3(32), dim3(256), 0, s, x, norm_w, eps, M, G, carve_sact(act, G));
+    const SAct a = carve_sact(act, G);
+    if (norm_w) hipLaunchKernelGGL(sact_norm_kernel, dim3(32), dim3(256), 0, s, x, norm_w, eps, M, G, a);
+    else hipLaunchKernelGGL(sact_kernel, dim3(32, (G + 31) / 32), dim3(256), 0, s, x, M, G, a);
     SLLM_HIP(hipGetLastError());
     return SLLM_OK;
 }

@@ -141,3 +141,75 @@ def test_wide_launches_equal_the_narrow_ones(qtype, K):
     torch.cuda.synchronize()
     for o in (g, u):
         assert np.array_equal(o.cpu().numpy().view(np.uint32), full.view(np.uint32))
+
+
+@pytest.mark.parametrize("qtype", ["q4_1", "q5k1"])
+@pytest.mark.parametrize("N,K,M,gemm", [
+    (4097, 256, 4, False), (4097, 256, 5, True), (4096, 256, 6, False), (4096, 256, 7, True), (40, 4096, 5, False),
+    (40, 4096, 6, True), (40, 3840, 6, False), (40, 3840, 7, True), (40, 4352, 7, False), (4097, 4352, 5, True)])
+def test_the_line_between_gemv_and_short_prompt_gemm(qtype, N, K, M, gemm):
+    _, w = weight(qtype, N, K, 13)
+    x = make_x(M, K, seed=14)
+    sq.set_param("gemm_min_rows", 1 << 20)
+    gemv = run(w, x)
+    sq.set_param("gemm_min_rows", 0)
+    assert np.array_equal(run(w, x).view(np.uint32), gemv.view(np.uint32)) is not gemm
+
+
+def _power_of_two_weight(qtype, N, K, rng):
+    """Blocks whose scales are powers of two and mins small multiples of them, and
+    the weights they stand for."""
+    G = K // 32
+    d = 2.0 ** rng.integers(-4, 1, (N, G))
+    f16 = lambda v: v.astype(np.float16).view(np.uint8).reshape(N, G, 2)
+    if qtype == "q8":
+        q = rng.integers(-127, 128, (N, G, 32)).astype(np.int8)
+        return np.concatenate([f16(d), q.view(np.uint8)], -1), (d[..., None] * q)
+    q = rng.integers(0, 16, (N, G, 32)).astype(np.uint8)
+    packed = q[..., :16] | (q[..., 16:] << 4)
+    if qtype == "q4":
+        return np.concatenate([f16(d), packed], -1), d[..., None] * (q.astype(np.int64) - 8)
+    m = d * rng.integers(-8, 9, (N, G))
+    lo = np.concatenate([f16(d), f16(m), packed], -1)
+    w = d[..., None] * q + m[..., None]
+    if qtype == "q4_1":
+        return lo, w
+    hb = rng.integers(0, 2, (N, G, 32)).astype(np.uint8)
+    hi = np.concatenate([f16(16 * d), f16(0 * d), hb[..., :16] | (hb[..., 16:] << 4)], -1)
+    return np.concatenate([lo.reshape(-1), hi.reshape(-1)]), w + 16 * d[..., None] * hb
+
+
+@pytest.mark.parametrize("qtype", QTYPES)
+@pytest.mark.parametrize("N,K,M", [(70, 512, 32), (33, 4096, 5), (4100, 768, 9)])
+def test_exact_sums_equal_the_integer_result(qtype, N, K, M):
+    # rows whose largest magnitude is 127 * 2^e quantize exactly (scale 2^e), block
+    # scales are powers of two: every dot, term and sum fits 24 bits, so the outputs
+    # pin the integer dots bit for bit
+    rng = np.random.default_rng(N + K)
+    raw, W = _power_of_two_weight(qtype, N, K, rng)
+    w = sq.DeviceWeight.from_quant(sq.QuantWeight(qtype, np.ascontiguousarray(raw).reshape(-1), K // 32, N, K))
+    x = np.zeros((M, K // 32, 32), np.float32)
+    for i in range(M):  # a few blocks of each row hold values: sums stay small
+        at = rng.choice(K // 32, 4, replace=False)
+        v = rng.integers(-2, 3, (4, 32)).astype(np.float32)
+        v[:, rng.integers(0, 32)] = 127
+        x[i, at] = v * 2.0 ** (i % 3)
+    x = x.reshape(M, K)
+    want = x.astype(np.float64) @ W.reshape(N, K).T
+    assert np.array_equal(run(w, x), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("M,K", [(5, 1024), (32, 1024), (9, 2304), (32, 4096)])
+@pytest.mark.parametrize("qtype", QTYPES)
+def test_normed_gate_up_pair_equals_norm_then_pair(qtype, M, K):
+    _, a = weight(qtype, 97, K, 15)
+    _, b = weight(qtype, 97, K, 16)
+    x = make_x(M, K, seed=17)
+    nw = np.random.default_rng(18).normal(1, 0.2, K).astype(np.float32)
+    normed = np.stack([oracle.rmsnorm(x[i:i + 1], nw, 1e-5, lib_order=True)[0] for i in range(M)])
+    xd, nd, wd = (torch.from_numpy(v).cuda() for v in (x, normed, nw))
+    h, want = (torch.full((M, 97), float("nan"), device="cuda") for _ in range(2))
+    sq.rmsnorm_matmul_swiglu_dev(a, b, xd.data_ptr(), wd.data_ptr(), 1e-5, M, K, h.data_ptr())
+    sq.matmul_swiglu_dev(a, b, nd.data_ptr(), M, K, want.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.isfinite(want).all() and torch.equal(h.view(torch.int32), want.view(torch.int32))
