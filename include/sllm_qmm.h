@@ -62,9 +62,15 @@ const char *sllm_last_error(void);
  * the prefill GEMM's activation codes and split partials, the attention's
  * q rows and split states and multi-row normed rows in a buffer owned by
  * (device, stream), grown on demand. Growth allocates, so it cannot happen
- * while the stream is being captured into a HIP graph (the call returns
- * SLLM_ERR_ARG, naming the size it needed): reserve at least that many bytes
- * with this call before capturing. A buffer that is outgrown is kept, not
+ * while the stream is being captured into a HIP graph: reserve at least that
+ * many bytes with this call before capturing. Without, a captured call whose
+ * workspace is too small returns SLLM_ERR_ARG, naming the size it needed, or,
+ * where a kernel that needs less can do its work, records that one: the split
+ * attention for prompts, the GEMV for Q2_K and Q3_K weights, the GEMV or the
+ * tiled GEMM for rows of the short-prompt GEMM, the GEMV for Q5_0 rows below
+ * the tiled GEMM's (sums in another order, so other last bits than an eager
+ * call's; decided for each weight by itself, so a call of several weights still
+ * gives the single calls' bits). A buffer that is outgrown is kept, not
  * freed, until the process ends, so graphs captured before a growth stay
  * valid. Growth at least doubles the buffer.
  */
@@ -241,8 +247,8 @@ sllm_status sllm_matmul_swiglu_dev(const sllm_weight *w_gate, const sllm_weight 
  * the normed rows (forwardBlock: model_f32.go:388-396 and 476-490;
  * outputLogits: model_f32.go:502-527). For one row (decode) the GEMV launch
  * computes the row statistic itself, so no normed vector goes through memory;
- * several rows are normed into the workspace first by a standalone kernel
- * with the same statistics. inv = 1 / float32(sqrt(
+ * several rows are normed as they are quantized where every weight takes an
+ * int8 GEMM, else into the workspace first, with the same statistics. inv = 1 / float32(sqrt(
  * float64(ss) / cols + float64(eps))) and normed = (x * inv) * w as in the
  * reference; the sum of squares ss is added in a fixed order of the library's
  * (256 strided partial sums, then a fixed tree) rather than the reference's

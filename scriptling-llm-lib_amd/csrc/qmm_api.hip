@@ -146,6 +146,7 @@ sllm_status workspace(hipStream_t stream, size_t need, void **out, size_t *cap, 
         if (capturing(stream)) {
             if (stuck) {
                 *stuck = true;
+                *cap = w.cap;
                 return SLLM_OK;
             }
             return set_error(SLLM_ERR_ARG, "the stream's workspace must grow to " + std::to_string(need) +
@@ -482,18 +483,27 @@ sllm_status with_upload(const void *host, size_t bytes, size_t extra, F fn) {
     return st;
 }
 
-// How the matmuls of one call may run. ws: the bf16 GEMM of the fp32-activation
-// formats and the short-prompt GEMM may; false on a stream under capture whose
-// workspace cannot hold what they need (those calls take the GEMV, which needs
-// none, or the tiled GEMM).
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// How the matmuls of one call may run. room: the bytes of workspace that a weight's GEMM
+// may take: any number, except on a stream under capture, whose workspace cannot grow.
+// A weight whose GEMM does not fit there takes what it took before that GEMM existed:
+// the short-prompt GEMM's weights the tiled GEMM or, below its rows, the GEMV; Q2_K and
+// Q3_K the GEMV; Q5_0 the GEMV below the tiled GEMM's rows. Decided for each weight by
+// itself, so that it gives the same bits alone and beside others.
 struct Route {
-    bool ws = true;
+    size_t room = SIZE_MAX;
 };
+// Takes b bytes of the room for something else.
+void take(Route &r, size_t b) {
+    if (r.room != SIZE_MAX) r.room = r.room > b ? r.room - b : 0;
+}
 
 // The short-prompt GEMM takes a weight's rows (an explicit tile shape or K split
 // asks for the tiled GEMM).
 bool sgemm_route(const sllm_weight *w, int x_rows, const Route &r) {
-    return r.ws && sgemm_supported(w->fmt, w->groups, x_rows, w->rows) && !tuning().gemm_shape && !tuning().gemm_splits;
+    return sgemm_supported(w->fmt, w->groups, x_rows, w->rows) && !tuning().gemm_shape && !tuning().gemm_splits &&
+           (r.room == SIZE_MAX || align256(sgemm_ws_bytes(w->groups, x_rows, w->rows)) <= r.room);
 }
 
 // Rows from which the bf16 GEMM is faster than the GEMV's launches of up to four.
@@ -511,7 +521,6 @@ int bf16_min_rows(const sllm_weight *w) {
 }
 
 bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
-    if (act_f32(w->fmt) && !r.ws) return false;
     // 0 (the default): the GEMM from 8 activation rows for weights of at least
     // 2^24 elements, from 16 for smaller ones. The GEMV takes up to 4 rows per
     // launch and streams the weight once per launch; the GEMM streams it once.
@@ -521,7 +530,13 @@ bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
     // M = 16 30.5 / 17.9. The formats with fp32 activations have a line of
     // their own (bf16_min_rows).
     int min_rows = tuning().gemm_min_rows;
-    if (min_rows == 0 && act_f32(w->fmt)) min_rows = bf16_min_rows(w);
+    const int tiled_rows = min_rows ? min_rows : (int64_t)w->rows * w->cols >= ((int64_t)1 << 24) ? 8 : 16;
+    if (act_f32(w->fmt)) {
+        if (kq_native(w->fmt) && !w->kq_gemm) return false;
+        if (x_rows < (min_rows ? min_rows : bf16_min_rows(w))) return false;
+        return r.room == SIZE_MAX || align256(gemm_workspace_bytes(w->fmt, w->rows, w->groups, x_rows)) <= r.room ||
+               (!kq_native(w->fmt) && x_rows >= tiled_rows);
+    }
     // The short-prompt GEMM from 5 rows, where the GEMV takes a second launch, for
     // weights of more than 4096 rows; from 6 for fewer of 4096 columns; from 7, where the
     // GEMV's second launch has three rows, for the rest. The line is the weight's own, so
@@ -532,8 +547,7 @@ bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
     // (Three weights in one launch, q / k / v of Q4_1 4096 + 2 x 1024 rows, would gain from 5
     // rows: 20.8 / 15.4.)
     if (min_rows == 0 && sgemm_route(w, x_rows, r)) min_rows = w->rows > 4096 ? 5 : w->cols >= 4096 ? 6 : 7;
-    if (min_rows == 0) min_rows = (int64_t)w->rows * w->cols >= ((int64_t)1 << 24) ? 8 : 16;
-    if (kq_native(w->fmt) && !w->kq_gemm) return false;
+    if (min_rows == 0) min_rows = tiled_rows;
     return x_rows >= min_rows && gemm_supported(w->fmt, w->groups);
 }
 
@@ -573,10 +587,8 @@ sllm_status run_matmul(const sllm_weight *w, const float *x, int x_rows, float *
     return launch_gemm(gemm_fmt(w), P, x, dst, w->rows, w->groups, x_rows, ws, cap, false, false, s);
 }
 
-size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
-
-// The workspace of a call that needs need() bytes, written to *bytes; r.ws is
-// cleared where the stream is being captured and its workspace is too small.
+// The workspace of a call that needs need() bytes, written to *bytes; on a stream under
+// capture whose workspace is smaller r.room is set first, and need() asked again.
 template <class F>
 sllm_status fit_workspace(hipStream_t s, Route &r, F need, void **ws, size_t *bytes) {
     size_t cap = 0;
@@ -585,7 +597,7 @@ sllm_status fit_workspace(hipStream_t s, Route &r, F need, void **ws, size_t *by
     bool stuck = false;
     const sllm_status st = workspace(s, *bytes, ws, &cap, &stuck);
     if (!stuck) return st;
-    r.ws = false;
+    r.room = cap;
     if ((*bytes = need()) == 0) return SLLM_OK;
     return workspace(s, *bytes, ws, &cap);
 }
@@ -669,18 +681,22 @@ bool swiglu_paired(const sllm_weight *wg, const sllm_weight *wu, int x_rows, con
     return !uses_gemm(wg, x_rows, r) && !uses_gemm(wu, x_rows, r) && gemv_fmt(wg) == gemv_fmt(wu);
 }
 
-// Workspace the unpaired SwiGLU path needs: the GEMM workspace, then gate / up
-// buffers the caller did not provide.
 bool swiglu_sgemm(const sllm_weight *wg, const sllm_weight *wu, int x_rows, const Route &r) {
     return uses_sgemm(wg, x_rows, r) && uses_sgemm(wu, x_rows, r) && gemm_fmt(wg) == gemm_fmt(wu);
 }
+// Workspace the SwiGLU needs: none for the paired GEMV, the short-prompt GEMM's, or the
+// two GEMMs' and the gate / up buffers the caller did not provide (which are taken of
+// the room first).
 size_t swiglu_ws_bytes(const sllm_weight *wg, const sllm_weight *wu, int x_rows, const float *gate,
-                       const float *up, const Route &r) {
+                       const float *up, Route &r) {
     if (swiglu_paired(wg, wu, x_rows, r)) return 0;
-    if (swiglu_sgemm(wg, wu, x_rows, r)) return sgemm_ws_bytes(wg->groups, x_rows, wg->rows);
+    if (swiglu_sgemm(wg, wu, x_rows, r)) return align256(sgemm_ws_bytes(wg->groups, x_rows, wg->rows));
     const sllm_weight *pair[2] = {wg, wu};
     const size_t mm = align256((size_t)x_rows * wg->rows * sizeof(float));
-    return multi_gemm_ws(pair, 2, x_rows, r) + (gate ? 0 : mm) + (up ? 0 : mm);
+    const size_t bufs = (gate ? 0 : mm) + (up ? 0 : mm);
+    take(r, bufs);
+    if (swiglu_paired(wg, wu, x_rows, r)) return 0;
+    return multi_gemm_ws(pair, 2, x_rows, r) + bufs;
 }
 
 sllm_status swiglu_impl(const sllm_weight *wg, const sllm_weight *wu, const float *x, int x_rows, float *h,
@@ -1193,11 +1209,19 @@ sllm_status sllm_rmsnorm_matmul_swiglu_dev(const sllm_weight *wg, const sllm_wei
     size_t need = 0;
     const sllm_weight *const both[2] = {wg, wu};
     Route r;
+    bool fused = false;  // normed as they are quantized
     auto bytes = [&] {
-        return (all_int8_gemm(both, 2, x_rows, r) ? 0 : nb) + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, r);
+        Route t = r;
+        const size_t b = swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, t);
+        if ((fused = all_int8_gemm(both, 2, x_rows, t))) {
+            r = t;
+            return b;
+        }
+        take(r, nb);
+        return nb + swiglu_ws_bytes(wg, wu, x_rows, nullptr, nullptr, r);
     };
     if ((st = fit_workspace(s, r, bytes, &ws, &need)) != SLLM_OK) return st;
-    if (all_int8_gemm(both, 2, x_rows, r))  // normed as they are quantized
+    if (fused)
         return swiglu_impl(wg, wu, x, x_rows, h, nullptr, nullptr, s, ws, norm_w, eps, r);
     float *normed = (float *)ws;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
@@ -1281,14 +1305,17 @@ sllm_status sllm_rmsnorm_matmul_multi_dev(const sllm_weight *const *ws, int coun
         return multi_impl(ws, count, x, x_rows, dst, s, nullptr, 0, norm_w, eps, Route{});
     const size_t nb = align256((size_t)x_rows * x_cols * sizeof(float));
     Route r;
-    auto bytes = [&] { return (all_int8_gemm(ws, count, x_rows, r) ? 0 : nb) + multi_gemm_ws(ws, count, x_rows, r); };
+    bool fused = false;  // normed as they are quantized
+    auto bytes = [&] {
+        if (!(fused = all_int8_gemm(ws, count, x_rows, r))) take(r, nb);
+        return (fused ? 0 : nb) + multi_gemm_ws(ws, count, x_rows, r);
+    };
     // several rows: normed rows into the workspace first, then every weight
     // reads them (GEMV and GEMM alike)
     void *ws_ = nullptr;
     size_t need = 0;
     if ((st = fit_workspace(s, r, bytes, &ws_, &need)) != SLLM_OK) return st;
-    if (all_int8_gemm(ws, count, x_rows, r))  // normed as they are quantized
-        return multi_impl(ws, count, x, x_rows, dst, s, ws_, need, norm_w, eps, r);
+    if (fused) return multi_impl(ws, count, x, x_rows, dst, s, ws_, need, norm_w, eps, r);
     float *normed = (float *)ws_;
     if ((st = launch_rmsnorm(x, norm_w, eps, x_rows, x_cols, normed, s)) != SLLM_OK) return st;
     return multi_impl(ws, count, normed, x_rows, dst, s, (char *)ws_ + nb, need - nb, nullptr, 0.0f, r);

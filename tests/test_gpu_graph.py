@@ -3,6 +3,9 @@ same bits as the eager launches, replay after replay, with eager work and
 input changes in between (the decode loop's use of the library)."""
 from __future__ import annotations
 
+import contextlib
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -147,3 +150,116 @@ def test_workspace_growth_under_capture_is_an_error_and_reserve_avoids_it():
         g2.replay()
         torch.cuda.synchronize()
         assert torch.equal(yb.view(torch.int32), want.view(torch.int32)), rep
+
+
+@contextlib.contextmanager
+def _capture(g, stream):
+    # no garbage collection inside: it could destroy an earlier graph or weight, which
+    # synchronizes the device, while this one is being captured
+    gc.collect()
+    gc.disable()
+    try:
+        with torch.cuda.graph(g, stream=stream):
+            yield
+    finally:
+        gc.enable()
+
+
+def _captured(call, stream):
+    g = torch.cuda.CUDAGraph()
+    with _capture(g, stream):
+        call(stream.cuda_stream)
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+    return g
+
+
+def _matmul(w, x, stream=0):
+    y = torch.full((x.shape[0], w.rows), float("nan"), device="cuda")
+    sq.matmul_dev(w, x.data_ptr(), x.shape[0], x.shape[1], y.data_ptr(), stream)
+    return y
+
+
+@pytest.mark.parametrize("qtype,N,K,M", [("q5", 96, 512, 15), ("q4_1", 40, 4096, 6), ("q8", 96, 512, 15),
+                                         ("q5k1", 4097, 256, 5)])
+def test_capture_without_workspace_takes_the_gemv_below_the_tiled_gemms_rows(qtype, N, K, M):
+    w = sq.DeviceWeight.from_quant(sq.QuantWeight(qtype, make_raw(qtype, N, K, seed=1), K // 32, N, K))
+    x = torch.from_numpy(make_x(M, K, seed=2)).cuda()
+    eager = _matmul(w, x)
+    sq.set_param("gemm_min_rows", 1 << 20)
+    gemv = _matmul(w, x)
+    sq.set_param("gemm_min_rows", 0)
+    y = torch.empty_like(gemv)
+    g = _captured(lambda s: sq.matmul_dev(w, x.data_ptr(), M, K, y.data_ptr(), s), torch.cuda.Stream())
+    assert torch.equal(y, gemv) and not torch.equal(y, eager)
+    del g
+
+
+@pytest.mark.parametrize("qtype,N,K,M", [("q5", 96, 512, 16), ("q5", 96, 512, 300), ("q8", 96, 512, 16),
+                                         ("q4_1", 40, 4096, 33)])
+def test_capture_without_workspace_refuses_the_tiled_gemms_rows(qtype, N, K, M):
+    w = sq.DeviceWeight.from_quant(sq.QuantWeight(qtype, make_raw(qtype, N, K, seed=1), K // 32, N, K))
+    x = torch.from_numpy(make_x(M, K, seed=2)).cuda()
+    y = torch.zeros((M, N), device="cuda")
+    s, err = torch.cuda.Stream(), None
+    g = torch.cuda.CUDAGraph()
+    with _capture(g, s):
+        y.fill_(1.0)
+        try:
+            sq.matmul_dev(w, x.data_ptr(), M, K, y.data_ptr(), s.cuda_stream)
+        except sq.SllmError as e:
+            err = (e.status, str(e))
+    del g
+    assert err is not None and err[0] == 1 and "sllm_workspace_reserve" in err[1]
+
+
+def test_capture_decides_for_each_weight_by_itself():
+    # the workspace holds the small weight's GEMM, not the large one's: beside it the
+    # small weight still gives its single call's bits
+    from test_gpu_kquant_native import make_kq
+    K, M = 2048, 9
+    small, large = (sq.load_weight_f32_direct(10, make_kq(10, n, K, n), n, K) for n in (96, 8192))
+    x = torch.from_numpy(make_x(M, K, seed=3)).cuda()
+    sq.set_param("gemm_splits", 16)  # 16 x 9 x 8192 floats of partial sums: more than the 4 MiB a stream starts with
+    try:
+        sq.set_param("gemm_min_rows", 1 << 20)
+        gemv = [_matmul(w, x) for w in (small, large)]
+        sq.set_param("gemm_min_rows", 0)
+        single = _matmul(small, x)
+        s = torch.cuda.Stream()
+        sq.workspace_reserve(s.cuda_stream, 1)
+        ys = [torch.empty_like(t) for t in gemv]
+        nys = [torch.empty_like(t) for t in gemv]
+        ones = torch.ones(K, device="cuda")
+
+        def call(st):
+            sq.matmul_multi_dev([small, large], x.data_ptr(), M, K, [y.data_ptr() for y in ys], st)
+            sq.rmsnorm_matmul_multi_dev([small, large], x.data_ptr(), ones.data_ptr(), 1e-5, M, K,
+                                        [y.data_ptr() for y in nys], st)
+        g = _captured(call, s)
+    finally:
+        sq.set_param("gemm_splits", 0)
+        sq.set_param("gemm_min_rows", 0)
+    assert not torch.equal(single, gemv[0])
+    assert torch.equal(ys[0], single) and torch.equal(ys[1], gemv[1])
+    assert all(torch.isfinite(y).all() for y in nys)
+    del g
+
+
+@pytest.mark.parametrize("M", [6, 12])
+def test_capture_of_a_mixed_gate_up_pair_without_workspace(M):
+    # int8 weights of two formats: the pair needs buffers of its own, so a stream
+    # without workspace refuses; with a little reserved it runs
+    K, N = 4096, 64
+    ws = [sq.DeviceWeight.from_quant(sq.QuantWeight(q, make_raw(q, N, K, seed=5), K // 32, N, K)) for q in ("q8", "q4_1")]
+    x = torch.from_numpy(make_x(M, K, seed=6)).cuda()
+    nw = torch.ones(K, device="cuda")
+    h, want = (torch.full((M, N), float("nan"), device="cuda") for _ in range(2))
+    call = lambda y: lambda s: sq.rmsnorm_matmul_swiglu_dev(*ws, x.data_ptr(), nw.data_ptr(), 1e-5, M, K, y.data_ptr(), s)
+    call(want)(0)
+    s = torch.cuda.Stream()
+    sq.workspace_reserve(s.cuda_stream, 1)
+    g = _captured(call(h), s)
+    assert torch.isfinite(want).all() and torch.equal(h, want)
+    del g
