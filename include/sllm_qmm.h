@@ -478,6 +478,11 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  moves the fp32 summation splits
  *   gemm_splits         0..64      GEMM K splits, added in split order (0: by tile count;
  *                                  the split count moves the fp32 summation splits)
+ *   workspace_max_mb    >= 0       MiB of a stream's workspace that one call may use (0: what
+ *                                  can be allocated). A call that needs more, or whose
+ *                                  workspace cannot be allocated, takes the kernels that
+ *                                  need less, as under capture (sllm_workspace_reserve),
+ *                                  or returns SLLM_ERR_OOM where there is none
  *   attn_target_blocks  1..65536   attention: about this many workgroups when splitting (512)
  *   attn_tile_groups    1..4       attention: most tile groups per workgroup (4)
  *   attn_head_slices    0..64      attention: workgroups sharing a kv head's q heads

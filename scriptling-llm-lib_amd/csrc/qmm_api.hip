@@ -135,18 +135,21 @@ sllm_status amax_scratch(hipStream_t stream, void **out) {
 // live one). The old buffer is retired, not freed (work queued on the stream
 // and graphs captured on it may still use it). A stream under capture cannot
 // grow its workspace: the caller reserves it first (sllm_workspace_reserve), or,
-// given `stuck`, is told so there instead of by an error.
+// given `stuck`, is told so there instead of by an error. Where it cannot be had,
+// *cap says what there is.
 sllm_status workspace(hipStream_t stream, size_t need, void **out, size_t *cap, bool *stuck = nullptr) {
     int dev = 0;
     SLLM_HIP(hipGetDevice(&dev));
     const uint64_t key = ((uint64_t)(uintptr_t)stream << 8) ^ (uint64_t)dev;
     std::lock_guard<std::mutex> lk(g_mu);
     Ws &w = g_ws[key];
+    const size_t limit = tuning().workspace_max_mb ? (size_t)tuning().workspace_max_mb << 20 : SIZE_MAX;
+    *cap = w.cap < limit ? w.cap : limit;
+    if (need > limit) return set_error(SLLM_ERR_OOM, "the workspace would exceed workspace_max_mb");
     if (w.cap < need) {
         if (capturing(stream)) {
             if (stuck) {
                 *stuck = true;
-                *cap = w.cap;
                 return SLLM_OK;
             }
             return set_error(SLLM_ERR_ARG, "the stream's workspace must grow to " + std::to_string(need) +
@@ -156,7 +159,11 @@ sllm_status workspace(hipStream_t stream, size_t need, void **out, size_t *cap, 
         size_t want = need < ((size_t)4 << 20) ? ((size_t)4 << 20) : need;
         want = want < 2 * w.cap ? 2 * w.cap : want;
         void *p = nullptr;
-        if (hipMalloc(&p, want) != hipSuccess) return set_error(SLLM_ERR_OOM, "workspace allocation failed");
+        want = want < limit ? want : limit;
+        if (hipMalloc(&p, want) != hipSuccess) {
+            (void)hipGetLastError();  // reported here, not by the next launch
+            return set_error(SLLM_ERR_OOM, "workspace allocation failed");
+        }
         if (w.p) w.retired.push_back(w.p);
         w.p = p;
         w.cap = want;
@@ -164,20 +171,6 @@ sllm_status workspace(hipStream_t stream, size_t need, void **out, size_t *cap, 
     *out = w.p;
     *cap = w.cap;
     return SLLM_OK;
-}
-
-// Whether workspace(stream, need) would succeed as far as capture goes: the
-// stream's workspace is large enough, or the stream is not being captured.
-bool workspace_at_hand(hipStream_t stream, size_t need) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return false;
-    const uint64_t key = ((uint64_t)(uintptr_t)stream << 8) ^ (uint64_t)dev;
-    {
-        std::lock_guard<std::mutex> lk(g_mu);
-        auto it = g_ws.find(key);
-        if (it != g_ws.end() && it->second.cap >= need) return true;
-    }
-    return !capturing(stream);
 }
 
 // The scratch of sllm_attention_noalloc_dev: the attention's rotated q rows
@@ -587,8 +580,9 @@ sllm_status run_matmul(const sllm_weight *w, const float *x, int x_rows, float *
     return launch_gemm(gemm_fmt(w), P, x, dst, w->rows, w->groups, x_rows, ws, cap, false, false, s);
 }
 
-// The workspace of a call that needs need() bytes, written to *bytes; on a stream under
-// capture whose workspace is smaller r.room is set first, and need() asked again.
+// The workspace of a call that needs need() bytes, written to *bytes; where that cannot
+// be had (a stream under capture, no memory) r.room is set to what there is, and need()
+// asked again.
 template <class F>
 sllm_status fit_workspace(hipStream_t s, Route &r, F need, void **ws, size_t *bytes) {
     size_t cap = 0;
@@ -596,7 +590,7 @@ sllm_status fit_workspace(hipStream_t s, Route &r, F need, void **ws, size_t *by
     if ((*bytes = need()) == 0) return SLLM_OK;
     bool stuck = false;
     const sllm_status st = workspace(s, *bytes, ws, &cap, &stuck);
-    if (!stuck) return st;
+    if (!stuck && st != SLLM_ERR_OOM) return st;
     r.room = cap;
     if ((*bytes = need()) == 0) return SLLM_OK;
     return workspace(s, *bytes, ws, &cap);
@@ -786,11 +780,10 @@ sllm_status attention_impl(sllm_kv_cache *kv, int layer, const sllm_attn_params 
     size_t wsb = 0;
     attention_plan(seq_len, p->n_heads, kv->n_kv, kv->d_k, cl + seq_len, &splits, &tps, &tw, &hs, &wsb);
     // The matrix-core kernel needs more scratch where rows are long: where that
-    // cannot be had (a stream under capture), the split kernel's plan holds. (The
-    // static scratch holds it for every call that it takes.)
+    // cannot be had (a stream under capture, no memory), the split kernel's plan holds.
+    // (The static scratch holds it for every call that it takes.)
     size_t fwsb = 0;
-    bool flash = attention_flash(seq_len, p->n_heads, kv->n_kv, kv->d_k, cl, out, &fwsb) &&
-                 (noalloc || fwsb <= wsb || workspace_at_hand(s, fwsb));
+    bool flash = attention_flash(seq_len, p->n_heads, kv->n_kv, kv->d_k, cl, out, &fwsb);
     void *ws = nullptr;
     size_t cap = 0;
     if (noalloc) {
@@ -800,8 +793,14 @@ sllm_status attention_impl(sllm_kv_cache *kv, int layer, const sllm_attn_params 
                                                  std::to_string(kNoallocBytes) +
                                                  " (fewer rows per call, or sllm_attention_dev)");
         if ((st = static_scratch(&ws)) != SLLM_OK) return st;
-    } else if ((st = workspace(s, flash ? fwsb : wsb, &ws, &cap)) != SLLM_OK) {
-        return st;
+    } else {
+        bool stuck = false;
+        if (flash) {
+            st = workspace(s, fwsb, &ws, &cap, &stuck);
+            if (stuck || st == SLLM_ERR_OOM) flash = false;
+            else if (st != SLLM_OK) return st;
+        }
+        if (!flash && (st = workspace(s, wsb, &ws, &cap)) != SLLM_OK) return st;
     }
     AttnArgs a{};
     a.q = q;
@@ -894,6 +893,7 @@ sllm_status sllm_set_param(const char *name, int value) {
     else if (!std::strcmp(name, "attn_head_slices") && value >= 0 && value <= 64) t.attn_head_slices = value;
     else if (!std::strcmp(name, "gemm_shape") && value >= 0 && value <= 5) t.gemm_shape = value;
     else if (!std::strcmp(name, "gemm_min_rows") && value >= 0) t.gemm_min_rows = value;
+    else if (!std::strcmp(name, "workspace_max_mb") && value >= 0) t.workspace_max_mb = value;
     else if (!std::strcmp(name, "gemm_splits") && value >= 0 && value <= 64) t.gemm_splits = value;
     else if (!std::strcmp(name, "gemv_q4k_stream") && (value == 0 || value == 1)) t.gemv_q4k_stream = value;
     else if (!std::strcmp(name, "gemv_q6k_stream") && (value == 0 || value == 1)) t.gemv_q6k_stream = value;

@@ -311,6 +311,7 @@ struct Tuning {
     int attn_target_blocks = 512;  // attention: splits chosen to give about this many workgroups
     int attn_tile_groups = 4;      // attention: most tile groups (of max(4, rep) waves) per workgroup
     int attn_head_slices = 0;      // attention: workgroups sharing one kv head's q heads (0: by workgroup count)
+    int workspace_max_mb = 0;      // MiB of a stream's workspace that a call may use (0: what can be allocated)
 };
 Tuning &tuning();
 
