@@ -874,9 +874,9 @@ const char *sllm_kernel_info(void) {
     char buf[512];
     std::snprintf(buf, sizeof buf,
                   "sllm_qmm gfx950 planes-v1 | gemv: persistent, <=%d waves/WG, %d WG/CU, fused Q8_0 LDS "
-                  "prologue, non-temporal weight stream | gemm: int8 MFMA from xRows>=%s",
+                  "prologue, non-temporal weight stream | gemm: int8 / bf16 MFMA from xRows>=%s",
                   t.gemv_waves, t.gemv_wg_per_cu,
-                  t.gemm_min_rows ? std::to_string(t.gemm_min_rows).c_str() : "8 (16 below 2^24 weights)");
+                  t.gemm_min_rows ? std::to_string(t.gemm_min_rows).c_str() : "5..16 (by format and weight)");
     info = buf;
     return info.c_str();
 }

@@ -1,5 +1,6 @@
-// Prefill GEMM of the int8 formats (xRows >= 8 or 16): the int8 matrix cores for
-// Q8_0 / Q4_0 / Q4_1 / Q5K1 (Q5_0, Q2_K and Q3_K keep fp32 activations:
+// Prefill GEMM of the int8 formats (prompts of more than 32 rows, and from 8 or 16 rows
+// the weights that the short-prompt GEMM, qmm_sgemm.hip, does not take): the int8 matrix
+// cores for Q8_0 / Q4_0 / Q4_1 / Q5K1 (Q5_0, Q2_K and Q3_K keep fp32 activations:
 // qmm_bgemm.hip).
 //
 // 1. The activation rows are quantized once into a workspace (xq int8 [M][K],

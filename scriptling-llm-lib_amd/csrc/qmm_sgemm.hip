@@ -477,9 +477,9 @@ sgemm_kernel(SegG S, SAct A, int M, int G) {
         const size_t o = (size_t)m * Ns + col;
         if (pair) {
             const float u = tree_sum(KW, [&](int w) { return lds[(KW + w) * E + e]; });
-            dst[o] = swiglu(s, u);
             if (S.dst[1]) S.dst[1][o] = s;
             if (S.dst[2]) S.dst[2][o] = u;
+            dst[o] = swiglu(s, u);  // last: h may lie over gate or up, as for the tiled GEMM
         } else {
             dst[o] = S.mode == kAdd ? dst[o] + s : s;
         }

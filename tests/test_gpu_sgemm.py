@@ -213,3 +213,19 @@ def test_normed_gate_up_pair_equals_norm_then_pair(qtype, M, K):
     sq.matmul_swiglu_dev(a, b, nd.data_ptr(), M, K, want.data_ptr())
     torch.cuda.synchronize()
     assert torch.isfinite(want).all() and torch.equal(h.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("over", ["gate", "up"])
+@pytest.mark.parametrize("M", [9, 33])
+def test_h_over_gate_or_up_holds_the_swiglu(M, over):
+    # the same buffer for h and gate (or up): the tiled GEMM's pass leaves h there, and
+    # so does the short-prompt GEMM's epilogue
+    _, a = weight("q8", 70, 512, 19)
+    _, b = weight("q8", 70, 512, 20)
+    x = torch.from_numpy(make_x(M, 512, seed=21)).cuda()
+    h, both = (torch.full((M, 70), float("nan"), device="cuda") for _ in range(2))
+    sq.matmul_swiglu_dev(a, b, x.data_ptr(), M, 512, h.data_ptr())
+    p = both.data_ptr()
+    sq.matmul_swiglu_dev(a, b, x.data_ptr(), M, 512, p, p if over == "gate" else 0, p if over == "up" else 0)
+    torch.cuda.synchronize()
+    assert torch.isfinite(h).all() and torch.equal(both, h)
