@@ -101,39 +101,30 @@ __device__ void prep_row(float *row, const float *src, int dk, const float *bias
 
 // Several rows (prefill): q heads go to the workspace, kv heads into the cache (k:
 // bias, norm, RoPE; v: bias) at rows cache_len + s (the append, model_f32.go:445-448).
-// prep_head: head t of row s (q heads, then kv heads) into row (LDS), rotated by `half`
-// frequencies; put_head: row to where it belongs.
-__device__ __forceinline__ void prep_head(const AttnArgs &a, int s, int t, float *row, int half, int lane) {
+// Few rows before the split kernel: one wave per (row, head).
+__global__ void __launch_bounds__(64) attn_prep_kernel(AttnArgs a) {
+    __shared__ float row[kMaxDk];
+    const int s = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
     const int dk = a.d_k;
     const bool isq = t < a.n_heads;
     const int h = isq ? t : t - a.n_heads;
     const int cols = (isq ? a.n_heads : a.n_kv) * dk;
     prep_row(row, (isq ? a.q : a.k) + (size_t)s * cols + (size_t)h * dk, dk, isq ? a.q_bias : a.k_bias, h * dk,
-             isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, a.freqs, half, a.start_pos + s, lane);
-}
-__device__ __forceinline__ void put_head(const AttnArgs &a, int s, int t, const float *row, int lane) {
-    const int dk = a.d_k;
-    if (t < a.n_heads) {
-        float *dst = a.qrot + ((size_t)s * a.n_heads + t) * dk;
+             isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, a.freqs, a.half_dim, a.start_pos + s,
+             lane);
+    if (isq) {
+        float *dst = a.qrot + ((size_t)s * a.n_heads + h) * dk;
         for (int d = lane; d < dk; d += 64) dst[d] = row[d];
         return;
     }
-    const int h = t - a.n_heads;
     const size_t at = ((size_t)h * a.cap + (size_t)(a.cache_len + s)) * dk;
-    const float *vs = a.v + ((size_t)s * a.n_kv + h) * dk;
+    const float *vs = a.v + (size_t)s * cols + (size_t)h * dk;
     for (int d = lane; d < dk; d += 64) {
         a.cache_k[at + d] = row[d];
         float x = vs[d];
         if (a.v_bias && h * dk + d < a.vb_len) x = x + a.v_bias[h * dk + d];
         a.cache_v[at + d] = x;
     }
-}
-
-// Few rows before the split kernel: one wave per (row, head).
-__global__ void __launch_bounds__(64) attn_prep_kernel(AttnArgs a) {
-    __shared__ float row[kMaxDk];
-    prep_head(a, blockIdx.x, blockIdx.y, row, a.half_dim, threadIdx.x);
-    put_head(a, blockIdx.x, blockIdx.y, row, threadIdx.x);
 }
 
 // Prompts: gridDim.y workgroups per row. The row's rotation (the same for every head)
@@ -149,12 +140,20 @@ __global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_rows_kernel(AttnArg
     __shared__ float rows[kPrepWaves][kMaxDk];
     __shared__ float rc[kMaxDk / 2], rs[kMaxDk / 2];
     const int s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int dk = a.d_k;
     float *row = rows[wave];
+    auto prep = [&](int t) {
+        const bool isq = t < a.n_heads;
+        const int h = isq ? t : t - a.n_heads;
+        const int cols = (isq ? a.n_heads : a.n_kv) * dk;
+        prep_row(row, (isq ? a.q : a.k) + (size_t)s * cols + (size_t)h * dk, dk, isq ? a.q_bias : a.k_bias, h * dk,
+                 isq ? a.qb_len : a.kb_len, isq ? a.q_norm : a.k_norm, a.eps, nullptr, 0, 0, lane);
+    };
     // the first head's row is loaded with the frequency (half_dim is below the
     // workgroup's threads), not behind the rotation's barrier
-    const float fr = (int)threadIdx.x < a.half_dim ? a.freqs[threadIdx.x] : 0.0f;
     const int first = blockIdx.y * kPrepWaves + wave;
-    if (first < a.n_heads + a.n_kv) prep_head(a, s, first, row, 0, lane);
+    const float fr = (int)threadIdx.x < a.half_dim ? a.freqs[threadIdx.x] : 0.0f;
+    if (first < a.n_heads + a.n_kv) prep(first);
     static_assert(kMaxDk / 2 <= 64 * kPrepWaves, "a thread per frequency");
     if ((int)threadIdx.x < a.half_dim) {
         const float ang = fr * (float)(a.start_pos + s);
@@ -165,7 +164,10 @@ __global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_rows_kernel(AttnArg
     }
     __syncthreads();
     for (int t = first; t < a.n_heads + a.n_kv; t += gridDim.y * kPrepWaves) {
-        if (t != first) prep_head(a, s, t, row, 0, lane);
+        const bool isq = t < a.n_heads;
+        const int h = isq ? t : t - a.n_heads;
+        const int cols = (isq ? a.n_heads : a.n_kv) * dk;
+        if (t != first) prep(t);
         // RoPE (applyRopeInPlaceF32, float32_ops.go:174-188)
         for (int i = lane; i < a.half_dim; i += 64) {
             const float c = rc[i], sn = rs[i];
@@ -174,7 +176,19 @@ __global__ void __launch_bounds__(64 * kPrepWaves) attn_prep_rows_kernel(AttnArg
             row[2 * i + 1] = x0 * sn + x1 * c;
         }
         wave_lds_sync();
-        put_head(a, s, t, row, lane);
+        if (isq) {
+            float *dst = a.qrot + ((size_t)s * a.n_heads + h) * dk;
+            for (int d = lane; d < dk; d += 64) dst[d] = row[d];
+        } else {
+            const size_t at = ((size_t)h * a.cap + (size_t)(a.cache_len + s)) * dk;
+            const float *vs = a.v + (size_t)s * cols + (size_t)h * dk;
+            for (int d = lane; d < dk; d += 64) {
+                a.cache_k[at + d] = row[d];
+                float x = vs[d];
+                if (a.v_bias && h * dk + d < a.vb_len) x = x + a.v_bias[h * dk + d];
+                a.cache_v[at + d] = x;
+            }
+        }
         wave_lds_sync();  // the row is read before the next head's is written
     }
 }
@@ -652,9 +666,11 @@ __global__ void __launch_bounds__(64 * kLongWaves) attn_combine_long_kernel(Attn
 // added by the MFMA), the exponentials float32(exp(float64(x))) as the reference's
 // (exp_neg), the sums fp32, in another association than the split kernel's.
 //
-// What bounds it: the fp32 matrix cores (64 cycles per 32 x 32 x 2; 2 DK of
-// them per tile); the split kernel spent 64-lane VALU dots and one pass over K
-// and V per query row (1024 rows of 32 / 8 heads, d_k 128: 882 us, now 139).
+// What bounds it: the fp32 matrix cores (64 cycles per 32 x 32 x 2, DK of them per tile:
+// busy for 47 % of 126 us) and what they wait on, issue behind each other and the
+// softmax between the two products (waves ready for 65 % of their cycles, VALU busy 18
+// %). The split kernel spent 64-lane VALU dots and one pass over K and V per query row
+// (1024 rows of 32 / 8 heads, d_k 128, whole call: 882 us, now 152).
 // Causal rows differ in length: a row block's tiles are cut into chunks of C
 // tiles (workgroups of their own; heaviest first) whose states
 // attn_flash_combine_kernel merges; C is about the tiles one workgroup slot gets
