@@ -476,7 +476,8 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  to 128, else 1); Q5_0, Q2K, Q3K: 1 = 32 x 256, 2 = 64 x
  *                                  128, 3 = 128 x 256 (0: by rows and weight). The shape
  *                                  moves the fp32 summation splits
- *   gemm_splits         0..64      GEMM K splits, added in split order (0: by tile count;
+ *   gemm_splits         0..64      GEMM K splits, added in split order (Q5_0, Q2K, Q3K: in
+ *                                  trees of eight; 0: by tile count;
  *                                  the split count moves the fp32 summation splits)
  *   workspace_max_mb    >= 0       MiB of a stream's workspace that one call may use (0: what
  *                                  can be allocated). A call that needs more, or whose

@@ -634,7 +634,7 @@ sllm_status launch_bgemm(int fmt, const Planes &P, const float *x, float *dst, i
     if (st != SLLM_OK || p.splits == 1) return st;
     const BWs L = layout(fmt, M, N, G, p);
     return launch_reduce_splits((const float *)((char *)ws + L.frag + L.xsum + L.flag), dst, (size_t)M * N, p.splits,
-                                add, s);
+                                add, true, s);
 }
 
 }  // namespace sllm

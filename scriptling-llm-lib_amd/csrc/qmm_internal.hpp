@@ -235,9 +235,9 @@ sllm_status launch_sgemm(int fmt, const Planes *P, float *const *dst, const int 
 sllm_status launch_bgemm(int fmt, const Planes &P, const float *x, float *dst, int N, int G, int M, void *ws, bool add,
                          hipStream_t s);
 size_t bgemm_workspace_bytes(int fmt, int N, int G, int M);
-// dst = part[0] + part[1] + ... + part[S - 1] (n floats each), in split order; add:
-// dst += that sum.
-sllm_status launch_reduce_splits(const float *part, float *dst, size_t n, int S, bool add, hipStream_t s);
+// dst = part[0] + part[1] + ... + part[S - 1] (n floats each), in split order or (tree)
+// eight at a time, each eight as a binary tree; add: dst += that sum.
+sllm_status launch_reduce_splits(const float *part, float *dst, size_t n, int S, bool add, bool tree, hipStream_t s);
 sllm_status launch_quantize_act(const float *x, int rows, int G, int8_t *xq, float *xs, int32_t *sx,
                                 hipStream_t s);
 sllm_status launch_block_dots(int fmt, const Planes &P, const float *x, int N, int G, int M,

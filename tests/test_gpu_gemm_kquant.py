@@ -169,3 +169,19 @@ def test_the_line_between_gemv_and_gemm(t, N, K, M, gemm_from):
     sq.set_param("gemm_min_rows", 0)
     assert not np.array_equal(gemv, forced)  # two orders
     assert np.array_equal(gemm(w, x), forced if M >= gemm_from else gemv)
+
+
+@pytest.mark.parametrize("t", [10, 11])
+@pytest.mark.parametrize("K,M", [(4096, 8), (14336, 8), (14336, 33), (4096, 130)])
+def test_gemm_is_as_close_to_64_bits_as_the_gemv(t, K, M):
+    # many K splits included (these shapes take up to 32): their sums are added in
+    # trees, not in one chain
+    N = 256
+    raw = make_kq(t, N, K, 51)
+    w = sq.load_weight_f32_direct(t, raw, N, K)
+    x = np.random.default_rng(52).normal(size=(M, K)).astype(np.float32)
+    ref = x.astype(np.float64) @ oracle.dense_weights(t, raw, N, K).astype(np.float64).T
+    err = lambda y: np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    e = err(gemm(w, x))
+    sq.set_param("gemm_min_rows", 1 << 20)
+    assert e <= 1.03 * err(gemm(w, x))
