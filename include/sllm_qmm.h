@@ -462,8 +462,9 @@ sllm_status sllm_debug_gemm_block_dots(const sllm_weight *w, const float *x, int
  *                                  above 2^22, else 9; the
  *                                  int8 formats where the short-prompt GEMM takes them (up
  *                                  to 32 rows and 8192 columns, a multiple of 256; 4096
- *                                  for at most 4096 weight rows): 5 above 4096 weight
- *                                  rows, else 6 at 4096 columns, else 7;
+ *                                  for at most 4096 weight rows): 8 above 4096
+ *                                  columns, else 5 above 4096 weight rows, else 6 at 4096
+ *                                  columns, else 7;
  *                                  the GEMM and GEMV sum a row's blocks in different
  *                                  orders, so a row's last bits can change with it)
  *   gemm_shape          0..5       GEMM workgroups: 1 = 64 x 128 tiles, 2 = 64 x 64 tiles with

@@ -532,14 +532,17 @@ bool uses_gemm(const sllm_weight *w, int x_rows, const Route &r) {
     }
     // The short-prompt GEMM from 5 rows, where the GEMV takes a second launch, for
     // weights of more than 4096 rows; from 6 for fewer of 4096 columns; from 7, where the
-    // GEMV's second launch has three rows, for the rest. The line is the weight's own, so
+    // GEMV's second launch has three rows, for the rest; and from 8, the tiled GEMM's
+    // rows, above 4096 columns, where the GEMV's sums are the more precise (error against
+    // 64 bits over 8192 columns 8.8e-8 / 9.6e-8, the tiled GEMM 10.9e-8). The line is the weight's own, so
     // that it gives the same bits alone and beside others. Measured (us, GEMV / GEMM, M =
     // 5, 6 and 7): Q4_1 14336x4096 25.7 / 21.0 (M = 5), 8192x2048 11.7 / 9.7 (M = 5), 4096x4096
     // 12.0 / 12.4, 13.2 / 12.4, 17.3 / 12.5, 2560x4096 11.3 / 12.1, 12.2 / 12.1, 16.2 / 12.1,
     // 2048x2048 8.0 / 9.1, 8.6 / 9.1, 11.5 / 9.1, 512x1024 7.0 / 8.3, 7.3 / 8.3, 10.1 / 8.3.
     // (Three weights in one launch, q / k / v of Q4_1 4096 + 2 x 1024 rows, would gain from 5
     // rows: 20.8 / 15.4.)
-    if (min_rows == 0 && sgemm_route(w, x_rows, r)) min_rows = w->rows > 4096 ? 5 : w->cols >= 4096 ? 6 : 7;
+    if (min_rows == 0 && sgemm_route(w, x_rows, r))
+        min_rows = w->cols > 4096 ? 8 : w->rows > 4096 ? 5 : w->cols == 4096 ? 6 : 7;
     if (min_rows == 0) min_rows = tiled_rows;
     return x_rows >= min_rows && gemm_supported(w->fmt, w->groups);
 }

@@ -20,11 +20,20 @@
 //   16 parts whose sums are added as a binary tree, whichever waves form them:
 //   an output's order depends on K alone, so a weight gives the same bits alone,
 //   beside others and in a gate / up pair.
-// The per-block arithmetic is the tiled GEMM's: v_mfma_i32_32x32x32_i8 gives a
-// block's exact dots on top of 1.5 * 2^23, t = fma(F, d, -1.5 * 2^23 d), acc =
-// fma(t, xs, acc), min terms two blocks at a time through v_mfma_f32_32x32x2_f32;
-// eight blocks that hold a non-finite scale, or an activation scale from 2^90,
-// are computed in the reference's operation order (qmm_gemm.hip has the reasons).
+// The per-block arithmetic: v_mfma_i32_32x32x32_i8 gives a block's exact dots (on top of
+// 1.5 * 2^23 as the tiled GEMM has them, or as integers), t = d dot with one rounding,
+// acc = fma(t, xs, acc). A min joins its block's term before the scale, t = fma(Σxq, m,
+// t), as the reference and the GEMV have it: d dot and m Σxq nearly cancel, and apart, as
+// the tiled GEMM adds them, they enter the sum at their own size (error against 64 bits
+// over K = 768 / 4096: Q4_1 6.4e-8 / 7.7e-8, apart 1.1e-7 / 1.2e-7, the GEMV 6.4e-8 / 7.8e-8;
+// Q5K1 6.7e-8 / 7.9e-8, apart 9.5e-8 / 1.0e-7, the GEMV 8.4e-8 / 9.5e-8; it costs Q5K1
+// 4096x4096 at M = 16 14.1 -> 15.0 us, Q4_1 12.8 -> 13.4). Eight blocks that hold a
+// non-finite scale, or an activation scale from 2^90, are computed in the reference's
+// operation order (qmm_gemm.hip has the reasons).
+//
+// Counters (RMSNorm + q / k / v, Q5K1 4096 / 1024, M = 30, 12.5 us for 39 MB of weights, of
+// which the caches held most): matrix cores busy 3 %, VALU 16 %, waves issuing 30 %,
+// waiting on loads and LDS 37 %: the chain of a wave's two chunks.
 #include <hip/hip_runtime.h>
 
 #include "qmm_device.hpp"
@@ -55,21 +64,19 @@ __host__ __device__ constexpr bool has_hb(int f) { return f == SLLM_Q5K1 || f ==
 
 // Quantized activations, 32 rows (rows past M: zeros):
 //   xq [g][lane][16]  codes: lane r + 32 h, elements 16 h .. of row r
-//   xs, xm, sx [g][32]  scale, float(Σxq) * scale, Σxq
+//   xs, sx [g][32]  scale, Σxq (exact in float32)
 struct SAct {
     int8_t *xq;
-    float *xs, *xm;
-    int *sx;
+    float *xs, *sx;
 };
 
-__host__ inline size_t sact_bytes(int G) { return (size_t)G * (1024 + 3 * 128); }
+__host__ inline size_t sact_bytes(int G) { return (size_t)G * (1024 + 2 * 128); }
 __host__ inline SAct carve_sact(void *ws, int G) {
     const size_t n = (size_t)G;
     SAct a;
     a.xq = (int8_t *)ws;
     a.xs = (float *)(a.xq + n * 1024);
-    a.xm = a.xs + n * 32;
-    a.sx = (int *)(a.xm + n * 32);
+    a.sx = a.xs + n * 32;
     return a;
 }
 
@@ -106,13 +113,12 @@ __device__ __forceinline__ void put_part(const SAct &a, int r, int g, int sub, c
     ((int *)(a.xq + t * 1024 + (r + 32 * (sub >> 2)) * 16))[sub & 3] = q[0];
     if (sub == 0) {
         a.xs[t * 32 + r] = s;
-        a.xm[t * 32 + r] = (float)sm * s;
-        a.sx[t * 32 + r] = sm;
+        a.sx[t * 32 + r] = (float)sm;
     }
 }
 
 // Without the norm: grid (32 rows, 32 blocks each). (One workgroup per row, its parts in
-// turn: every call 0.8-1 us longer, Q4_1 4096x4096 at M = 16 13.8 against 12.8.)
+// turn: every call 0.8-1 us longer, Q4_1 4096x4096 at M = 16 13.8 against 12.8 us.)
 __global__ void __launch_bounds__(256) sact_kernel(const float *__restrict__ x, int M, int G, SAct a) {
     const int r = blockIdx.x, sub = threadIdx.x & 7, g = blockIdx.y * 32 + (threadIdx.x >> 3);
     if (g >= G) return;  // eight lanes alike
@@ -180,6 +186,7 @@ struct alignas(16) Image {
     v4i hb[has_hb(FMT) ? 32 : 1][3];
     v4i a[kCh][64];  // the activation codes, lane's own
     float xs[kCh][32];
+    float sx[has_min(FMT) ? kCh : 1][32];
 };
 
 template <int FMT>
@@ -245,12 +252,11 @@ __device__ __forceinline__ void operand(const Image<FMT> &I, int b, int r32, int
     }
 }
 
-// The activation scales of a lane's 16 rows of block b.
-template <int FMT>
-__device__ __forceinline__ void read_xs(const Image<FMT> &I, int b, int h, float (&xv)[16]) {
+// The activation scales (or sums) of a lane's 16 rows of a block.
+__device__ __forceinline__ void read_rows(const float *x, int h, float (&xv)[16]) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const v4f u = *(const v4f *)(I.xs[b] + 8 * i + 4 * h);
+        const v4f u = *(const v4f *)(x + 8 * i + 4 * h);
 #pragma unroll
         for (int k = 0; k < 4; k++) xv[4 * i + k] = u[k];
     }
@@ -302,9 +308,12 @@ sgemm_kernel(SegG S, SAct A, int M, int G) {
     v16f acc;
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+    // a dot comes on top of 1.5 * 2^23 as a float, or (has_hb: registers are short) as an
+    // integer, converted
     v16i cmag;
 #pragma unroll
-    for (int v = 0; v < 16; v++) cmag[v] = kMagicBits;
+    for (int v = 0; v < 16; v++) cmag[v] = has_hb(FMT) ? 0 : kMagicBits;
+    auto dot_of = [](int d) { return has_hb(FMT) ? (float)d : __int_as_float(d) - kMagic; };  // exact
 
     // acc: the current part's sum; ones, twos: finished parts that wait for their
     // neighbours in the tree
@@ -328,19 +337,17 @@ sgemm_kernel(SegG S, SAct A, int M, int G) {
     if (c0 < c1) {
         Image<FMT> &I = ((Image<FMT> *)lds)[wave];
         Chunk<FMT> ck;
-        v4f xr;
+        v4f xr, sr;
         // Everything a chunk needs is requested a whole chunk ahead, the weights
         // last: loads return in order, so a load issued behind the next weights and
         // needed before them would wait for memory in every chunk.
         v4i a[kCh];
-        float xm[4], xmn[4];  // the min terms' activation parts, two blocks (one per lane half) at a time
         auto load = [&](int c) {
 #pragma unroll
             for (int i = 0; i < kCh; i++) a[i] = *(const v4i *)(A.xq + ((size_t)c * kCh + i) * 1024 + lane * 16);
             // kCh x 32 scales are contiguous, four per lane
             xr = *(const v4f *)(A.xs + (size_t)c * kCh * 32 + 4 * lane);
-#pragma unroll
-            for (int i = 0; i < 4; i++) xmn[i] = has_min(FMT) ? A.xm[((size_t)c * kCh + 2 * i + h) * 32 + r32] : 0.0f;
+            if (has_min(FMT)) sr = *(const v4f *)(A.sx + (size_t)c * kCh * 32 + 4 * lane);
             load_chunk<FMT>(ck, P, n0, N, G, c * kCh, lane);
         };
         load(c0);
@@ -356,9 +363,8 @@ sgemm_kernel(SegG S, SAct A, int M, int G) {
             put_chunk<FMT>(ck, I, lane);
 #pragma unroll
             for (int i = 0; i < kCh; i++) I.a[i][lane] = a[i];
-#pragma unroll
-            for (int i = 0; i < 4; i++) xm[i] = xmn[i];
             *(v4f *)((float *)I.xs + 4 * lane) = xr;
+            if (has_min(FMT)) *(v4f *)((float *)I.sx + 4 * lane) = sr;
 #pragma unroll
             for (int k = 0; k < 4; k++) slow |= !(xr[k] < kHugeXs);
             const bool exact = __ballot(slow) != 0;
@@ -379,21 +385,25 @@ sgemm_kernel(SegG S, SAct A, int M, int G) {
                         operand<FMT>(I, b, r32, h, q, qh);
                         const float wd = FMT == SLLM_Q8_0 ? f16_lut(half_of(du, i)) : f16_exact(half_of(du, i));
                         const float wdh = dual(FMT) ? f16_exact(half_of(hu, i)) : 0.0f;
-                        const float cd = -kMagic * wd, cdh = -kMagic * wdh;  // exact
-                        float xv[16];
-                        read_xs<FMT>(I, b, h, xv);
+                        const float cd = -kMagic * wd;  // exact
+                        const float wm = has_min(FMT) ? f16_exact(half_of(mu, i)) : 0.0f;
                         const v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(I.a[b][lane], q, cmag, 0, 0, 0);
                         v16i Dh = {};
                         if (dual(FMT)) Dh = __builtin_amdgcn_mfma_i32_32x32x32_i8(I.a[b][lane], qh, cmag, 0, 0, 0);
 #pragma unroll
-                        for (int v = 0; v < 16; v++) {
-                            float f = __builtin_fmaf(__int_as_float(D[v]), wd, cd);
-                            if (dual(FMT)) f = f + __builtin_fmaf(__int_as_float(Dh[v]), wdh, cdh);
-                            acc[v] = __builtin_fmaf(f, xv[v], acc[v]);
-                        }
-                        if (has_min(FMT) && (i & 1)) {
-                            const float mn = h ? f16_exact(half_of(mu, i)) : f16_exact(half_of(mu, i - 1));
-                            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xm[b >> 1], mn, acc, 0, 0, 0);
+                        for (int r = 0; r < 4; r++) {
+                            // four rows' scales and sums
+                            const v4f xv = *(const v4f *)(I.xs[b] + 8 * r + 4 * h);
+                            v4f sv = {};
+                            if (has_min(FMT)) sv = *(const v4f *)(I.sx[has_min(FMT) ? b : 0] + 8 * r + 4 * h);
+#pragma unroll
+                            for (int k = 0; k < 4; k++) {
+                                const int v = 4 * r + k;
+                                float f = has_hb(FMT) ? dot_of(D[v]) * wd : __builtin_fmaf(__int_as_float(D[v]), wd, cd);
+                                if (has_min(FMT)) f = __builtin_fmaf(sv[k], wm, f);
+                                if (dual(FMT)) f = __builtin_fmaf(dot_of(Dh[v]), wdh, f);
+                                acc[v] = __builtin_fmaf(f, xv[k], acc[v]);
+                            }
                         }
                     }
                 }
@@ -418,15 +428,15 @@ sgemm_kernel(SegG S, SAct A, int M, int G) {
                     const float wm = has_min(FMT) ? f16_exact(((const uint16_t *)&I.sc[1][r32])[b]) : 0.0f;
                     const float wdh = dual(FMT) ? f16_exact(((const uint16_t *)&I.dh[dual(FMT) ? r32 : 0])[b]) : 16.0f * wd;
                     const v4i av = I.a[b][lane];
-                    const int *sx = A.sx + ((size_t)c * kCh + b) * 32;
-                    float xv[16];
-                    read_xs<FMT>(I, b, h, xv);
+                    float xv[16], sv[16];
+                    read_rows(I.xs[b], h, xv);
+                    if (has_min(FMT)) read_rows(I.sx[has_min(FMT) ? b : 0], h, sv);
                     const v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, q, cmag, 0, 0, 0);
                     v16i Dh = {};
                     if (has_hb(FMT)) Dh = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, hq, cmag, 0, 0, 0);
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const float dot = __int_as_float(D[v]) - kMagic;  // exact
+                        const float dot = dot_of(D[v]);
                         if (!has_min(FMT)) {
                             // q8q8.go:193-195 + vnni_amd64.s:70-73; q4q8.go:37-43
                             const float cmb = wd * xv[v];
@@ -435,12 +445,12 @@ sgemm_kernel(SegG S, SAct A, int M, int G) {
                         } else {
                             // q41q8_row_amd64.s:65-71; the high half of Q5K1 has min +0
                             const float t1 = dot * wd;
-                            const float t2 = (float)sx[8 * (v >> 2) + 4 * h + (v & 3)] * wm;
+                            const float t2 = sv[v] * wm;
                             float tt = t1 + t2;
                             tt = tt * xv[v];
                             acc[v] = acc[v] + tt;
                             if (has_hb(FMT)) {
-                                const float h1 = (__int_as_float(Dh[v]) - kMagic) * wdh;
+                                const float h1 = dot_of(Dh[v]) * wdh;
                                 const float hh = h1 * xv[v];
                                 acc[v] = acc[v] + hh;
                             }
@@ -534,13 +544,14 @@ sllm_status launch_f(const SegG &S, const SAct &A, int M, int G, hipStream_t s) 
 // Up to 32 rows, and 8192 columns above 4096 weight rows, else 4096 (fewer tiles than
 // waves' chunks of K in turn), whatever else the call holds: a weight's bits do not
 // depend on its company. Measured (us, with the quantize pass; this / the tiled GEMM, M =
-// 16 and 32): Q4_1 14336x4096 21.5 / 29.6 (M = 16), 4096x4096 12.8 / 15.9 and 13.0 / 18.9,
-// 1024x4096 10.1 / 11.7 and 10.6 / 12.5, 4608x8192 19.5 / 27.3 and 20.0 / 29.3, 1536x768 7.6 /
-// 12.1 (M = 16); Q5K1 4096x4096 14.1 / 15.1 and 14.3 / 16.9, 1024x4096 10.4 / 11.3 and 10.8 /
-// 12.2; but (before the quantize pass lost 0.8 us) Q5K1 4096x8192 24.2 / 20.0 and 24.5 /
-// 21.6, 2304x4608 17.4 / 14.5 and 17.5 / 15.9, Q4_1 4096x8192 22.1 / 21.5, Q8_0 4096x14336
-// 37.2 / 26.2 (a wave's seven chunks of K in turn), and with two row tiles (33 to 64 rows)
-// Q4_1 14336x4096 39.4 / 28.8.
+// 16 and 32): Q4_1 14336x4096 22.2 / 29.6 (M = 16), 4096x4096 13.4 / 15.9 and 13.6 / 18.9,
+// 1024x4096 10.1 / 11.7 and 10.5 / 12.5, 4608x8192 21.0 / 27.3 and 21.3 / 29.3, 1536x768 7.6 /
+// 12.1 (M = 16); Q5K1 4096x4096 15.0 / 14.9 and 15.4 / 16.9, 1024x4096 10.7 / 11.3 and 11.3 /
+// 12.2, the one that loses 3072x3072 14.3 / 12.9 and 14.5 / 14.2 (alone; beside others, as q /
+// k / v, the shared launch gains more); but Q5K1 4096x8192 24.2 / 20.0 and 24.5 / 21.6,
+// 2304x4608 17.4 / 14.5 and 17.5 / 15.9, Q4_1 4096x8192 22.1 / 21.5, Q8_0 4096x14336 37.2 /
+// 26.2 (a wave's seven chunks of K in turn), and with two row tiles (33 to 64 rows) Q4_1
+// 14336x4096 39.4 / 28.8.
 bool sgemm_supported(int fmt, int G, int M, int64_t rows) {
     return !act_f32(fmt) && G % kCh == 0 && M <= 32 && G <= (rows <= 4096 ? 128 : 256);
 }

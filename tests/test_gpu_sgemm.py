@@ -146,7 +146,7 @@ def test_wide_launches_equal_the_narrow_ones(qtype, K):
 @pytest.mark.parametrize("qtype", ["q4_1", "q5k1"])
 @pytest.mark.parametrize("N,K,M,gemm", [
     (4097, 256, 4, False), (4097, 256, 5, True), (4096, 256, 6, False), (4096, 256, 7, True), (40, 4096, 5, False),
-    (40, 4096, 6, True), (40, 3840, 6, False), (40, 3840, 7, True), (40, 4352, 7, False), (4097, 4352, 5, True)])
+    (40, 4096, 6, True), (40, 3840, 6, False), (40, 3840, 7, True), (40, 4352, 7, False), (4097, 4352, 7, False), (4097, 4352, 8, True)])
 def test_the_line_between_gemv_and_short_prompt_gemm(qtype, N, K, M, gemm):
     _, w = weight(qtype, N, K, 13)
     x = make_x(M, K, seed=14)
@@ -229,3 +229,32 @@ def test_h_over_gate_or_up_holds_the_swiglu(M, over):
     sq.matmul_swiglu_dev(a, b, x.data_ptr(), M, 512, p, p if over == "gate" else 0, p if over == "up" else 0)
     torch.cuda.synchronize()
     assert torch.isfinite(h).all() and torch.equal(both, h)
+
+
+@pytest.mark.parametrize("qtype", QTYPES)
+@pytest.mark.parametrize("K,M", [(768, 7), (2048, 7), (4096, 32)])
+def test_as_close_to_64_bits_as_the_gemv(qtype, K, M):
+    # the min joins its block's term before the scale: apart, the two would enter the sum
+    # at their own size (1.8 times the GEMV's error)
+    N = 512
+    rng = np.random.default_rng(K)
+    raw, W = _power_of_two_weight(qtype, N, K, rng)
+    if qtype in ("q4_1", "q5k1"):
+        # mins that centre the weights on zero, as a trained layer's do
+        d = raw.reshape(-1)[:N * K // 32 * 20].reshape(N, K // 32, 20)
+        s = d[..., 0:2].copy().view(np.float16)[..., 0].astype(np.float64)
+        m0 = d[..., 2:4].copy().view(np.float16)[..., 0].astype(np.float64)
+        m = s * (-7.5 if qtype == "q4_1" else -15.5)
+        d[..., 2:4] = m.astype(np.float16).view(np.uint8).reshape(N, K // 32, 2)
+        W = W + (m - m0)[..., None]
+    w = sq.DeviceWeight.from_quant(sq.QuantWeight(qtype, np.ascontiguousarray(raw).reshape(-1), K // 32, N, K))
+    # activations that quantize exactly (127 in every block)
+    x = rng.integers(-126, 127, (M, K // 32, 32)).astype(np.float32)
+    x[..., 0] = 127
+    x = (x * 2.0 ** rng.integers(-6, 1, (M, K // 32, 1))).astype(np.float32).reshape(M, K)
+    ref = x.astype(np.float64) @ W.reshape(N, K).T
+    err = lambda y: np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    e = err(run(w, x))
+    sq.set_param("gemm_min_rows", 1 << 20)
+    g = err(run(w, x))
+    assert e <= 1.05 * g, (e, g)
