@@ -332,8 +332,9 @@ def test_the_merge_adds_in_split_order(splits):
 
 @pytest.mark.slow
 def test_prefill_rows_beyond_the_grid_limit():
-    # seq_len x n_kv_heads above 65535 (the split kernel's grid y): the rows
-    # run in chunks, each against the whole cache the prep kernel filled
+    # seq_len x n_kv_heads above 65535, the split kernel's grid y (which runs them in
+    # chunks: test_gpu_attention_prompt.py); with an aligned output, as here, they take
+    # the matrix cores
     rng = np.random.default_rng(5)
     m = Model(64, 64, 8, 4, rng)
     run_case(m, 1030, 0, rng, layer=0, n_layers=2)
