@@ -24,13 +24,15 @@
 // roundings; measured against 64 bits the error is no larger than the GEMV's
 // (gemm_kquant tests).
 //
-// What bounds it: the matrix cores (192 cycles per 32 x 32 tile and 32
-// elements, three part products). A wave owns 32 rows x 32 CT columns; its
-// activation fragments go from L2 straight to registers (they are stored in
-// lane order, so each load is 1 KB contiguous), one block ahead; only the
-// decoded weights pass through LDS, in MFMA order (conflict-free without
-// padding), KB blocks per stage, double-buffered, decoded once per workgroup
-// of 32 WM rows.
+// What bounds it: from about 100 rows the matrix cores with what runs beside them (192
+// cycles per 32 x 32 tile and 32 elements, three part products: busy 36 % of the 51.5 us
+// of Q5_0 14336x4096 at M = 100, VALU 33 %, both at once 11 %); below, neither (Q3_K 14336x4096
+// at M = 64, 46 us: matrix cores 19 %, VALU 32 %): the waves decode, write LDS (conflicts in
+// 64-row tiles as many cycles as accesses) and wait at a barrier every two blocks. A wave
+// owns 32 rows x 32 CT columns; its activation fragments go from L2 straight to registers
+// (they are stored in lane order, so each load is 1 KB contiguous), one block ahead;
+// only the decoded weights pass through LDS, in MFMA order, KB blocks per stage,
+// double-buffered, decoded once per workgroup of 32 WM rows.
 #include <hip/hip_runtime.h>
 
 #include "qmm_device.hpp"
@@ -298,7 +300,7 @@ __device__ __forceinline__ void slow_block(const Planes &P, const float *__restr
 // Blocks whose terms are added one by one before they join the total (0: one
 // chain over the whole range). One chain rounds at the total's size at every
 // group: relative error against 64 bits over K = 4096 / 14336, Q3_K in one chain
-// 2.9e-7 / 5.3e-7, in runs 1.1e-7 / 1.3e-7, the GEMV 1.25e-7 / 1.33e-7. Q5_0
+// 2.9e-7 / 5.3e-7, in runs 0.98e-7 / 1.04e-7, the GEMV 1.25e-7 / 1.33e-7. Q5_0
 // on 128-row tiles keeps one chain: its runs spill (14336x4096 at M = 512 180
 // -> 358 us).
 constexpr int run_of(int fmt, int ct) { return fmt == SLLM_Q5_0 ? (ct == 4 ? 0 : 16) : 8; }

@@ -31,9 +31,9 @@
 // non-finite scale, or an activation scale from 2^90, are computed in the reference's
 // operation order (qmm_gemm.hip has the reasons).
 //
-// Counters (RMSNorm + q / k / v, Q5K1 4096 / 1024, M = 30, 12.5 us for 39 MB of weights, of
-// which the caches held most): matrix cores busy 3 %, VALU 16 %, waves issuing 30 %,
-// waiting on loads and LDS 37 %: the chain of a wave's two chunks.
+// Counters (RMSNorm + q / k / v, Q5K1 4096 / 1024, M = 30, 12.5 us for 20 MB of weights):
+// matrix cores busy 3 %, VALU 16 %, waves issuing 30 %, waiting on loads and LDS 37 %: the
+// chain of a wave's two chunks.
 #include <hip/hip_runtime.h>
 
 #include "qmm_device.hpp"
