@@ -505,10 +505,18 @@ __global__ void __launch_bounds__(256) split_sum_kernel(const float *__restrict_
     dst[i] = add ? dst[i] + s : s;
 }
 
-// A weight of 64 tiles or fewer and more than 64 blocks of K: launched by itself it
-// is cut into K splits, one chunk of K to a wave (Q5K1 1024x4096 at M = 32 11.7 us,
-// 13.3 in four splits of two chunks, 14.8 in one launch).
-bool narrow(int64_t rows, int G) { return rows <= 2048 && G > 64; }
+// A weight of 64 tiles or fewer and more than 64 blocks of K, launched by itself, is cut
+// into K splits, one chunk of K to a wave; while the partial sums stay small also one of up
+// to 96 tiles, 128 for the formats with high bits, whose waves take longest. The bits are
+// the same. Measured (us, in splits / in one launch): Q5K1 1024x4096 at M = 32 11.3 / 14.8,
+// 3072x3072 at M = 8 12.2 / 14.1, M = 16 12.6 / 13.8, M = 32 13.9 / 14.5, 4096x4096 at M = 16
+// 14.5 / 15.0, M = 24 15.5 / 15.1; Q4_0 2560x2560 at M = 16 10.6 / 12.0; Q8_0 3072x4096 at
+// M = 24 12.8 / 13.1, M = 32 13.6 / 13.2, 4096x4096 at M = 8 13.6 / 12.5.
+bool narrow(bool high_bits, int64_t rows, int G, int M) {
+    if (G <= 64) return false;
+    if (rows <= 3072) return rows <= 2048 || rows * M <= (high_bits ? 100000 : 75000);
+    return high_bits && rows <= 4096 && rows * M <= 75000;
+}
 
 template <int FMT, int W>
 sllm_status launch_w(const SegG &S, const SAct &A, int M, int G, hipStream_t s, int splits = 1) {
@@ -525,7 +533,7 @@ sllm_status launch_w(const SegG &S, const SAct &A, int M, int G, hipStream_t s, 
 // eight parts to hold sums of.
 template <int FMT>
 sllm_status launch_f(const SegG &S, const SAct &A, int M, int G, hipStream_t s) {
-    if (S.n == 1 && S.mode != kPair && narrow(S.N[0], G)) {
+    if (S.n == 1 && S.mode != kPair && narrow(has_hb(FMT), S.N[0], G, M)) {
         SegG T = S;
         T.mode = kStore;
         T.dst[0] = (float *)((char *)A.xq + ((sact_bytes(G) + 255) & ~(size_t)255));
@@ -546,9 +554,8 @@ sllm_status launch_f(const SegG &S, const SAct &A, int M, int G, hipStream_t s) 
 // depend on its company. Measured (us, with the quantize pass; this / the tiled GEMM, M =
 // 16 and 32): Q4_1 14336x4096 22.2 / 29.6 (M = 16), 4096x4096 13.4 / 15.9 and 13.6 / 18.9,
 // 1024x4096 10.1 / 11.7 and 10.5 / 12.5, 4608x8192 21.0 / 27.3 and 21.3 / 29.3, 1536x768 7.6 /
-// 12.1 (M = 16); Q5K1 4096x4096 15.0 / 14.9 and 15.4 / 16.9, 1024x4096 10.7 / 11.3 and 11.3 /
-// 12.2, the one that loses 3072x3072 14.3 / 12.9 and 14.5 / 14.2 (alone; beside others, as q /
-// k / v, the shared launch gains more); but Q5K1 4096x8192 24.2 / 20.0 and 24.5 / 21.6,
+// 12.1 (M = 16); Q5K1 4096x4096 14.6 / 14.9 and 15.4 / 16.9, 1024x4096 10.7 / 11.3 and 11.3 /
+// 12.2, 3072x3072 12.6 / 13.0 and 13.9 / 14.2; but Q5K1 4096x8192 24.2 / 20.0 and 24.5 / 21.6,
 // 2304x4608 17.4 / 14.5 and 17.5 / 15.9, Q4_1 4096x8192 22.1 / 21.5, Q8_0 4096x14336 37.2 /
 // 26.2 (a wave's seven chunks of K in turn), and with two row tiles (33 to 64 rows) Q4_1
 // 14336x4096 39.4 / 28.8.
@@ -560,7 +567,7 @@ bool sgemm_supported(int fmt, int G, int M, int64_t rows) {
 // itself.
 size_t sgemm_ws_bytes(int G, int M, int64_t rows) {
     const size_t act = (sact_bytes(G) + 255) & ~(size_t)255;
-    return act + (narrow(rows, G) ? (size_t)kSplits * M * rows * sizeof(float) : 0);
+    return act + (narrow(true, rows, G, M) ? (size_t)kSplits * M * rows * sizeof(float) : 0);
 }
 
 sllm_status launch_sact(const float *x, const float *norm_w, float eps, int M, int G, void *act, hipStream_t s) {

@@ -258,3 +258,19 @@ def test_as_close_to_64_bits_as_the_gemv(qtype, K, M):
     sq.set_param("gemm_min_rows", 1 << 20)
     g = err(run(w, x))
     assert e <= 1.05 * g, (e, g)
+
+
+@pytest.mark.parametrize("qtype", ["q4", "q5k1"])
+@pytest.mark.parametrize("N,M", [(2048, 32), (2049, 32), (3072, 24), (3072, 32), (3073, 24), (4096, 18), (4096, 19), (4097, 9)])
+def test_splits_of_wider_weights_give_the_bits_of_one_launch(qtype, N, M):
+    # alone (in K splits where the rule says so) and beside another weight (one launch)
+    K = 2304
+    _, a = weight(qtype, N, K, 22)
+    _, b = weight(qtype, 33, K, 23)
+    x = torch.from_numpy(make_x(M, K, seed=24)).cuda()
+    alone, ya = (torch.full((M, N), float("nan"), device="cuda") for _ in range(2))
+    yb = torch.empty((M, 33), device="cuda")
+    sq.matmul_dev(a, x.data_ptr(), M, K, alone.data_ptr())
+    sq.matmul_multi_dev([a, b], x.data_ptr(), M, K, [ya.data_ptr(), yb.data_ptr()])
+    torch.cuda.synchronize()
+    assert torch.isfinite(alone).all() and torch.equal(alone, ya)
