@@ -1160,7 +1160,8 @@ FlashPlan flash_plan(int seq, int n_heads, int n_kv, int d_k, int cache_len, siz
     }
     // about two workgroups per resident one (two per CU); few tiles in all are cut
     // to one, two or three each, where a workgroup's fixed cost (first loads, the
-    // merge) weighs against the idle CUs. Measured (us): 32/8/128, 128 rows
+    // merge) weighs against the idle CUs. Measured (us, with the exponential in 32 bits;
+    // in 64 bits each takes 3 to 5 % more): 32/8/128, 128 rows
     // with chunks of 1 / 3 24.7 / 35.2; 200 rows 1 / 2 / 3 36.7 / 32.2 / 37.8; 512
     // rows 2 / 3 / 5 66.0 / 59.8 / 75.5; 1024 rows 3 / 5 / 9 148 / 139 / 149.7
     const int64_t all = total * n_kv, slots = 2 * (int64_t)tuning().attn_target_blocks;
